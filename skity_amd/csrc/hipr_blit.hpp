@@ -1,7 +1,8 @@
 // hipr_blit.hpp -- analytic trapezoid coverage of one scanline step.
 //
 // blit_trapezoid_row / blit_aaa_trapezoid_row and their alpha helpers
-// (src/render/sw/sw_raster.cc:138-544), evaluated per pixel in closed form.
+// (src/render/sw/sw_raster.cc:138-544), evaluated per pixel in closed form and
+// spread over the lanes of a wave.
 // Coverage goes into one LDS delta row, prefix-summed when the pixel row is
 // complete.  Each 32-bit entry carries two fields whose prefix sums are
 // non-negative and below 2^16, so one integer prefix sum S decodes as
@@ -36,44 +37,18 @@ struct RowSink {
   // job whose blend mode does change pixels under a transparent source keeps
   // them (they still count as a direct span of the pixel).
   bool keep_zero;
-  __device__ __forceinline__ int Clamp(int i) const {
-    return i < 0 ? 0 : (i > width ? width : i);
+  // Adds v to the delta at pixel x (clamped into the row).
+  __device__ __forceinline__ void Add(int x, int v) {
+    if (v == 0) return;
+    const int i = x - left;
+    atomicAdd(&d[i < 0 ? 0 : (i > width ? width : i)], v);
   }
-  // kClamp = false: the caller guarantees left <= x and x + len <= left +
-  // width (the per-pixel loop of BlitAAARow, which runs over visible
-  // columns only), so the two entries need no clamping.
-  template <bool kClamp = true>
-  __device__ __forceinline__ void Direct(int x, int len, int v) {
-    if ((v == 0 && !keep_zero) || len <= 0) return;
-    int i = x - left, e = x - left + len;
-    if (kClamp) {
-      i = Clamp(i);
-      e = Clamp(e);
-      if (i == e) return;
-    }
-    int inc = (kDirectCount + v) << 16;
-    atomicAdd(&d[i], inc);
-    atomicAdd(&d[e], -inc);
-  }
-  template <bool kClamp = true>
-  __device__ __forceinline__ void Acc(int x, int len, int v) {
-    if (v == 0 || len <= 0) return;
-    int i = x - left, e = x - left + len;
-    if (kClamp) {
-      i = Clamp(i);
-      e = Clamp(e);
-      if (i == e) return;
-    }
-    atomicAdd(&d[i], v);
-    atomicAdd(&d[e], -v);
-  }
-  template <bool kClamp = true>
-  __device__ __forceinline__ void Put(bool direct, int x, int len, int v) {
-    if (direct) {
-      Direct<kClamp>(x, len, v);
-    } else {
-      Acc<kClamp>(x, len, v);
-    }
+  // A one-pixel span of cover v at a visible pixel.
+  __device__ __forceinline__ void Pixel(bool direct, int x, int v) {
+    if (v == 0 && !(direct && keep_zero)) return;
+    const int inc = direct ? (kDirectCount + v) << 16 : v;
+    atomicAdd(&d[x - left], inc);
+    atomicAdd(&d[x - left + 1], -inc);
   }
 };
 
@@ -131,100 +106,75 @@ __device__ __forceinline__ Alpha AlphaAbove(int i, int R, Fixed l, Fixed r, Fixe
   return (Alpha)(a16 >> 8);
 }
 
-// blit_aaa_trapezoid_row (sw_raster.cc:370-455), one pixel at a time.
-__device__ void BlitAAARow(RowSink* s, Fixed ul, Fixed ur, Fixed ll, Fixed lr, Fixed lDY,
-                           Fixed rDY, Alpha full, bool no_real) {
-  int L = FixedFloorToInt(ul), R = FixedCeilToInt(lr);
-  int len = R - L;
-  bool direct = full == 0xFF && !no_real;
-  if (len == 1) {
-    Alpha a = TrapezoidToAlpha(ur - ul, lr - ll);
-    if (direct) {
-      s->Direct(L, 1, a);
+// Cover of pixel x of blit_aaa_trapezoid_row (sw_raster.cc:370-455): `full`
+// less what lies left of the left edge (ul at the step's top, ll at its
+// bottom) and right of the right edge.  The left edge covers the pixels
+// [floor(ul), ceil(ll)) in part, the right edge [floor(ur), ceil(lr)).
+__device__ __forceinline__ Alpha TrapezoidPixel(int x, Fixed ul, Fixed ur, Fixed ll, Fixed lr,
+                                                Fixed lDY, Fixed rDY, Alpha full) {
+  const int uL = FixedFloorToInt(ul), lL = FixedCeilToInt(ll);
+  const int uR = FixedFloorToInt(ur), lR = FixedCeilToInt(lr);
+  Alpha a = full;
+  if (x >= uL && x < lL) {
+    Alpha t;
+    if (uL + 2 == lL) {
+      const Fixed first = IntToFixed(uL) + kFixed1 - ul;
+      t = x == uL ? (Alpha)(full - PartialTriangleToAlpha(first, lDY))
+                  : PartialTriangleToAlpha(ll - ul - first, lDY);
     } else {
-      s->Acc(L, 1, PartialAlphaA(a, full));
+      const Fixed l = ul - IntToFixed(uL), r = ll - IntToFixed(uL);
+      t = AlphaBelow(x - uL, FixedCeilToInt(r), l, r, lDY, full);
     }
-    return;
+    a = a > t ? (Alpha)(a - t) : 0;
   }
-  int uL = FixedFloorToInt(ul), lL = FixedCeilToInt(ll);
-  int uR = FixedFloorToInt(ur), lR = FixedCeilToInt(lr);
-  bool left_two = uL + 2 == lL;
-  bool right_two = uR + 2 == lR;
-  Fixed lfirst = 0, lsecond = 0, rfirst = 0, rsecond = 0;
-  Alpha la1 = 0, la2 = 0, ra1 = 0, ra2 = 0;
-  if (left_two) {
-    lfirst = IntToFixed(uL) + kFixed1 - ul;
-    lsecond = ll - ul - lfirst;
-    la1 = (Alpha)(full - PartialTriangleToAlpha(lfirst, lDY));
-    la2 = PartialTriangleToAlpha(lsecond, lDY);
-  }
-  if (right_two) {
-    rfirst = IntToFixed(uR) + kFixed1 - ur;
-    rsecond = lr - ur - rfirst;
-    ra1 = PartialTriangleToAlpha(rfirst, rDY);
-    ra2 = (Alpha)(full - PartialTriangleToAlpha(rsecond, rDY));
-  }
-  Fixed bl_l = ul - IntToFixed(uL), bl_r = ll - IntToFixed(uL);
-  int bl_R = FixedCeilToInt(bl_r);
-  Fixed ab_l = ur - IntToFixed(uR), ab_r = lr - IntToFixed(uR);
-  int ab_R = FixedCeilToInt(ab_r);
-  // Run of equal full alphas between the two AA regions goes out as one
-  // delta span; every other pixel individually.  Pixels outside the visible
-  // columns add nothing any visible pixel reads (RowSink), so they are
-  // skipped.
-  int run_begin = -1, run_len = 0;
-  const int i_end = Min32(len, s->left + s->width - L);
-  for (int i = Max32(0, s->left - L); i < i_end; i++) {
-    int x = L + i;
-    Alpha a = full;
-    bool touched = false;
-    if (left_two) {
-      if (i == 0) {
-        a = a > la1 ? (Alpha)(a - la1) : 0;
-        touched = true;
-      } else if (i == 1) {
-        a = a > la2 ? (Alpha)(a - la2) : 0;
-        touched = true;
-      }
-    } else if (x >= uL && x < lL) {
-      Alpha t = AlphaBelow(x - uL, bl_R, bl_l, bl_r, lDY, full);
-      a = a > t ? (Alpha)(a - t) : 0;
-      touched = true;
-    }
-    if (right_two) {
-      if (i == len - 2) {
-        a = a > ra1 ? (Alpha)(a - ra1) : 0;
-        touched = true;
-      } else if (i == len - 1) {
-        a = a > ra2 ? (Alpha)(a - ra2) : 0;
-        touched = true;
-      }
-    } else if (x >= uR && x < lR) {
-      Alpha t = AlphaAbove(x - uR, ab_R, ab_l, ab_r, rDY, full);
-      a = a > t ? (Alpha)(a - t) : 0;
-      touched = true;
-    }
-    if (!touched) {
-      if (run_begin < 0) run_begin = x;
-      run_len++;
+  if (x >= uR && x < lR) {
+    Alpha t;
+    if (uR + 2 == lR) {
+      const Fixed first = IntToFixed(uR) + kFixed1 - ur;
+      t = x == uR ? PartialTriangleToAlpha(first, rDY)
+                  : (Alpha)(full - PartialTriangleToAlpha(lr - ur - first, rDY));
     } else {
-      if (run_len > 0) {
-        s->Put<false>(direct, run_begin, run_len, full);
-        run_begin = -1;
-        run_len = 0;
-      }
-      s->Put<false>(direct, x, 1, a);
+      const Fixed l = ur - IntToFixed(uR), r = lr - IntToFixed(uR);
+      t = AlphaAbove(x - uR, FixedCeilToInt(r), l, r, rDY, full);
     }
+    a = a > t ? (Alpha)(a - t) : 0;
   }
-  if (run_len > 0) s->Put<false>(direct, run_begin, run_len, full);
+  return a;
 }
 
-// blit_trapezoid_row (sw_raster.cc:457-544).
-__device__ void BlitTrapezoidRow(RowSink* s, Fixed ul, Fixed ur, Fixed ll, Fixed lr,
-                                 Fixed lDY, Fixed rDY, Alpha full, bool no_real) {
-  if (ul > ur) return;
+// Number of lanes below this one whose bit is set.
+__device__ __forceinline__ int CountBelow(uint64_t m, int base = 0) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                        __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)base));
+}
+
+// LDS of BlitIntervals: two int4 per trapezoid with per-pixel work, and one
+// mark per work item of a pass.
+struct BlitScratch {
+  int4* items;   // 2 x 64
+  int32_t* mark; // 64
+};
+constexpr int kBlitScratchInts = 2 * kWave * 4 + kWave;
+
+// blit_trapezoid_row (sw_raster.cc:457-544) for up to 64 trapezoids of one
+// step, one per lane (`act`).
+//
+// A trapezoid is a run of `full` pixels between a left and a right edge.  An
+// edge that stays within one or two pixels is done by the trapezoid's own
+// lane as deltas.  A flatter one covers a row of pixels in part, each with
+// its own cover (TrapezoidPixel), as does every pixel of a trapezoid whose
+// edges share pixels.  Those pixels, a few for most trapezoids and hundreds
+// for a nearly horizontal edge, are laid end to end and handed out one per
+// lane, so a wave takes ceil(total / 64) passes over them however unevenly
+// they are spread; looping over them per lane took as many passes as the
+// longest one has pixels (measured with the change in hipr_walk.hpp).
+__device__ __forceinline__ void BlitIntervals(RowSink& s, const BlitScratch& L, bool act, Fixed ul,
+                                              Fixed ur, Fixed ll, Fixed lr, Fixed lDY, Fixed rDY,
+                                              Alpha full, bool no_real) {
+  const int lane = Lane();
+  bool go = act && ul <= ur;
   if (ll > lr) ll = lr = ApproxIntersection(ul, ll, ur, lr);
-  if (ul == ur && ll == lr) return;
+  go = go && !(ul == ur && ll == lr);
   if (ul > ll) {
     Fixed t = ul;
     ul = ll;
@@ -235,56 +185,100 @@ __device__ void BlitTrapezoidRow(RowSink* s, Fixed ul, Fixed ur, Fixed ll, Fixed
     ur = lr;
     lr = t;
   }
-  bool direct = full == 0xFF && !no_real;
-  Fixed join_left = FixedCeilToFixed(ll);
-  Fixed join_rite = FixedFloorToFixed(ur);
-  if (join_left <= join_rite) {
-    if (ul < join_left) {
-      int len = FixedCeilToInt(join_left - ul);
-      if (len == 1) {
-        Alpha a = TrapezoidToAlpha(join_left - ul, join_left - ll);
-        if (direct) {
-          s->Direct(ul >> 16, 1, a);
+  const bool direct = full == 0xFF && !no_real;
+  // a span's increment at its first pixel; its end takes it back
+  auto inc = [&](int v) -> int {
+    if (!direct) return v;
+    return v != 0 || s.keep_zero ? (kDirectCount + v) << 16 : 0;
+  };
+  auto part = [&](Alpha a) -> int { return inc(direct ? a : PartialAlphaA(a, full)); };
+  const int vis_end = s.left + s.width;
+  int cnt_a = 0, cnt = 0;
+  if (go) {
+    const Fixed join_left = FixedCeilToFixed(ll), join_rite = FixedFloorToFixed(ur);
+    const int x0 = ul >> 16;
+    if (join_left <= join_rite) {
+      const int JL = join_left >> 16, JR = join_rite >> 16;
+      int last = 0, first = 0;  // increments left of JL and right of JR
+      if (ul < join_left) {
+        const int len = FixedCeilToInt(join_left - ul);
+        if (len == 1) {
+          last = part(TrapezoidToAlpha(join_left - ul, join_left - ll));
+          s.Add(x0, last);
+        } else if (len == 2) {
+          const Fixed f = join_left - kFixed1 - ul;
+          const Fixed sec = ll - ul - f;
+          const int i1 = inc(PartialTriangleToAlpha(f, lDY));
+          last = inc((Alpha)(full - PartialTriangleToAlpha(sec, lDY)));
+          s.Add(x0, i1);
+          s.Add(x0 + 1, last - i1);
         } else {
-          s->Acc(ul >> 16, 1, PartialAlphaA(a, full));
+          cnt_a = Max32(0, Min32(JL, vis_end) - Max32(x0, s.left));
+          cnt = cnt_a;
         }
-      } else if (len == 2) {
-        Fixed first = join_left - kFixed1 - ul;
-        Fixed second = ll - ul - first;
-        Alpha a1 = PartialTriangleToAlpha(first, lDY);
-        Alpha a2 = (Alpha)(full - PartialTriangleToAlpha(second, lDY));
-        s->Put(direct, ul >> 16, 1, a1);
-        s->Put(direct, (ul >> 16) + 1, 1, a2);
+      }
+      if (lr > join_rite) {
+        const int len = FixedCeilToInt(lr - join_rite);
+        if (len == 1) {
+          first = part(TrapezoidToAlpha(ur - join_rite, lr - join_rite));
+          s.Add(JR + 1, -first);
+        } else if (len == 2) {
+          const Fixed f = join_rite + kFixed1 - ur;
+          const Fixed sec = lr - ur - f;
+          first = inc((Alpha)(full - PartialTriangleToAlpha(f, rDY)));
+          const int i2 = inc(PartialTriangleToAlpha(sec, rDY));
+          s.Add(JR + 1, i2 - first);
+          s.Add(JR + 2, -i2);
+        } else {
+          cnt += Max32(0, Min32(FixedCeilToInt(lr), vis_end) - Max32(JR, s.left));
+        }
+      }
+      const int run = join_left < join_rite ? inc(full) : 0;
+      s.Add(JL, run - last);
+      s.Add(JR, first - run);
+    } else {
+      const int R = FixedCeilToInt(lr);
+      if (R - x0 == 1) {
+        const int v = part(TrapezoidToAlpha(ur - ul, lr - ll));
+        s.Add(x0, v);
+        s.Add(R, -v);
       } else {
-        BlitAAARow(s, ul, join_left, ll, join_left, lDY, kMaxS32, full, no_real);
+        cnt_a = Max32(0, Min32(R, vis_end) - Max32(x0, s.left));
+        cnt = cnt_a;
       }
     }
-    if (join_left < join_rite) {
-      s->Put(direct, FixedFloorToInt(join_left), FixedFloorToInt(join_rite - join_left),
-             full);
+  }
+  const uint64_t have = __ballot(cnt > 0);
+  if (have == 0) return;
+  const int incl = ScanSum(cnt);
+  const int total = __builtin_amdgcn_readlane(incl, kWave - 1);
+  const int start = incl - cnt;
+  if (cnt > 0) {
+    int4* it = L.items + 2 * CountBelow(have);
+    it[0] = make_int4(ul, ur, ll, lr);
+    it[1] = make_int4(lDY, rDY, (cnt_a << 1) | (direct ? 1 : 0), start);
+  }
+  int before = 0;  // trapezoids whose pixels start before this pass
+  for (int base = 0; base < total; base += kWave) {
+    // mark where each trapezoid's pixels start; the marks up to a lane count
+    // the trapezoids up to its pixel
+    L.mark[lane] = 0;
+    WaveSync();
+    if (cnt > 0 && start >= base && start < base + kWave) L.mark[start - base] = 1;
+    WaveSync();
+    const uint64_t marks = __ballot(L.mark[lane] != 0);
+    const int t = base + lane;
+    if (t < total) {
+      const int own = CountBelow(marks, before) + (int)((marks >> lane) & 1) - 1;
+      const int4 a = L.items[2 * own], b = L.items[2 * own + 1];
+      const int o = t - b.w, ca = b.z >> 1;
+      const int x = o < ca ? Max32(a.x >> 16, s.left) + o
+                           : Max32(FixedFloorToInt(a.y), s.left) + (o - ca);
+      const Alpha v = TrapezoidPixel(x, a.x, a.y, a.z, a.w, b.x, b.y, full);
+      s.Pixel((b.z & 1) != 0, x, v);
     }
-    if (lr > join_rite) {
-      int len = FixedCeilToInt(lr - join_rite);
-      if (len == 1) {
-        Alpha a = TrapezoidToAlpha(ur - join_rite, lr - join_rite);
-        if (direct) {
-          s->Direct(join_rite >> 16, 1, a);
-        } else {
-          s->Acc(join_rite >> 16, 1, PartialAlphaA(a, full));
-        }
-      } else if (len == 2) {
-        Fixed first = join_rite + kFixed1 - ur;
-        Fixed second = lr - ur - first;
-        Alpha a1 = (Alpha)(full - PartialTriangleToAlpha(first, rDY));
-        Alpha a2 = PartialTriangleToAlpha(second, rDY);
-        s->Put(direct, join_rite >> 16, 1, a1);
-        s->Put(direct, (join_rite >> 16) + 1, 1, a2);
-      } else {
-        BlitAAARow(s, join_rite, ur, join_rite, lr, kMaxS32, rDY, full, no_real);
-      }
-    }
-  } else {
-    BlitAAARow(s, ul, ur, ll, lr, lDY, rDY, full, no_real);
+    before += __popcll(marks);
+    WaveSync();
   }
 }
 

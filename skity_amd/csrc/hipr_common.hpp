@@ -193,6 +193,15 @@ __device__ __forceinline__ int DppScanMax(int v) {
   v = DppMax2(v, __builtin_amdgcn_update_dpp(lo, v, kDppBcast31, 0xc, 0xf, false));
   return v;
 }
+// Lanes 2i and 2i + 1 trade places (quad_perm 1, 0, 3, 2).
+__device__ __forceinline__ int DppSwapPairs(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true);
+}
+// Smallest value of the wave, in every lane.
+__device__ __forceinline__ int DppWaveMin(int v) {
+  // ~v turns the minimum into the maximum the scan leaves in lane 63
+  return ~__builtin_amdgcn_readlane(DppScanMax(~v), kWave - 1);
+}
 // Lane i receives lane i-1 (lane 0 receives `fill`).
 __device__ __forceinline__ int DppShiftUp(int v, int fill) {
   return __builtin_amdgcn_update_dpp(fill, v, kDppWaveShr1, 0xf, 0xf, false);

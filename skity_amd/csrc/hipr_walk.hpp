@@ -163,12 +163,14 @@ __host__ __device__ inline int BandStartRow(const PixBounds& pb, int nb, int b) 
   return (v + kTile - 1) & ~(kTile - 1);
 }
 
-// meta word of an active edge: bit 0 winding < 0, bit 1 quad, bits 2.. index
-__device__ __forceinline__ int MetaWinding(int m) { return (m & 1) ? -1 : 1; }
+// meta word of an active edge: bit 0 winding < 0, bit 1 quad, bit 2 the quad's
+// state has moved on (it lives in qstate; before that it is the sorted edge
+// record's), bits 3.. index
 __device__ __forceinline__ bool MetaQuad(int m) { return (m & 2) != 0; }
-__device__ __forceinline__ int MetaIndex(int m) { return (int)((uint32_t)m >> 2); }
-__device__ __forceinline__ int MakeMeta(int winding, bool quad, int idx) {
-  return (winding < 0 ? 1 : 0) | (quad ? 2 : 0) | (idx << 2);
+__device__ __forceinline__ bool MetaMoved(int m) { return (m & 4) != 0; }
+__device__ __forceinline__ int MetaIndex(int m) { return (int)((uint32_t)m >> 3); }
+__device__ __forceinline__ int MakeMeta(int winding, bool quad, bool moved, int idx) {
+  return (winding < 0 ? 1 : 0) | (quad ? 2 : 0) | (moved ? 4 : 0) | (idx << 3);
 }
 
 struct WalkLds {
@@ -181,7 +183,18 @@ struct WalkLds {
   int32_t* sDY;
   int32_t* sLY;
   int32_t* sM;
+  // left and right edges of the step's intervals {x, next x, dy, the next
+  // edge is too close}; they share the permutation scratch, which is free
+  // while the intervals are drawn
+  int4* iL;        // CAP / 2 entries each
+  int4* iR;
+  BlitScratch blit;
 };
+// LDS words of a K-slot walk whose rows are up to `w` pixels wide (w a
+// multiple of 16).
+__host__ __device__ inline int WalkLdsInts(int K, int w) {
+  return kBlitScratchInts + 5 * K * kWave + (w + 1) + 3 * (w / kTile + 2);
+}
 
 // Bitonic sort (ascending) of N = 64 * 2^j keys held as element
 // p = slot * 64 + lane; keys at p >= N are not touched (N <= 64 * K).
@@ -287,15 +300,19 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
   // the band ends where the next band's snapshot was taken
   const Fixed stop_y = (kWrite && rband + 1 < nb) ? snap_at(rband + 1)->y : kMaxS32;
   WalkLds L;
-  L.d = lds;
-  L.slot0 = L.d + (P.lds_width + 1);
-  L.slot1 = L.slot0 + (P.lds_width / kTile + 2);
-  L.rows = L.slot1 + (P.lds_width / kTile + 2);
-  L.sX = L.rows + (P.lds_width / kTile + 2);
+  L.blit.items = (int4*)lds;
+  L.blit.mark = lds + 2 * kWave * 4;
+  L.sX = lds + kBlitScratchInts;
   L.sDX = L.sX + CAP;
   L.sDY = L.sDX + CAP;
   L.sLY = L.sDY + CAP;
   L.sM = L.sLY + CAP;
+  L.iL = (int4*)L.sX;
+  L.iR = L.iL + CAP / 2;
+  L.d = L.sM + CAP;
+  L.slot0 = L.d + (P.lds_width + 1);
+  L.slot1 = L.slot0 + (P.lds_width / kTile + 2);
+  L.rows = L.slot1 + (P.lds_width / kTile + 2);
   for (int i = lane; i <= W; i += kWave) {
     L.d[i] = 0;
   }
@@ -326,6 +343,8 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
   // Active list registers.
   Fixed X[K], DX[K], DY[K], LY[K];
   int M[K];
+#pragma unroll
+  for (int t = 0; t < K; t++) X[t] = DX[t] = DY[t] = LY[t] = M[t] = 0;
   int n = 0;
   int next_slot = 0;  // tile planes allocated so far
   int band = -1;      // current 16-row band
@@ -386,7 +405,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
 
   // Resolve pixel row r (prefix-sum the deltas) and emit its tile rows.
   auto flush_row = [&](int r) {
-    int lo = WaveMin(dmin), hi = WaveMax(dmax);
+    int lo = DppWaveMin(dmin), hi = -DppWaveMin(-dmax);
     dmin = 0x7FFFFFFF;
     dmax = -0x7FFFFFFF;
     if (lo > hi) return;  // nothing drawn in this row
@@ -546,65 +565,312 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
     WaveSync();
   };
 
-  // Insert `k` new edges already in scratch (sX.. at [CAP-k.. ) no: at 0..k-1
-  // of the n* arrays) -- implemented inline below.
-
   // ---- pending edges ---------------------------------------------------------
+  // The next 64 pending edges are kept in registers, lane i holding sorted
+  // edge w_base + i, so that looking at the next one and activating edges
+  // takes no memory access.
   int pp = 0;  // next pending edge (sorted position)
-  int pu_idx = -1;
-  Fixed pu_val = kMaxS32;  // upper_y of edge pu_idx, read once
-  auto pending_upper = [&](int idx) -> Fixed {
-    if (idx != pu_idx) {
-      pu_idx = idx;
-      pu_val = idx < nE ? E[idx].upper_y : kMaxS32;
+  int w_base = 0;
+  Fixed w_x = 0, w_dx = 0, w_dy = 0, w_uy = kMaxS32, w_ly = 0;
+  int w_pk = 0;
+  auto load_window = [&](int base) {
+    w_base = base;
+    const int idx = base + lane;
+    w_uy = kMaxS32;
+    if (idx < nE) {
+      const int4* e = (const int4*)&E[idx];
+      const int4 a = e[0], b = e[1];
+      w_x = a.x;
+      w_dx = a.z;
+      w_dy = a.w;
+      w_uy = b.y;
+      w_ly = b.z;
+      w_pk = b.w;
     }
-    return pu_val;
   };
+  // upper_y of the next pending edge (kMaxS32 after the last)
+  auto pending_upper = [&]() -> Fixed {
+    if (pp - w_base >= kWave) load_window(pp);
+    return __builtin_amdgcn_readlane(w_uy, pp - w_base);
+  };
+  Fixed nny = kMaxS32;
+  Fixed min_ly = kMaxS32;  // smallest lower_y of the active list
 
-  // Gathers the new edges with upper_y <= y into scratch slots
-  // [CAP/2 ...] -- uses separate regions of the scratch arrays: survivors are
-  // reloaded before new edges are staged, so the whole scratch is free.
-  // Returns the number of new edges (sorted by x, dx, index).
-  auto gather_new = [&](Fixed y, int* out_k) -> bool {
-    int k = 0;
-    for (;;) {
-      int idx = pp + k + lane;
-      Fixed uy = idx < nE ? E[idx].upper_y : kMaxS32;
-      bool ready = uy <= y;
-      uint64_t b = __ballot(ready);
-      int cnt = __popcll(b);
-      if (k + cnt > CAP) return false;
-      if (ready) {
-        const EdgeRec* er = &E[idx];
-        const int32_t packed = er->packed;
-        if (EdgeIsQuad(packed)) {
-          // the quad's state from here on; four 16-byte moves (a struct
-          // copy would be staged through scratch memory)
-          const int4* src = (const int4*)er;
-          int4* dst = (int4*)&Q[idx];
-          const int4 q0 = src[0], q1 = src[1], q2 = src[2], q3 = src[3];
-          dst[0] = q0;
-          dst[1] = q1;
-          dst[2] = q2;
-          dst[3] = q3;
-        }
-        int p = k + lane;
-        L.sX[p] = er->x;
-        L.sDX[p] = er->dx;
-        L.sDY[p] = er->dy;
-        L.sLY[p] = er->lower_y;
-        L.sM[p] = MakeMeta(EdgeWinding(packed), EdgeIsQuad(packed), idx);
-      }
-      k += cnt;
-      if (cnt < kWave) break;
+  // Takes the pending edges with upper_y <= y into the active list
+  // (insert_new_edges; with an empty list, the initial activation).  Returns
+  // false when the list outgrows the walk.
+  auto insert_new = [&](Fixed y, bool initial) -> bool {
+    if (pp - w_base >= kWave) load_window(pp);
+    int off = pp - w_base;
+    uint64_t ready = __ballot(lane >= off && w_uy <= y);
+    if ((ready >> (kWave - 1)) != 0 && off > 0) {
+      // the run may go on past the window
+      load_window(pp);
+      off = 0;
+      ready = __ballot(w_uy <= y);
     }
-    *out_k = k;
+    int k = __popcll(ready);
+    if (k == kWave) {
+      // 64 or more at once: count them all
+      for (;;) {
+        const int idx = pp + k + lane;
+        const int cnt = __popcll(__ballot(idx < nE && E[idx < nE ? idx : 0].upper_y <= y));
+        k += cnt;
+        if (n + k > CAP) return false;
+        if (cnt < kWave) break;
+      }
+    }
+    if (n + k > CAP) return false;
+    WaveSync();
+    if (k <= kWave) {
+      // lane i takes new edge i
+      const bool mine = lane < k;
+      Fixed nX = w_x, nDX = w_dx, nDY = w_dy, nLY = w_ly;
+      int nM = MakeMeta(EdgeWinding(w_pk), EdgeIsQuad(w_pk), false, w_base + lane);
+      if (off != 0) {
+        const int src = (lane + off) & (kWave - 1);
+        nX = __shfl(nX, src, kWave);
+        nDX = __shfl(nDX, src, kWave);
+        nDY = __shfl(nDY, src, kWave);
+        nLY = __shfl(nLY, src, kWave);
+        nM = __shfl(nM, src, kWave);
+      }
+      if (k > 1) {
+        // sorted by (x, dx, sorted position): rank by counting
+        int r = 0;
+        for (int q = 0; q < k; q++) {
+          const Fixed xq = __builtin_amdgcn_readlane(nX, q);
+          const Fixed dxq = __builtin_amdgcn_readlane(nDX, q);
+          r += (xq < nX || (xq == nX && (dxq < nDX || (dxq == nDX && q < lane)))) ? 1 : 0;
+        }
+        if (!mine) r = lane;
+        if (__ballot(r != lane) != 0) {
+          nX = __builtin_amdgcn_ds_permute(4 * r, nX);
+          nDX = __builtin_amdgcn_ds_permute(4 * r, nDX);
+          nDY = __builtin_amdgcn_ds_permute(4 * r, nDY);
+          nLY = __builtin_amdgcn_ds_permute(4 * r, nLY);
+          nM = __builtin_amdgcn_ds_permute(4 * r, nM);
+        }
+      }
+      const int mn = DppWaveMin(mine && (!initial || nLY > y) ? nLY : kMaxS32);
+      min_ly = Min32(min_ly, mn);
+      // insertion positions: P0 = #{a : x_a <= x_N0};
+      // Pi = max(P(i-1), #{a : x_a < x_Ni}); list element q moves to
+      // q + #{i : Pi <= q}, new edge i goes to Pi + i
+      int my_pos = 0, p_cur = 0, first_pos = 0;
+      int shift[K];
+#pragma unroll
+      for (int s = 0; s < K; s++) shift[s] = 0;
+      const int S0 = (n + kWave - 1) / kWave;
+      if (n > 0) {
+        for (int i = 0; i < k; i++) {
+          const Fixed xi = __builtin_amdgcn_readlane(nX, i);
+          int cnt = 0;
+#pragma unroll
+          for (int s = 0; s < K; s++) {
+            if (s >= S0) break;
+            const int p = s * kWave + lane;
+            cnt += __popcll(__ballot(p < n && (i == 0 ? X[s] <= xi : X[s] < xi)));
+          }
+          if (i == 0) first_pos = cnt;
+          p_cur = Max32(p_cur, cnt);
+          my_pos = lane == i ? p_cur : my_pos;
+#pragma unroll
+          for (int s = 0; s < K; s++) {
+            if (s >= S0) break;
+            shift[s] += (s * kWave + lane >= p_cur) ? 1 : 0;
+          }
+        }
+      }
+      if (!initial) {
+        // check_intersection with the predecessor at insertion: the new edge
+        // before it if that sits right there, else the list element before
+        bool crosses = false;
+        if (n > 0) {
+#pragma unroll
+          for (int s = 0; s < K; s++) {
+            if (s >= S0) break;
+            L.sM[s * kWave + lane] = X[s] + DX[s];
+          }
+          WaveSync();
+        }
+        const Fixed v = nX + nDX;
+        const Fixed pv = ShiftUp(v, 0);
+        const int ppos = ShiftUp(my_pos, -1);
+        if (mine) {
+          if (lane > 0 && ppos == my_pos) {
+            crosses = pv > v;
+          } else if (my_pos > 0) {
+            crosses = L.sM[my_pos - 1] > v;
+          }
+        }
+        if (__ballot(crosses) != 0) nny = y + (kFixed1 >> kAcc);
+        WaveSync();
+      }
+      if (mn > y && mn < nny) nny = mn;
+      // merge through scratch, from the slot of the first new edge on
+      const int s_from = first_pos / kWave;
+#pragma unroll
+      for (int s = 0; s < K; s++) {
+        if (s >= S0) break;
+        if (s < s_from) continue;
+        const int q = s * kWave + lane;
+        if (q < n) {
+          const int d = q + shift[s];
+          L.sX[d] = X[s];
+          L.sDX[d] = DX[s];
+          L.sDY[d] = DY[s];
+          L.sLY[d] = LY[s];
+          L.sM[d] = M[s];
+        }
+      }
+      if (mine) {
+        const int d = my_pos + lane;
+        L.sX[d] = nX;
+        L.sDX[d] = nDX;
+        L.sDY[d] = nDY;
+        L.sLY[d] = nLY;
+        L.sM[d] = nM;
+      }
+      WaveSync();
+      n += k;
+      pp += k;
+#pragma unroll
+      for (int s = 0; s < K; s++) {
+        if (s < s_from) continue;
+        const int p = s * kWave + lane;
+        if (p < n) {
+          X[s] = L.sX[p];
+          DX[s] = L.sDX[p];
+          DY[s] = L.sDY[p];
+          LY[s] = L.sLY[p];
+          M[s] = L.sM[p];
+        }
+      }
+      WaveSync();
+      return true;
+    }
+    if (K == 1) return false;
+    // More than 64 at once (K > 1): the same through scratch.
+    for (int p = lane; p < k; p += kWave) {
+      const EdgeRec* er = &E[pp + p];
+      const int32_t packed = er->packed;
+      L.sX[p] = er->x;
+      L.sDX[p] = er->dx;
+      L.sDY[p] = er->dy;
+      L.sLY[p] = er->lower_y;
+      L.sM[p] = MakeMeta(EdgeWinding(packed), EdgeIsQuad(packed), false, pp + p);
+    }
+    WaveSync();
+    int rk[K];
+    Fixed nX[K], nDX[K], nDY[K], nLY[K];
+    int nM[K];
+    int mn = kMaxS32;
+#pragma unroll
+    for (int s = 0; s < K; s++) {
+      const int p = s * kWave + lane;
+      rk[s] = 0;
+      if (p < k) {
+        const Fixed xi = L.sX[p], dxi = L.sDX[p];
+        int r = 0;
+        for (int q = 0; q < k; q++) {
+          const Fixed xq = L.sX[q], dxq = L.sDX[q];
+          r += (xq < xi || (xq == xi && (dxq < dxi || (dxq == dxi && q < p)))) ? 1 : 0;
+        }
+        rk[s] = r;
+        nX[s] = xi;
+        nDX[s] = dxi;
+        nDY[s] = L.sDY[p];
+        nLY[s] = L.sLY[p];
+        nM[s] = L.sM[p];
+        if (!initial || nLY[s] > y) mn = Min32(mn, nLY[s]);
+      }
+    }
+    mn = DppWaveMin(mn);
+    min_ly = Min32(min_ly, mn);
+    WaveSync();
+#pragma unroll
+    for (int s = 0; s < K; s++) {
+      const int p = s * kWave + lane;
+      if (p < k) {
+        L.sX[rk[s]] = nX[s];
+        L.sDX[rk[s]] = nDX[s];
+      }
+    }
+    WaveSync();
+    // positions of the new edges in sorted order, kept in sLY
+    int p_cur = 0;
+    bool crosses = false;
+    int shift[K];
+#pragma unroll
+    for (int s = 0; s < K; s++) shift[s] = 0;
+    for (int i = 0; i < k; i++) {
+      const Fixed xi = L.sX[i];
+      int cnt = 0;
+#pragma unroll
+      for (int s = 0; s < K; s++) {
+        const int p = s * kWave + lane;
+        cnt += __popcll(__ballot(p < n && (i == 0 ? X[s] <= xi : X[s] < xi)));
+      }
+      const int prev = p_cur;
+      p_cur = Max32(p_cur, cnt);
+      Fixed pred = 0;
+      bool has_pred = false;
+      if (i > 0 && p_cur == prev) {
+        pred = L.sX[i - 1] + L.sDX[i - 1];
+        has_pred = true;
+      } else if (p_cur > 0) {
+        const int q = __builtin_amdgcn_readfirstlane(p_cur - 1);
+#pragma unroll
+        for (int t = 0; t < K; t++)
+          if (t == q / kWave) pred = __builtin_amdgcn_readlane(X[t] + DX[t], q % kWave);
+        has_pred = true;
+      }
+      if (has_pred && pred > xi + L.sDX[i]) crosses = true;
+      if (lane == 0) L.sLY[i] = p_cur;
+#pragma unroll
+      for (int s = 0; s < K; s++) shift[s] += (s * kWave + lane >= p_cur) ? 1 : 0;
+    }
+    if (!initial && crosses) nny = y + (kFixed1 >> kAcc);
+    if (mn > y && mn < nny) nny = mn;
+    WaveSync();
+    int posN[K];
+#pragma unroll
+    for (int s = 0; s < K; s++) {
+      const int p = s * kWave + lane;
+      posN[s] = p < k ? L.sLY[rk[s]] + rk[s] : 0;
+    }
+    WaveSync();
+#pragma unroll
+    for (int s = 0; s < K; s++) {
+      const int q = s * kWave + lane;
+      if (q < n) {
+        const int d = q + shift[s];
+        L.sX[d] = X[s];
+        L.sDX[d] = DX[s];
+        L.sDY[d] = DY[s];
+        L.sLY[d] = LY[s];
+        L.sM[d] = M[s];
+      }
+      if (q < k) {
+        const int d = posN[s];
+        L.sX[d] = nX[s];
+        L.sDX[d] = nDX[s];
+        L.sDY[d] = nDY[s];
+        L.sLY[d] = nLY[s];
+        L.sM[d] = nM[s];
+      }
+    }
+    WaveSync();
+    n += k;
+    pp += k;
+    load_from_scratch(n);
+    WaveSync();
     return true;
   };
 
   // ---- initial activation (sw_raster.cc:554-563) -------------------------------
   Fixed y = Max32(E[0].upper_y, IntToFixed(path_top));
-  Fixed nny = kMaxS32;
   if (rband > 0) {
     // resume from the band's snapshot
     const SnapHeader* h = snap_at(rband);
@@ -615,6 +881,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
     n = h->n;
     const int32_t* a = (const int32_t*)(h + 1);
     const EdgeRec* qs = (const EdgeRec*)(a + 5 * CAP);
+    int mn = kMaxS32;
 #pragma unroll
     for (int s = 0; s < K; s++) {
       int p = s * kWave + lane;
@@ -624,79 +891,26 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
         DY[s] = a[2 * CAP + p];
         LY[s] = a[3 * CAP + p];
         M[s] = a[4 * CAP + p];
-        if (MetaQuad(M[s])) Q[MetaIndex(M[s])] = qs[p];
+        if (MetaMoved(M[s])) Q[MetaIndex(M[s])] = qs[p];
+        mn = Min32(mn, LY[s]);
       }
     }
+    min_ly = DppWaveMin(mn);
+    load_window(pp);
   } else {
-    int k;
-    if (!gather_new(y, &k)) {
-      flags |= 2;
-      k = 0;
-    }
-    WaveSync();
-    // sort the k new edges by (x, dx, index): rank by counting
-    // (the sorted-by-upper_y input keeps index order within equal keys)
-    int rk[K];
-#pragma unroll
-    for (int s = 0; s < K; s++) {
-      int p = s * kWave + lane;
-      rk[s] = 0;
-      if (p < k) {
-        Fixed xi = L.sX[p], dxi = L.sDX[p];
-        int r = 0;
-        for (int q = 0; q < k; q++) {
-          Fixed xq = L.sX[q], dxq = L.sDX[q];
-          bool less = xq < xi || (xq == xi && (dxq < dxi || (dxq == dxi && q < p)));
-          r += less ? 1 : 0;
-        }
-        rk[s] = r;
-      }
-    }
-    Fixed tX[K], tDX[K], tDY[K], tLY[K];
-    int tM[K];
-#pragma unroll
-    for (int s = 0; s < K; s++) {
-      int p = s * kWave + lane;
-      if (p < k) {
-        tX[s] = L.sX[p];
-        tDX[s] = L.sDX[p];
-        tDY[s] = L.sDY[p];
-        tLY[s] = L.sLY[p];
-        tM[s] = L.sM[p];
-      }
-    }
-    WaveSync();
-#pragma unroll
-    for (int s = 0; s < K; s++) {
-      int p = s * kWave + lane;
-      if (p < k) {
-        L.sX[rk[s]] = tX[s];
-        L.sDX[rk[s]] = tDX[s];
-        L.sDY[rk[s]] = tDY[s];
-        L.sLY[rk[s]] = tLY[s];
-        L.sM[rk[s]] = tM[s];
-      }
-    }
-    WaveSync();
-    load_from_scratch(k);
-    n = k;
-    pp = k;
-    int mn = kMaxS32;
-#pragma unroll
-    for (int s = 0; s < K; s++) {
-      int p = s * kWave + lane;
-      if (p < n && LY[s] > y) mn = Min32(mn, LY[s]);
-    }
-    nny = WaveMin(mn);
-    Fixed nu = pending_upper(pp);
+    load_window(0);
+    if (!insert_new(y, true)) flags |= 2;
+    const Fixed nu = pending_upper();
     if (nu > y && nu < nny) nny = nu;
-    WaveSync();
   }
 
   const Fixed stop_fixed = IntToFixed(pb.b);
   int guard = 0;
-  uint64_t ph[5] = {0, 0, 0, 0, 0};  // phase times (10 ns units)
-  uint64_t tp_loop = wall_clock64();
+  // Phase times (10 ns units) of every 16th step: reading the clock waits for
+  // it and for the LDS operations in flight, which took a third of a small
+  // step when every step did it five times.
+  uint64_t ph[5] = {0, 0, 0, 0, 0};
+  const uint64_t tp_loop = wall_clock64();
   int next_b = 1;  // next band snapshot to record (count / schedule passes)
   for (;;) {
     if (y >= stop_y) break;  // the next band starts here
@@ -721,7 +935,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
             a[2 * CAP + p] = DY[s];
             a[3 * CAP + p] = LY[s];
             a[4 * CAP + p] = M[s];
-            if (MetaQuad(M[s])) qs[p] = Q[MetaIndex(M[s])];
+            if (MetaMoved(M[s])) qs[p] = Q[MetaIndex(M[s])];
           }
         }
         next_b++;
@@ -731,6 +945,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
       flags |= 32;
       break;
     }
+    const bool sample = (guard & 15) == 1;
     max_active = Max32(max_active, n);
     Fixed next_y = Min32(nny, FixedCeilToFixed(y + 1));
     int y_shift = 0;
@@ -743,137 +958,141 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
     const Alpha full = (Alpha)FixedRoundToInt(0xFF * (next_y - y));
     const int row = y >> 16;
     const int S = (n + kWave - 1) / kWave;
+    // rows off the canvas are stepped but not drawn
+    const bool draw = kBlit && row >= cy0 && row < cy1;
 
-    uint64_t tp0 = wall_clock64();
-    Fixed XN[K];
-    if (!kBlit) {
+    uint64_t tp0 = 0, tp1 = 0, tp2 = 0, tp3 = 0, tp4 = 0;
+    if (sample) tp0 = wall_clock64();
+    // ---- one pass over the list: interval edges, step, order checks -----------
+    // An edge opens or closes an interval where the winding sum up to it
+    // changes between inside and outside.  The k-th opening edge belongs to
+    // the k-th closing one, so both kinds are packed into LDS in list order
+    // and interval k reads entries k (and k - 1 for the interval before).
+    // Windings are counted from ballots: no scan.  The step itself and the
+    // two order checks (is the stepped list still sorted, does an edge cross
+    // its predecessor within the next step) use the same registers; when no
+    // edge ends and the order holds, which is most steps, the step is done.
+    uint64_t ends = 0;
+    bool bad = false, cross = false;
+    int carry_w = 0, nl = 0, nr = 0;
+    uint64_t carry_in = 0;
+    {
+      Fixed cx = kMinS32, cv = kMinS32;
 #pragma unroll
-      for (int s = 0; s < K; s++) XN[s] = X[s] + (DX[s] >> y_shift);
-    }
-    // ---- phases 1-3: roles, trapezoids --------------------------------------
-    if (kBlit) {
-    int carry_w = 0;
-    int carry_in = 0;
-    int carry_lidx = -1;
-    Fixed carry_lxo = 0, carry_lxn = 0, carry_ldy = 0;
-    int carry_ridx = -1;
-    Fixed carry_rxo = 0, carry_rxn = 0;
-#pragma unroll
-    for (int s = 0; s < K; s++) {
-      if (s >= S) break;
-      int p = s * kWave + lane;
-      bool valid = p < n;
-      int wv = valid ? MetaWinding(M[s]) : 0;
-      int incl = ScanSum(wv) + carry_w;
-      int in = (valid && (incl & winding_mask) != 0) ? 1 : 0;
-      int prev_in = ShiftUp(in, carry_in);
-      bool is_left = valid && in && !prev_in;
-      bool is_right = valid && !in && prev_in;
-      Fixed xo = X[s];
-      Fixed xn = valid ? xo + (DX[s] >> y_shift) : 0;
-      XN[s] = xn;
-      // nearest left edge at or before p
-      int lsel = ScanMax(is_left ? lane : -1);
-      Fixed lxo = __shfl(xo, lsel < 0 ? 0 : lsel, kWave);
-      Fixed lxn = __shfl(xn, lsel < 0 ? 0 : lsel, kWave);
-      Fixed ldy = __shfl(DY[s], lsel < 0 ? 0 : lsel, kWave);
-      if (lsel < 0) {
-        lxo = carry_lxo;
-        lxn = carry_lxn;
-        ldy = carry_ldy;
-      }
-      // previous right edge strictly before p
-      int rsel_incl = ScanMax(is_right ? lane : -1);
-      int rsel = ShiftUp(rsel_incl, -1);
-      Fixed rxo = __shfl(xo, rsel < 0 ? 0 : rsel, kWave);
-      Fixed rxn = __shfl(xn, rsel < 0 ? 0 : rsel, kWave);
-      bool has_prev_right = rsel >= 0 || carry_ridx >= 0;
-      if (rsel < 0) {
-        rxo = carry_rxo;
-        rxn = carry_rxn;
-      }
-      // next element (old x, dx); lane 63's successor is lane 0 of slot s+1
-      Fixed nxo = ShiftDown(xo, xo), ndx = ShiftDown(DX[s], DX[s]);
-      int next_p = p + 1;
-      if (s + 1 < K) {
-        Fixed n0x = __builtin_amdgcn_readlane(X[s + 1 < K ? s + 1 : s], 0);
-        Fixed n0dx = __builtin_amdgcn_readlane(DX[s + 1 < K ? s + 1 : s], 0);
-        if (lane == kWave - 1) {
-          nxo = n0x;
-          ndx = n0dx;
+      for (int s = 0; s < K; s++) {
+        if (s >= S) break;
+        const int rem = n - s * kWave;
+        const uint64_t bval = rem >= kWave ? ~0ull : (1ull << rem) - 1;
+        const bool valid = lane < rem;
+        const Fixed xo = X[s], dx = DX[s];
+        const Fixed xn = xo + (dx >> y_shift);
+        if (draw) {
+          const bool neg = (M[s] & 1) != 0;
+          const uint64_t bneg = __ballot(neg) & bval, bpos = bval & ~bneg;
+          const int incl = CountBelow(bpos, carry_w) - CountBelow(bneg) + (neg ? -1 : 1);
+          const uint64_t bin = __ballot((incl & winding_mask) != 0) & bval;
+          const uint64_t prev = (bin << 1) | carry_in;
+          const uint64_t bl = bin & ~prev, br = bval & ~bin & prev;
+          // the next element (old x, dx); lane 63's is lane 0 of slot s + 1
+          Fixed nxo = ShiftDown(xo, xo), ndx = ShiftDown(dx, dx);
+          if (s + 1 < K) {
+            const Fixed n0x = __builtin_amdgcn_readlane(X[s + 1 < K ? s + 1 : s], 0);
+            const Fixed n0dx = __builtin_amdgcn_readlane(DX[s + 1 < K ? s + 1 : s], 0);
+            if (lane == kWave - 1) {
+              nxo = n0x;
+              ndx = n0dx;
+            }
+          }
+          if (__builtin_amdgcn_inverse_ballot_w64(bl))
+            L.iL[CountBelow(bl, nl)] = make_int4(xo, xn, DY[s], 0);
+          if (__builtin_amdgcn_inverse_ballot_w64(br)) {
+            const bool close = lane + 1 < rem && (xn + kFixed1 >= nxo - Abs32(ndx));
+            L.iR[CountBelow(br, nr)] = make_int4(xo, xn, DY[s], close ? 1 : 0);
+          }
+          nl += __popcll(bl);
+          nr += __popcll(br);
+          carry_w += __popcll(bpos) - __popcll(bneg);
+          carry_in = (bin >> ((rem >= kWave ? kWave : rem) - 1)) & 1;
         }
-      }
-      bool next_active = next_p < n;
-      if (is_right) {
-        Fixed left = Max32(lxo, left_clip);
-        Fixed right = Min32(right_clip, xo);
-        Fixed next_left = Max32(left_clip, lxn);
-        Fixed next_right = Min32(right_clip, xn);
-        int prev_right = has_prev_right
-                             ? FixedCeilToInt(Max32(Min32(right_clip, rxo), rxn))
-                             : FixedFloorToInt(left_clip);
-        bool too_close_prev =
-            prev_right > FixedFloorToInt(left) || prev_right > FixedFloorToInt(lxn);
-        bool too_close_next = next_active && (xn + kFixed1 >= nxo - Abs32(ndx));
-        bool no_real = full == 0xFF && (too_close_prev || too_close_next);
-        BlitTrapezoidRow(&sink, left, right, next_left, next_right, ldy, DY[s], full,
-                         no_real);
-        int lo = FixedFloorToInt(Min32(Min32(left, next_left), Min32(right, next_right))) - ox;
-        int hi = FixedCeilToInt(Max32(Max32(left, next_left), Max32(right, next_right))) - ox;
-        dmin = Min32(dmin, Max32(lo, 0));
-        dmax = Max32(dmax, Min32(hi, W));
-      }
-      // carries
-      carry_w = __builtin_amdgcn_readlane(incl, kWave - 1);
-      carry_in = __builtin_amdgcn_readlane(in, kWave - 1);
-      int lastl = __builtin_amdgcn_readlane(lsel, kWave - 1);
-      if (lastl >= 0) {
-        carry_lidx = s * kWave + lastl;
-        carry_lxo = __builtin_amdgcn_readlane(xo, lastl);
-        carry_lxn = __builtin_amdgcn_readlane(xn, lastl);
-        carry_ldy = __builtin_amdgcn_readlane(DY[s], lastl);
-      }
-      int lastr = __builtin_amdgcn_readlane(rsel_incl, kWave - 1);
-      if (lastr >= 0) {
-        carry_ridx = s * kWave + lastr;
-        carry_rxo = __builtin_amdgcn_readlane(xo, lastr);
-        carry_rxn = __builtin_amdgcn_readlane(xn, lastr);
+        ends |= __ballot(LY[s] <= next_y) & bval;
+        X[s] = xn;
+        const Fixed v = xn + dx;
+        const Fixed px = ShiftUp(xn, cx), pv = ShiftUp(v, cv);
+        bad |= valid && px > xn;
+        cross |= valid && pv > v;
+        cx = __builtin_amdgcn_readlane(xn, kWave - 1);
+        cv = __builtin_amdgcn_readlane(v, kWave - 1);
       }
     }
-    // open interval at the end of the list (right edge culled away)
-    if (carry_in) {
-      flags |= 8;
-      // The reference tests edges_too_close(left_edge->prev, left_edge);
-      // with a closed path the winding sum is 0 here, so this is not reached
-      // on the parity scenes.  The left edge's list predecessor is not
-      // tracked; the span is emitted as accumulated coverage.
-      Fixed left = Max32(carry_lxo, left_clip);
-      if (lane == 0) {
-        BlitTrapezoidRow(&sink, left, right_clip, Max32(left_clip, carry_lxn), right_clip,
-                         carry_ldy, 0, full, full == 0xFF);
-        int lo = FixedFloorToInt(Min32(left, Max32(left_clip, carry_lxn))) - ox;
-        dmin = Min32(dmin, Max32(lo, 0));
-        dmax = Max32(dmax, W);
+    // ---- the step's trapezoids -------------------------------------------------
+    if (draw) {
+      if (carry_in) {
+        // open interval at the end of the list (right edge culled away): it
+        // runs to the right clip.  The reference tests
+        // edges_too_close(left_edge->prev, left_edge); with a closed path the
+        // winding sum is 0 here, so this is not reached on the parity scenes.
+        // The left edge's list predecessor is not tracked; the span is
+        // emitted as accumulated coverage.
+        flags |= 8;
+        if (lane == 0) L.iR[nr] = make_int4(right_clip, right_clip, 0, 1);
+        nr++;
       }
+      WaveSync();
+      for (int k0 = 0; k0 < nr; k0 += kWave) {
+        const int k = k0 + lane;
+        const bool act = k < nr;
+        int4 l = make_int4(0, 0, 0, 0), r = l, q = l;
+        if (act) {
+          l = L.iL[k];
+          r = L.iR[k];
+          if (k > 0) q = L.iR[k - 1];
+        }
+        const Fixed left = Max32(l.x, left_clip), next_left = Max32(left_clip, l.y);
+        const Fixed right = Min32(right_clip, r.x), next_right = Min32(right_clip, r.y);
+        const int prev_right = k > 0 ? FixedCeilToInt(Max32(Min32(right_clip, q.x), q.y))
+                                     : FixedFloorToInt(left_clip);
+        const bool close_prev =
+            prev_right > FixedFloorToInt(left) || prev_right > FixedFloorToInt(l.y);
+        const bool no_real = full == 0xFF && (close_prev || r.w != 0);
+        if (act) {
+          const int lo = FixedFloorToInt(Min32(Min32(left, next_left), Min32(right, next_right)));
+          const int hi = FixedCeilToInt(Max32(Max32(left, next_left), Max32(right, next_right)));
+          dmin = Min32(dmin, Max32(lo - ox, 0));
+          dmax = Max32(dmax, Min32(hi - ox, W));
+        }
+        BlitIntervals(sink, L.blit, act, left, right, next_left, next_right, l.z, r.z, full,
+                      no_real);
+      }
+      WaveSync();
     }
-    WaveSync();
-    }  // kBlit
 
-    uint64_t tp1 = wall_clock64();
-    ph[0] += tp1 - tp0;
-    // ---- phase 4: GoY and quad updates -----------------------------------------
+    if (sample) {
+      tp1 = wall_clock64();
+      ph[0] += tp1 - tp0;
+    }
+    // ---- quad updates ------------------------------------------------------------
+    int m = n;
+    uint64_t dead = 0;
+    if (ends != 0) {
 #pragma unroll
-    for (int s = 0; s < K; s++) {
-      if (s >= S) break;
-      int p = s * kWave + lane;
-      if (p < n) {
-        X[s] = XN[s];
-        if (LY[s] <= next_y && MetaQuad(M[s])) {
+      for (int s = 0; s < K; s++) {
+        if (s >= S) break;
+        int p = s * kWave + lane;
+        if (p < n && LY[s] <= next_y && MetaQuad(M[s])) {
           // while (lower_y <= next_y) { KeepContinuous; UpdateQuad } with
           // KeepContinuous taking the edge's current x and y
           // (sw_raster.cc:628-638, sw_edge.cc:294-297).
-          int idx = MetaIndex(M[s]);
-          EdgeRec e = Q[idx];
+          const int idx = MetaIndex(M[s]);
+          EdgeRec e;
+          {
+            const int4* src = (const int4*)(MetaMoved(M[s]) ? (const EdgeRec*)&Q[idx] : &E[idx]);
+            int4* dst = (int4*)&e;
+            const int4 q0 = src[0], q1 = src[1], q2 = src[2], q3 = src[3];
+            dst[0] = q0;
+            dst[1] = q1;
+            dst[2] = q2;
+            dst[3] = q3;
+          }
           Fixed sy = next_y;
           Fixed cx = X[s];
           while (LY[s] <= next_y && EdgeCurveCount(e.packed) > 0) {
@@ -886,91 +1105,87 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
             LY[s] = e.lower_y;
           }
           X[s] = cx;
-          M[s] = MakeMeta(EdgeWinding(e.packed), true, idx);
+          M[s] = MakeMeta(EdgeWinding(e.packed), true, true, idx);
           Q[idx] = e;
+        }
+        dead |= __ballot(p < n && LY[s] <= next_y);
+      }
+      if (dead == 0) {
+        // every edge lives on: check the order in place
+        bad = false;
+        cross = false;
+        Fixed cx = kMinS32, cv = kMinS32;
+#pragma unroll
+        for (int s = 0; s < K; s++) {
+          if (s >= S) break;
+          const bool valid = s * kWave + lane < n;
+          const Fixed v = X[s] + DX[s];
+          const Fixed px = ShiftUp(X[s], cx), pv = ShiftUp(v, cv);
+          bad |= valid && px > X[s];
+          cross |= valid && pv > v;
+          cx = __builtin_amdgcn_readlane(X[s], kWave - 1);
+          cv = __builtin_amdgcn_readlane(v, kWave - 1);
         }
       }
     }
 
-    uint64_t tp2 = wall_clock64();
-    ph[1] += tp2 - tp1;
-    // ---- phases 5-6: survivors, stable x order, intersection checks ----------
-    int m = 0;
+    if (sample) {
+      tp2 = wall_clock64();
+      ph[1] += tp2 - tp1;
+    }
+    // ---- survivors, stable x order, intersection checks ------------------------
     bool flag_isect = false;
-    {
-      int cnt_carry = 0;
-      bool sorted = true;
-      Fixed prevX_carry = kMinS32;
-      bool has_prev_carry = false;
-      int C[K];
-      bool SV[K];
+    if (dead == 0 && __ballot(bad) == 0) {
+      flag_isect = __ballot(cross) != 0;
+    } else {
+      // write the survivors to scratch in list order
+      m = 0;
 #pragma unroll
       for (int s = 0; s < K; s++) {
         if (s >= S) break;
         int p = s * kWave + lane;
-        bool sv = p < n && LY[s] > next_y;
-        SV[s] = sv;
-        int inc = ScanSum(sv ? 1 : 0);
-        C[s] = cnt_carry + inc - (sv ? 1 : 0);
-        // previous survivor's x
-        int psel_incl = ScanMax(sv ? lane : -1);
-        int psel = ShiftUp(psel_incl, -1);
-        Fixed px = __shfl(X[s], psel < 0 ? 0 : psel, kWave);
-        Fixed pdx = __shfl(DX[s], psel < 0 ? 0 : psel, kWave);
-        bool hp = psel >= 0;
-        if (!hp) {
-          px = prevX_carry;
-          hp = has_prev_carry;
-        }
-        if (sv && hp && X[s] < px) sorted = false;
-        (void)pdx;
-        int lastp = __builtin_amdgcn_readlane(psel_incl, kWave - 1);
-        if (lastp >= 0) {
-          prevX_carry = __builtin_amdgcn_readlane(X[s], lastp);
-          has_prev_carry = true;
-        }
-        cnt_carry += __builtin_amdgcn_readlane(inc, kWave - 1);
-      }
-      m = cnt_carry;
-      bool all_sorted = __ballot(!sorted) == 0;
-      if (all_sorted && m == n) {
-        // every edge survives in place: the predecessor of element p is
-        // p - 1 (check_intersection against the previous element)
-        bool f = false;
-        Fixed carry_v = 0;
-#pragma unroll
-        for (int s = 0; s < K; s++) {
-          if (s >= S) break;
-          int p = s * kWave + lane;
-          Fixed v = X[s] + DX[s];
-          Fixed pv = ShiftUp(v, carry_v);
-          if (p >= 1 && p < n && pv > v) f = true;
-          carry_v = __builtin_amdgcn_readlane(v, kWave - 1);
-        }
-        flag_isect = __ballot(f) != 0;
-      } else {
-      // write survivors to scratch in survivor order
-#pragma unroll
-      for (int s = 0; s < K; s++) {
-        if (s >= S) break;
-        if (SV[s]) {
-          int c = C[s];
+        const bool sv = p < n && LY[s] > next_y;
+        const uint64_t b = __ballot(sv);
+        if (sv) {
+          const int c = CountBelow(b, m);
           L.sX[c] = X[s];
           L.sDX[c] = DX[s];
           L.sDY[c] = DY[s];
           L.sLY[c] = LY[s];
           L.sM[c] = M[s];
         }
+        m += __popcll(b);
       }
       WaveSync();
-      if (all_sorted) {
-        // predecessor = previous survivor
-        bool f = false;
-        for (int c = lane + 1; c < m; c += kWave) {
-          if (L.sX[c - 1] + L.sDX[c - 1] > L.sX[c] + L.sDX[c]) f = true;
+      const int S2 = (m + kWave - 1) / kWave;
+      bad = false;
+      cross = false;
+#pragma unroll
+      for (int s = 0; s < K; s++) {
+        if (s >= S2) break;
+        const int c = s * kWave + lane;
+        if (c < m) {
+          X[s] = L.sX[c];
+          DX[s] = L.sDX[c];
+          if (c > 0) {
+            const Fixed px = L.sX[c - 1], pdx = L.sDX[c - 1];
+            bad |= px > X[s];
+            cross |= px + pdx > X[s] + DX[s];
+          }
         }
-        flag_isect = __ballot(f) != 0;
-        load_from_scratch(m);
+      }
+      if (__ballot(bad) == 0) {
+        flag_isect = __ballot(cross) != 0;
+#pragma unroll
+        for (int s = 0; s < K; s++) {
+          if (s >= S2) break;
+          const int c = s * kWave + lane;
+          if (c < m) {
+            DY[s] = L.sDY[c];
+            LY[s] = L.sLY[c];
+            M[s] = L.sM[c];
+          }
+        }
       } else {
         // Stable re-sort by x.  The survivors stay in scratch in list order;
         // only the keys (x, list position) are sorted in registers, by
@@ -979,12 +1194,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
         // passes do not; then the other fields are gathered by position.
         int O[K];
 #pragma unroll
-        for (int s = 0; s < K; s++) {
-          int p = s * kWave + lane;
-          O[s] = p;
-          if (p < m) X[s] = L.sX[p];
-        }
-        const int S2 = (m + kWave - 1) / kWave;
+        for (int s = 0; s < K; s++) O[s] = s * kWave + lane;
         auto gt_key = [](Fixed xa, int oa, Fixed xb, int ob) {
           return xa > xb || (xa == xb && oa > ob);
         };
@@ -996,8 +1206,8 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
             if (s >= S2) break;
             int p = s * kWave + lane;
             int q = p ^ 1;
-            Fixed ox = __shfl_xor(X[s], 1, kWave);
-            int oo = __shfl_xor(O[s], 1, kWave);
+            Fixed ox = DppSwapPairs(X[s]);
+            int oo = DppSwapPairs(O[s]);
             bool both = p < m && q < m;
             bool left = (lane & 1) == 0;
             bool take = both && (left ? gt_key(X[s], O[s], ox, oo) : gt_key(ox, oo, X[s], O[s]));
@@ -1019,8 +1229,8 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
             int q = left ? p + 1 : p - 1;
             const Fixed c63x = __builtin_amdgcn_readlane(X[s], kWave - 1);
             const int c63o = __builtin_amdgcn_readlane(O[s], kWave - 1);
-            Fixed dnx = ShiftDown(X[s], 0), upx = ShiftUp(X[s], 0);
-            int dno = ShiftDown(O[s], 0), upo = ShiftUp(O[s], 0);
+            Fixed dnx = ShiftDown(X[s], 0), upx = ShiftUp(X[s], p63x);
+            int dno = ShiftDown(O[s], 0), upo = ShiftUp(O[s], p63o);
             if (s + 1 < K) {
               const int t = s + 1 < K ? s + 1 : s;
               const Fixed n0x = __builtin_amdgcn_readlane(X[t], 0);
@@ -1029,10 +1239,6 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
                 dnx = n0x;
                 dno = n0o;
               }
-            }
-            if (lane == 0) {
-              upx = p63x;
-              upo = p63o;
             }
             bool both = p < m && q >= 0 && q < m;
             bool take = both && (left ? gt_key(X[s], O[s], dnx, dno) : gt_key(upx, upo, X[s], O[s]));
@@ -1044,8 +1250,8 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
             p63o = c63o;
           }
           // sorted when every element exceeds its predecessor
-          bool bad = false;
-          Fixed cx = 0;
+          bool worse = false;
+          Fixed cx = kMinS32;
           int co = 0;
 #pragma unroll
           for (int s = 0; s < K; s++) {
@@ -1053,11 +1259,11 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
             int p = s * kWave + lane;
             Fixed px = ShiftUp(X[s], cx);
             int po = ShiftUp(O[s], co);
-            if (p >= 1 && p < m && gt_key(px, po, X[s], O[s])) bad = true;
+            if (p >= 1 && p < m && gt_key(px, po, X[s], O[s])) worse = true;
             cx = __builtin_amdgcn_readlane(X[s], kWave - 1);
             co = __builtin_amdgcn_readlane(O[s], kWave - 1);
           }
-          sorted = __ballot(bad) == 0;
+          sorted = __ballot(worse) == 0;
         }
         if (!sorted) {
           // bitonic sort of the keys (x, list position)
@@ -1084,6 +1290,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
         // the other fields, by list position
 #pragma unroll
         for (int s = 0; s < K; s++) {
+          if (s >= S2) break;
           int c = s * kWave + lane;
           if (c < m) {
             DX[s] = L.sDX[O[s]];
@@ -1098,10 +1305,10 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
         // smaller (edges that moved in front of it were processed later).
 #pragma unroll
         for (int s = 0; s < K; s++) {
+          if (s >= S2) break;
           int c = s * kWave + lane;
           if (c < m) {
-            L.sX[c] = X[s];
-            L.sDX[c] = DX[s];
+            L.sX[c] = X[s] + DX[s];
             L.sLY[c] = O[s];
           }
         }
@@ -1109,214 +1316,56 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
         bool f = false;
 #pragma unroll
         for (int s = 0; s < K; s++) {
+          if (s >= S2) break;
           int c = s * kWave + lane;
           if (c < m) {
             int q = c - 1;
             while (q >= 0 && L.sLY[q] > O[s]) q--;
-            if (q >= 0 && L.sX[q] + L.sDX[q] > X[s] + DX[s]) f = true;
+            if (q >= 0 && L.sX[q] > X[s] + DX[s]) f = true;
           }
         }
         flag_isect = __ballot(f) != 0;
       }
       WaveSync();
-      }  // survivors moved
     }
     n = m;
-    {
+    if (ends != 0) {
+      // the smallest lower_y changes only when an edge ends or moves on
       int mn = kMaxS32;
 #pragma unroll
       for (int s = 0; s < K; s++) {
+        if (s * kWave >= n) break;
         int p = s * kWave + lane;
         if (p < n) mn = Min32(mn, LY[s]);
       }
-      nny = WaveMin(mn);
-      if (flag_isect) nny = next_y + (kFixed1 >> kAcc);
+      min_ly = DppWaveMin(mn);
     }
+    nny = flag_isect ? next_y + (kFixed1 >> kAcc) : min_ly;
 
-    uint64_t tp3 = wall_clock64();
-    ph[2] += tp3 - tp2;
+    if (sample) {
+      tp3 = wall_clock64();
+      ph[2] += tp3 - tp2;
+    }
     // ---- row completion ------------------------------------------------------
     y = next_y;
     if (kBlit && (y & 0xFFFF) == 0) flush_row(row);
-    uint64_t tp4 = wall_clock64();
-    ph[3] += tp4 - tp3;
+    if (sample) {
+      tp4 = wall_clock64();
+      ph[3] += tp4 - tp3;
+    }
     if (y >= stop_fixed) break;
 
-    // ---- phase 7: insert new edges (insert_new_edges) --------------------------
-    Fixed nu = pending_upper(pp);
+    // ---- insert new edges (insert_new_edges) -----------------------------------
+    Fixed nu = pending_upper();
     if (nu <= y) {
-      int k;
-      if (!gather_new(y, &k) || n + k > CAP) {
+      if (!insert_new(y, false)) {
         flags |= 2;
         break;
       }
-      WaveSync();
-      // sort the new edges by (x, dx, sorted position)
-      int rk[K];
-      Fixed tX[K], tDX[K], tDY[K], tLY[K];
-      int tM[K];
-#pragma unroll
-      for (int s = 0; s < K; s++) {
-        int p = s * kWave + lane;
-        rk[s] = 0;
-        if (p < k) {
-          Fixed xi = L.sX[p], dxi = L.sDX[p];
-          int r = 0;
-          for (int q = 0; q < k; q++) {
-            Fixed xq = L.sX[q], dxq = L.sDX[q];
-            r += (xq < xi || (xq == xi && (dxq < dxi || (dxq == dxi && q < p)))) ? 1 : 0;
-          }
-          rk[s] = r;
-          tX[s] = L.sX[p];
-          tDX[s] = L.sDX[p];
-          tDY[s] = L.sDY[p];
-          tLY[s] = L.sLY[p];
-          tM[s] = L.sM[p];
-        }
-      }
-      WaveSync();
-#pragma unroll
-      for (int s = 0; s < K; s++) {
-        int p = s * kWave + lane;
-        if (p < k) {
-          L.sX[rk[s]] = tX[s];
-          L.sDX[rk[s]] = tDX[s];
-          L.sDY[rk[s]] = tDY[s];
-          L.sLY[rk[s]] = tLY[s];
-          L.sM[rk[s]] = tM[s];
-        }
-      }
-      WaveSync();
-      // insertion positions: P1 = #{a : x_a <= x_N1};
-      // Pi = max(P(i-1), #{a : x_a < x_Ni}).
-      // The new edges are at scratch[0..k); positions go to sLY? keep in regs
-      int Pcur = 0;
-      bool fnew = false;
-      int posN[K];
-#pragma unroll
-      for (int s = 0; s < K; s++) posN[s] = 0;
-      for (int i = 0; i < k; i++) {
-        Fixed xi = L.sX[i];
-        int cnt = 0;
-#pragma unroll
-        for (int s = 0; s < K; s++) {
-          int p = s * kWave + lane;
-          bool v = p < n && (i == 0 ? X[s] <= xi : X[s] < xi);
-          cnt += __popcll(__ballot(v));
-        }
-        int Pi = i == 0 ? cnt : Max32(Pcur, cnt);
-        // predecessor at insertion: N(i-1) if it sits right before, else A[Pi-1]
-        Fixed predx = 0, preddx = 0;
-        bool has_pred = false;
-        if (i > 0 && Pi == Pcur) {
-          predx = L.sX[i - 1];
-          preddx = L.sDX[i - 1];
-          has_pred = true;
-        } else if (Pi > 0) {
-          int q = Pi - 1;
-          // q is the same for every lane: read the element from its slot
-          const int s = __builtin_amdgcn_readfirstlane(q / kWave);
-          const int ln = __builtin_amdgcn_readfirstlane(q % kWave);
-          Fixed ax = 0, adx = 0;
-#pragma unroll
-          for (int t = 0; t < K; t++) {
-            if (t == s) {
-              ax = __builtin_amdgcn_readlane(X[t], ln);
-              adx = __builtin_amdgcn_readlane(DX[t], ln);
-            }
-          }
-          predx = ax;
-          preddx = adx;
-          has_pred = true;
-        }
-        if (has_pred && predx + preddx > L.sX[i] + L.sDX[i]) fnew = true;
-        if (i % kWave == lane) {
-#pragma unroll
-          for (int s = 0; s < K; s++)
-            if (s == i / kWave) posN[s] = Pi + i;
-        }
-        Pcur = Pi;
-      }
-      if (fnew) nny = y + (kFixed1 >> kAcc);
-      // lower_y of new edges
-      {
-        int mn = kMaxS32;
-#pragma unroll
-        for (int s = 0; s < K; s++) {
-          int p = s * kWave + lane;
-          if (p < k) mn = Min32(mn, L.sLY[p]);
-        }
-        mn = WaveMin(mn);
-        if (mn > y && mn < nny) nny = mn;
-      }
-      // merge: A[q] moves to q + #{i : P_i <= q}; N_i goes to P_i + i
-      // P_i are stored as posN - i; count with a loop over i
-      Fixed nX[K], nDX[K], nDY[K], nLY[K];
-      int nM[K];
-#pragma unroll
-      for (int s = 0; s < K; s++) {
-        int p = s * kWave + lane;
-        if (p < k) {
-          nX[s] = L.sX[p];
-          nDX[s] = L.sDX[p];
-          nDY[s] = L.sDY[p];
-          nLY[s] = L.sLY[p];
-          nM[s] = L.sM[p];
-        }
-      }
-      // P_i broadcast through LDS (reuse sLY region after reading)
-      WaveSync();
-#pragma unroll
-      for (int s = 0; s < K; s++) {
-        int p = s * kWave + lane;
-        if (p < k) L.sLY[CAP - 1 - p] = posN[s] - p;  // P_p, stored from the end
-      }
-      WaveSync();
-      int shiftA[K];
-#pragma unroll
-      for (int s = 0; s < K; s++) {
-        int q = s * kWave + lane;
-        int c = 0;
-        if (q < n) {
-          for (int i = 0; i < k; i++) c += (L.sLY[CAP - 1 - i] <= q) ? 1 : 0;
-        }
-        shiftA[s] = c;
-      }
-      WaveSync();
-#pragma unroll
-      for (int s = 0; s < K; s++) {
-        int q = s * kWave + lane;
-        if (q < n) {
-          int d = q + shiftA[s];
-          L.sX[d] = X[s];
-          L.sDX[d] = DX[s];
-          L.sDY[d] = DY[s];
-          L.sLY[d] = LY[s];
-          L.sM[d] = M[s];
-        }
-      }
-#pragma unroll
-      for (int s = 0; s < K; s++) {
-        int p = s * kWave + lane;
-        if (p < k) {
-          int d = posN[s];
-          L.sX[d] = nX[s];
-          L.sDX[d] = nDX[s];
-          L.sDY[d] = nDY[s];
-          L.sLY[d] = nLY[s];
-          L.sM[d] = nM[s];
-        }
-      }
-      WaveSync();
-      n += k;
-      pp += k;
-      load_from_scratch(n);
-      WaveSync();
-      Fixed nu2 = pending_upper(pp);
-      if (nu2 > y && nu2 < nny) nny = nu2;
-    } else if (nu > y && nu < nny) {
-      nny = nu;
+      nu = pending_upper();
     }
+    if (nu > y && nu < nny) nny = nu;
+    if (sample) ph[4] += wall_clock64() - tp4;
   }
   finish_band();
   if (!kWrite) {
@@ -1330,7 +1379,15 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
   if (lane == 0) {
     uint64_t t_end = wall_clock64();
     uint64_t dt = t_end - t_start;
-    ph[4] = (t_end - tp_loop) - (ph[0] + ph[1] + ph[2] + ph[3]);
+    // the sampled steps' split, scaled to the whole walk
+    uint64_t sampled = 0;
+    for (int k = 0; k < 5; k++) sampled += ph[k];
+    if (sampled > 0) {
+      const double scale = (double)(t_end - tp_loop) / (double)sampled;
+      for (int k = 0; k < 5; k++) ph[k] = (uint64_t)((double)ph[k] * scale);
+    } else {
+      ph[4] = t_end - tp_loop;
+    }
     int32_t dt32 = (int32_t)(dt < 0x7FFFFFFF ? dt : 0x7FFFFFFF);
     if (kWrite) {
       JobCov* c = &P.cov[j];

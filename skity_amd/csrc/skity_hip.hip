@@ -1113,11 +1113,8 @@ constexpr int kBandMinEdges = 4 * kWave + 1;
 constexpr int kBandMinRows = 512;
 constexpr int kBandSlots = 512;
 
-// LDS of a walk wave: row deltas, three per-tile-column rows (two slots,
-// written rows), five scratch arrays of K * 64 entries.
 size_t WalkLdsBytes(int K, int lds_width) {
-  return (size_t)((lds_width + 1) + 3 * (lds_width / kTile + 2) + 5 * K * kWave) *
-         sizeof(int32_t);
+  return (size_t)WalkLdsInts(K, lds_width) * sizeof(int32_t);
 }
 
 hipr_result WalkLdsCheck(hipr_context ctx, int K, size_t lds) {
