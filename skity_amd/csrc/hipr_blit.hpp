@@ -30,7 +30,8 @@ constexpr int kDirectCount = 1 << 12;  // one direct span, in the D field
 // which no visible pixel's prefix sum reads, so every visible pixel sums the
 // same deltas as over the path's full width.
 struct RowSink {
-  int32_t* d;
+  int32_t* d;       // the delta entry of the first visible column
+  uint32_t* touch;  // a bit per tile column, from the first visible column's
   int32_t left;   // pixel x of delta index 0 (the first visible column)
   int32_t width;  // visible columns; entry `width` is the end-of-row entry
   // Direct spans of cover 0 blend nothing in src-over, and are dropped; a
@@ -42,6 +43,18 @@ struct RowSink {
     if (v == 0) return;
     const int i = x - left;
     atomicAdd(&d[i < 0 ? 0 : (i > width ? width : i)], v);
+  }
+  // Marks the tile columns of the deltas at pixels a .. b (clamped into the
+  // row) as touched.
+  __device__ __forceinline__ void Touch(int a, int b) {
+    const int c0 = left >> 4;
+    const int lo = (Min32(Max32(a, left), left + width) >> 4) - c0;
+    const int hi = (Min32(Max32(b, left), left + width) >> 4) - c0;
+    for (int w = lo >> 5; w <= hi >> 5; w++) {
+      const uint32_t from = w == lo >> 5 ? ~0u << (lo & 31) : ~0u;
+      const uint32_t to = w == hi >> 5 ? (2u << (hi & 31)) - 1 : ~0u;
+      atomicOr(&touch[w], from & to);
+    }
   }
   // A one-pixel span of cover v at a visible pixel.
   __device__ __forceinline__ void Pixel(bool direct, int x, int v) {
@@ -236,8 +249,11 @@ __device__ __forceinline__ void BlitIntervals(RowSink& s, const BlitScratch& L, 
       const int run = join_left < join_rite ? inc(full) : 0;
       s.Add(JL, run - last);
       s.Add(JR, first - run);
+      s.Touch(x0, JL);
+      s.Touch(JR, FixedCeilToInt(lr));
     } else {
       const int R = FixedCeilToInt(lr);
+      s.Touch(x0, R);
       if (R - x0 == 1) {
         const int v = part(TrapezoidToAlpha(ur - ul, lr - ll));
         s.Add(x0, v);

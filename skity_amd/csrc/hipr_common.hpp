@@ -80,7 +80,8 @@ __host__ __device__ inline bool ClipIsCull(const float c[4]) {
 struct JobCov {
   int32_t left, top, right, bottom;   // floored/ceiled bounds (pixels)
   int32_t tiles;        // coverage tiles written
-  int32_t planes;       // coverage planes written (>= tiles)
+  int32_t planes;       // coverage planes (>= tiles; a solid tile counts as one)
+  int32_t alloc;        // planes taken from the job's range and the pool
   int32_t max_active;
   int32_t flags;        // bit0 plane overflow, bit1 active overflow,
                         // bit2 stacked direct spans, bit3 open interval
@@ -196,6 +197,10 @@ __device__ __forceinline__ int DppScanMax(int v) {
 // Lanes 2i and 2i + 1 trade places (quad_perm 1, 0, 3, 2).
 __device__ __forceinline__ int DppSwapPairs(int v) {
   return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true);
+}
+// The lane pairs of each four lanes trade places (quad_perm 2, 3, 0, 1).
+__device__ __forceinline__ int DppSwapHalves(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, true);
 }
 // Smallest value of the wave, in every lane.
 __device__ __forceinline__ int DppWaveMin(int v) {

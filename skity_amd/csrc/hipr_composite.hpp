@@ -570,7 +570,7 @@ __global__ void __launch_bounds__(64) CompositeKernel(CompositeParams P) {
         } else {
           int64_t mi = P.map_base[j] + (int64_t)(ty - tb.y) * (tb.z - tb.x) + (tx - tb.x);
           s0 = P.map0[mi];
-          if (s0 >= 0) {
+          if (s0 != kNoTile) {
             s1 = P.map1[mi];
             present = true;
           }
@@ -602,9 +602,13 @@ __global__ void __launch_bounds__(64) CompositeKernel(CompositeParams P) {
           cov0 |= (in ? 0xFFu : 0u) << (8 * q);
         }
       } else {
-        // the maps hold absolute plane numbers
+        // the maps hold absolute plane numbers; a solid tile has no plane 0
         const uint32_t* pl0 = (const uint32_t*)(P.planes + (int64_t)q0 * kTilePlaneBytes) + lane;
-        cov0 = pl0[0];
+        if (q0 == kSolidTile) {
+          cov0 = row_ok ? ~0u : 0u;
+        } else {
+          cov0 = pl0[0];
+        }
         if (three) {
           // direct covers (0 included), accumulated covers, and which
           // pixels have a direct span

@@ -20,7 +20,8 @@
 // Coverage of a pixel row is collected as LDS deltas (hipr_blit.hpp) and, when
 // the row is complete, resolved into at most two covers per pixel (the
 // directly emitted span first, then the accumulated one), which are written
-// into the plane(s) of the 16x16 tile holding the pixel.
+// into the plane(s) of the 16x16 tile holding the pixel.  A tile whose every
+// pixel is covered by 255 gets no plane, only a map entry.
 #ifndef SKITY_HIP_WALK_HPP_
 #define SKITY_HIP_WALK_HPP_
 
@@ -32,6 +33,10 @@ namespace hipr {
 constexpr int kTilePlaneBytes = kTile * kTile;
 // Tile slot of an allocation that found no plane (capacity and pool spent).
 constexpr int32_t kNoPlane = 0x7FFFFFFF;
+// Map entries: a plane number, or no coverage, or a tile whose every pixel
+// has the first cover 255, which needs no plane.
+constexpr int32_t kNoTile = -1;
+constexpr int32_t kSolidTile = -2;
 
 // Walk modes: count the tile planes, write them, or only follow the step
 // schedule (no coverage) to record the row-band snapshots.
@@ -174,10 +179,12 @@ __device__ __forceinline__ int MakeMeta(int winding, bool quad, bool moved, int 
 }
 
 struct WalkLds {
-  int32_t* d;      // packed row deltas (RowSink)
+  int32_t* d;      // packed row deltas (RowSink), from the first tile column's left edge
+  uint32_t* touch; // a bit per tile column: the row has deltas there
   int32_t* slot0;  // per tile column of the current band
   int32_t* slot1;
   int32_t* rows;   // per tile column: rows written, plane 0 (bits 0-15), plane 1 (16-31)
+  int32_t* full;   // per tile column: rows whose 16 pixels all have the cover 255
   int32_t* sX;     // permutation scratch (CAP entries each)
   int32_t* sDX;
   int32_t* sDY;
@@ -189,11 +196,19 @@ struct WalkLds {
   int4* iL;        // CAP / 2 entries each
   int4* iR;
   BlitScratch blit;
+  // row flush (in the blit scratch): the touched tile columns of a group of
+  // 64, and each one's value at its last pixel
+  int32_t* list;
+  int32_t* vend;
 };
 // LDS words of a K-slot walk whose rows are up to `w` pixels wide (w a
-// multiple of 16).
+// multiple of 16), the rows starting and ending anywhere in their tiles.
+__host__ __device__ inline int WalkTouchInts(int w) {
+  return 2 * ((w / kTile + 2 + kWave - 1) / kWave);
+}
 __host__ __device__ inline int WalkLdsInts(int K, int w) {
-  return kBlitScratchInts + 5 * K * kWave + (w + 1) + 3 * (w / kTile + 2);
+  return kBlitScratchInts + 5 * K * kWave + (w + 2 * kTile) + WalkTouchInts(w) +
+         4 * (w / kTile + 2);
 }
 
 // Bitonic sort (ascending) of N = 64 * 2^j keys held as element
@@ -242,9 +257,9 @@ __device__ void BitonicSortSlots(int64_t (&key)[K], int N, int lane) {
 }
 
 // Write pass (kWalkWrite): one wave per (job, band) item; the job's map
-// starts at -1 (filled before the launch), its JobCov at zero, and planes are
-// taken from the job's counter (JobCov::planes) with atomics, so the bands of
-// a job run concurrently.  Count and schedule passes: one wave per job, band
+// starts at kNoTile (filled before the launch), its JobCov at zero, and planes
+// are taken from the job's counter (JobCov::alloc) with atomics, so the bands
+// of a job run concurrently.  Count and schedule passes: one wave per job, band
 // 0, walking every row and recording the band snapshots.
 template <int K, int kMode>
 __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* lds) {
@@ -283,6 +298,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
       c->bottom = pb.b;
       c->tiles = 0;
       c->planes = 0;
+      c->alloc = 0;
       c->max_active = 0;
       c->flags = flags;
       c->steps = 0;
@@ -310,17 +326,21 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
   L.iL = (int4*)L.sX;
   L.iR = L.iL + CAP / 2;
   L.d = L.sM + CAP;
-  L.slot0 = L.d + (P.lds_width + 1);
+  L.touch = (uint32_t*)(L.d + P.lds_width + 2 * kTile);
+  L.slot0 = (int32_t*)L.touch + WalkTouchInts(P.lds_width);
   L.slot1 = L.slot0 + (P.lds_width / kTile + 2);
   L.rows = L.slot1 + (P.lds_width / kTile + 2);
-  for (int i = lane; i <= W; i += kWave) {
-    L.d[i] = 0;
-  }
+  L.full = L.rows + (P.lds_width / kTile + 2);
+  L.list = lds;
+  L.vend = lds + kWave;
+  for (int i = lane; i < tr.ntc * (kTile / 4); i += kWave) ((int4*)L.d)[i] = make_int4(0, 0, 0, 0);
   for (int i = lane; i < tr.ntc; i += kWave) {
     L.slot0[i] = -1;
     L.slot1[i] = -1;
     L.rows[i] = 0;
+    L.full[i] = 0;
   }
+  for (int i = lane; i < WalkTouchInts(P.lds_width); i += kWave) L.touch[i] = 0;
   WaveSync();
 
   const EdgeRec* E = P.wedges + P.edge_base[j];
@@ -332,13 +352,12 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
   const Fixed left_clip = (Fixed)((uint32_t)pb.l << 16);
   const Fixed right_clip = (Fixed)((uint32_t)pb.r << 16);
   const int winding_mask = job.fill == HIPR_FILL_EVEN_ODD ? 1 : -1;
-  const int cx0 = pb.l > 0 ? pb.l : 0, cx1 = pb.r < cv.width ? pb.r : cv.width;
   const int cy0 = pb.t > 0 ? pb.t : 0, cy1 = pb.b < cv.height ? pb.b : cv.height;
   // A job whose blend mode is not a no-op for a transparent source keeps the
   // reference's zero-cover direct spans: its tiles take three planes (direct
   // covers, accumulated covers, and a byte per pixel marking a direct span).
   const bool triple = (job.flags & kJobKeepZero) != 0;
-  RowSink sink{L.d, ox, W, triple};
+  RowSink sink{L.d + (ox & (kTile - 1)), L.touch, ox, W, triple};
 
   // Active list registers.
   Fixed X[K], DX[K], DY[K], LY[K];
@@ -346,9 +365,8 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
 #pragma unroll
   for (int t = 0; t < K; t++) X[t] = DX[t] = DY[t] = LY[t] = M[t] = 0;
   int n = 0;
-  int next_slot = 0;  // tile planes allocated so far
+  int n_planes = 0;   // planes of this lane's tiles (a solid tile counts one)
   int band = -1;      // current 16-row band
-  int dmin = 0x7FFFFFFF, dmax = -0x7FFFFFFF;  // dirty x range of this row
 
   // ---- helpers ---------------------------------------------------------------
   // Write the active list (m elements in lane/slot layout) from scratch.
@@ -366,28 +384,87 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
     }
   };
 
+  // Takes planes for the tile columns `c` of the lanes that need one: plane 0
+  // (three of them for a keep-zero job) and / or plane 1 of the column.
+  // Count pass: nothing to take, the slots are only marked as held.
+  auto take_planes = [&](bool need0, bool need1, int c) {
+    int a0 = 0, a1 = 0;
+    if (kWrite) {
+      const int req = triple ? (need0 ? 3 : 0) : (need0 ? 1 : 0) + (need1 ? 1 : 0);
+      const int rincl = ScanSum(req);
+      const int rtot = __builtin_amdgcn_readlane(rincl, kWave - 1);
+      // the bands of a job share its plane range
+      int got = 0;
+      if (lane == 0) got = atomicAdd(&P.cov[j].alloc, rtot);
+      const int slot_base = __builtin_amdgcn_readlane(got, 0);
+      a0 = slot_base + rincl - req;
+      a1 = a0 + (need0 ? 1 : 0);
+      // absolute plane numbers, from the job's range or (past its capacity)
+      // from the pool
+      const int over_from = slot_base > pcap ? slot_base : pcap;
+      const int over = slot_base + rtot - over_from;
+      int pool0 = 0;
+      if (over > 0) {
+        int pg = 0;
+        if (lane == 0) pg = atomicAdd(P.pool_ctr, over);
+        pool0 = __builtin_amdgcn_readlane(pg, 0);
+      }
+      auto to_abs = [&](int sl) -> int {
+        if (sl < pcap) return (int)(pbase + sl);
+        int pi = pool0 + (sl - over_from);
+        return pi < P.pool_cap ? P.pool_base + pi : kNoPlane;
+      };
+      // a triple must be contiguous: it never comes from the pool (a
+      // job that outgrows its range that way is walked again exactly)
+      a0 = triple ? (a0 + 2 < pcap ? (int)(pbase + a0) : kNoPlane) : to_abs(a0);
+      a1 = to_abs(a1);
+      if ((need0 && a0 == kNoPlane) || (need1 && a1 == kNoPlane)) flags |= 1;
+    }
+    if (need0) L.slot0[c] = a0;
+    if (need1) L.slot1[c] = a1;
+    WaveSync();
+  };
+
   // Finish a band: publish the tile slots of every column to the job map.
-  // Each plane row is written once: with coverage by the row flush, or with
-  // zeros here for the rows the band never wrote.
+  // Each plane row is written once: by the row flush, or here, with zeros
+  // for the rows the band never wrote and with 255 for the full rows (which
+  // the flush only notes, so that a tile of 16 full rows, most tiles of a
+  // large fill, costs neither a plane nor its 256 bytes written and read).
   auto finish_band = [&]() {
     if (band < 0) return;
-    int trow = band - tr.tr0;
-    for (int c = lane; c < tr.ntc; c += kWave) {
-      int s0 = L.slot0[c], s1 = L.slot1[c];
-      // Only planes that were found are published; a job that found none is
-      // reported through flags and redone by the exact path.
-      if (kWrite && s0 >= 0 && s0 != kNoPlane) {
-        map0[(int64_t)trow * tr.ntc + c] = s0;
-        map1[(int64_t)trow * tr.ntc + c] = (s1 >= 0 && s1 != kNoPlane) ? s1 : -1;
+    const int trow = band - tr.tr0;
+    // rows of this band on the canvas
+    const int brows = cv.height - band * kTile;
+    const int all_rows = brows >= kTile ? 0xFFFF : (1 << brows) - 1;
+    for (int c0 = 0; c0 < tr.ntc; c0 += kWave) {
+      const int c = c0 + lane;
+      const bool ok = c < tr.ntc;
+      uint32_t written = 0;
+      int fm = 0;
+      if (ok) {
+        written = (uint32_t)L.rows[c];
+        fm = L.full[c];
       }
+      const bool has0 = (written & 0xFFFF) != 0 || fm != 0, has1 = (written >> 16) != 0;
+      n_tiles += has0 ? 1 : 0;
+      n_planes += triple ? (has0 ? 3 : 0) : (has0 ? 1 : 0) + (has1 ? 1 : 0);
       if (kWrite) {
-        const uint32_t written = (uint32_t)L.rows[c];
-        const int4 zero = {0, 0, 0, 0};
+        const bool solid = fm == all_rows && (written & 0xFFFF) == 0;
+        const bool need = fm != 0 && !solid && L.slot0[ok ? c : 0] < 0;
+        if (__ballot(need) != 0) take_planes(need, false, c);
+        const int s0 = ok ? L.slot0[c] : -1, s1 = ok ? L.slot1[c] : -1;
+        // Only planes that were found are published; a job that found none is
+        // reported through flags and redone by the exact path.
+        if (solid || (s0 >= 0 && s0 != kNoPlane)) {
+          map0[(int64_t)trow * tr.ntc + c] = solid ? kSolidTile : s0;
+          map1[(int64_t)trow * tr.ntc + c] = (s1 >= 0 && s1 != kNoPlane) ? s1 : kNoTile;
+        }
+        const int4 zero = {0, 0, 0, 0}, ones = {-1, -1, -1, -1};
         if (s0 >= 0 && s0 != kNoPlane) {
           for (int t = 0; t < (triple ? 3 : 1); t++) {
             int4* pl = (int4*)(planes + (int64_t)(s0 + t) * kTilePlaneBytes);
             for (int k = 0; k < kTile; k++)
-              if (!((written >> k) & 1)) pl[k] = zero;
+              if (!((written >> k) & 1)) pl[k] = (fm >> k) & 1 ? ones : zero;
           }
         }
         if (s1 >= 0 && s1 != kNoPlane) {
@@ -396,172 +473,167 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
             if (!((written >> (16 + k)) & 1)) pl[k] = zero;
         }
       }
-      L.slot0[c] = -1;
-      L.slot1[c] = -1;
-      L.rows[c] = 0;
+      if (ok) {
+        L.slot0[c] = -1;
+        L.slot1[c] = -1;
+        L.rows[c] = 0;
+        L.full[c] = 0;
+      }
     }
     WaveSync();
   };
 
-  // Resolve pixel row r (prefix-sum the deltas) and emit its tile rows.
+  // The covers of a pixel whose deltas sum to S: the directly emitted span
+  // (or the accumulated one where there is none), then the accumulated one;
+  // for a keep-zero job the direct cover, the accumulated one, and whether
+  // there is a direct span.
+  auto covers = [&](int S, uint32_t* first, uint32_t* second, uint32_t* third) {
+    const int a = S & 0xFFFF, d = S >> 16;
+    const int av = a > 255 ? 255 : a;
+    const int cnt = d >> 12;  // direct spans
+    const bool dir = cnt != 0;
+    const int dv = d & (kDirectCount - 1);
+    if (triple) {
+      *first = dir ? dv & 0xFF : 0;
+      *second = av;
+      *third = dir ? 1 : 0;
+    } else {
+      *first = (dir ? dv : av) & 0xFF;
+      *second = dir ? av : 0;
+      *third = 0;
+    }
+    if (cnt >= 2) flags |= 4;
+  };
+
+  // Resolve pixel row r and emit its tile rows.  Only the tile columns that
+  // hold deltas are summed, 16 of them at a time (four lanes of four pixels
+  // each, in column order, so one prefix sum runs through them); the columns
+  // between take the value at the end of the touched column before them, one
+  // lane per column.
   auto flush_row = [&](int r) {
-    int lo = DppWaveMin(dmin), hi = -DppWaveMin(-dmax);
-    dmin = 0x7FFFFFFF;
-    dmax = -0x7FFFFFFF;
-    if (lo > hi) return;  // nothing drawn in this row
     WaveSync();
-    bool visible = r >= cy0 && r < cy1;
-    int rb = r >> 4;
-    if (visible && rb != band) {
+    const int rb = r >> 4;
+    if (rb != band) {
       finish_band();
       band = rb;
     }
-    // canvas-aligned 16-pixel chunks; lane owns 4 pixels
-    int base = (ox + lo) & ~15;
-    int end = ox + hi;  // exclusive pixel bound of the dirty range
+    const int rowk = r & 15;
     int carry = 0;
-    // deltas left of `base` are zero: base <= ox + lo
-    for (int x0 = base; x0 <= end; x0 += 4 * kWave) {
-      int px = x0 + 4 * lane;
-      int32_t vS[4];
-      int sS = 0;
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        int i = px + q - ox;
-        int dv = 0;
-        if (i >= 0 && i <= W) {
-          dv = L.d[i];
-          L.d[i] = 0;
-        }
-        sS += dv;
-        vS[q] = sS;
-      }
-      int iS = ScanSum(sS);
-      int eS = iS - sS + carry;
-      carry += __builtin_amdgcn_readlane(iS, kWave - 1);
-      uint32_t c0 = 0, c1 = 0, c2 = 0;
-      bool stacked = false;
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        int S = vS[q] + eS;
-        int a = S & 0xFFFF, d = S >> 16;
-        int cnt = d >> 12, dv = d & 0xFFF;
-        int av = a > 255 ? 255 : a;
-        int first = cnt ? dv : av;
-        int second = (cnt && av) ? av : 0;
-        int third = 0;
-        if (triple) {
-          first = cnt ? dv : 0;
-          second = av;
-          third = cnt ? 1 : 0;
-        }
-        if (cnt >= 2) stacked = true;
-        int x = px + q;
-        if (!visible || x < cx0 || x >= cx1) {
-          first = 0;
-          second = 0;
-          third = 0;
-        }
-        c0 |= (uint32_t)(first & 0xFF) << (8 * q);
-        c1 |= (uint32_t)(second & 0xFF) << (8 * q);
-        c2 |= (uint32_t)third << (8 * q);
-      }
-      if (stacked) flags |= 4;
-      if (!visible) continue;
-      // chunk (4 lanes = 16 px) status
-      uint64_t nz0 = __ballot(triple ? (c0 | c1 | c2) != 0 : c0 != 0);
-      uint64_t nz1 = __ballot(!triple && c1 != 0);
-      int g = lane >> 2;
-      bool chunk0 = ((nz0 >> (4 * g)) & 0xF) != 0;
-      bool chunk1 = ((nz1 >> (4 * g)) & 0xF) != 0;
-      int tcol = (px >> 4) - tr.tc0;
-      bool in_cols = tcol >= 0 && tcol < tr.ntc;
-      bool leader = (lane & 3) == 0;
-      // allocate planes for chunks that become non-empty in this band
-      int cur0 = in_cols ? L.slot0[tcol] : -1;
-      int cur1 = in_cols ? L.slot1[tcol] : -1;
-      bool need0 = in_cols && leader && chunk0 && cur0 < 0;
-      bool need1 = in_cols && leader && chunk1 && cur1 < 0;
-      // most chunks already hold their planes: allocate only when needed
-      if (__ballot(need0 || need1) != 0) {
-        int req = triple ? (need0 ? 3 : 0) : (need0 ? 1 : 0) + (need1 ? 1 : 0);
-        int rincl = ScanSum(req);
-        int rtot = __builtin_amdgcn_readlane(rincl, kWave - 1);
-        int slot_base = next_slot;
-        if (kWrite && rtot > 0) {
-          // the bands of a job share its plane range
-          int got = 0;
-          if (lane == 0) got = atomicAdd(&P.cov[j].planes, rtot);
-          slot_base = __builtin_amdgcn_readlane(got, 0);
-        }
-        int first_slot = slot_base + rincl - req;
-        next_slot += rtot;
-        // Count pass: tile slots are job-relative.  Write pass: absolute plane
-        // numbers, from the job's range or (past its capacity) from the pool.
-        int a0 = first_slot, a1 = first_slot + (need0 ? 1 : 0);
-        if (kWrite) {
-          const int over_from = slot_base > pcap ? slot_base : pcap;
-          const int over = slot_base + rtot - over_from;
-          int pool0 = 0;
-          if (over > 0) {
-            int got = 0;
-            if (lane == 0) got = atomicAdd(P.pool_ctr, over);
-            pool0 = __builtin_amdgcn_readlane(got, 0);
-          }
-          auto to_abs = [&](int sl) -> int {
-            if (sl < pcap) return (int)(pbase + sl);
-            int pi = pool0 + (sl - over_from);
-            return pi < P.pool_cap ? P.pool_base + pi : kNoPlane;
-          };
-          // a triple must be contiguous: it never comes from the pool (a
-          // job that outgrows its range that way is walked again exactly)
-          a0 = triple ? (a0 + 2 < pcap ? (int)(pbase + a0) : kNoPlane) : to_abs(a0);
-          a1 = to_abs(a1);
-        }
-        if (need0) {
-          L.slot0[tcol] = a0;
-          n_tiles++;
-        }
-        if (need1) L.slot1[tcol] = a1;
+    for (int g = 0; g < tr.ntc; g += kWave) {
+      const uint32_t* tw = L.touch + 2 * (g / kWave);
+      const uint64_t T = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)tw[0]) |
+                         (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)tw[1]) << 32;
+      if (T == 0 && carry == 0) continue;
+      const int v_in = carry;
+      if (T != 0) {
+        if (lane < 2) L.touch[2 * (g / kWave) + lane] = 0;
+        if (__builtin_amdgcn_inverse_ballot_w64(T)) L.list[CountBelow(T)] = lane;
         WaveSync();
-        cur0 = in_cols ? L.slot0[tcol] : -1;
-        cur1 = in_cols ? L.slot1[tcol] : -1;
-      }
-      if (kWrite) {
-        int sub = lane & 3;
-        int rowk = r & 15;
-        if (in_cols) {
-          if (sub == 0) {
-            // rows written in this band (the other rows are zeroed when the
-            // band ends); one lane per tile column
-            int wr = (chunk0 && cur0 >= 0 ? 1 << rowk : 0) | (chunk1 && cur1 >= 0 ? 1 << (16 + rowk) : 0);
-            if (wr) L.rows[tcol] |= wr;
+        const int nt = __popcll(T);
+        for (int b = 0; b < nt; b += kWave / 4) {
+          const int ti = b + (lane >> 2), sub = lane & 3;
+          // (a bit past the last column is the end-of-row entry's)
+          const int col = ti < nt ? L.list[ti] : kWave;
+          const int tcol = g + col;
+          const bool ok = col < kWave && tcol < tr.ntc;
+          int4 dv = make_int4(0, 0, 0, 0);
+          if (ok) {
+            int4* dp = (int4*)(L.d + tcol * kTile + 4 * sub);
+            dv = *dp;
+            *dp = make_int4(0, 0, 0, 0);
           }
-          if (chunk0 && cur0 >= 0) {
-            if (cur0 != kNoPlane) {
+          const int t1 = dv.x + dv.y, t2 = t1 + dv.z, t3 = t2 + dv.w;
+          const int incl = ScanSum(t3);
+          const int e = incl - t3 + carry;
+          carry += __builtin_amdgcn_readlane(incl, kWave - 1);
+          if (ok && sub == 3) L.vend[col] = e + t3;
+          uint32_t c0 = 0, c1 = 0, c2 = 0, f, s2, t;
+          covers(e + dv.x, &f, &s2, &t);
+          c0 = f, c1 = s2, c2 = t;
+          covers(e + t1, &f, &s2, &t);
+          c0 |= f << 8, c1 |= s2 << 8, c2 |= t << 8;
+          covers(e + t2, &f, &s2, &t);
+          c0 |= f << 16, c1 |= s2 << 16, c2 |= t << 16;
+          covers(e + t3, &f, &s2, &t);
+          c0 |= f << 24, c1 |= s2 << 24, c2 |= t << 24;
+          // the tile row's state over its four lanes: bit 0 a cover in plane
+          // 0, bit 1 one in plane 1, bit 2 not full
+          int st = 0;
+          if (ok) {
+            st = triple ? ((c0 | c1 | c2) != 0 ? 5 : 4)
+                        : (c0 != 0 ? 1 : 0) | (c1 != 0 ? 2 : 0) |
+                              (c0 != 0xFFFFFFFFu || c1 != 0 ? 4 : 0);
+          }
+          st |= DppSwapPairs(st);
+          st |= DppSwapHalves(st);
+          const bool plane0 = (st & 5) == 5, plane1 = (st & 2) != 0;
+          const int cc = ok ? tcol : 0;
+          if (sub == 0 && ok) {
+            if ((st & 5) == 1) atomicOr(&L.full[cc], 1 << rowk);
+            const int wr = (plane0 ? 1 << rowk : 0) | (plane1 ? 1 << (16 + rowk) : 0);
+            if (wr) atomicOr(&L.rows[cc], wr);
+          }
+          int cur0 = L.slot0[cc], cur1 = L.slot1[cc];
+          const bool need0 = sub == 0 && plane0 && cur0 < 0;
+          const bool need1 = sub == 0 && plane1 && cur1 < 0;
+          // most columns already hold their planes: allocate only when needed
+          if (__ballot(need0 || need1) != 0) {
+            take_planes(need0, need1, cc);
+            cur0 = L.slot0[cc];
+            cur1 = L.slot1[cc];
+          }
+          if (kWrite) {
+            if (plane0 && cur0 != kNoPlane) {
               uint32_t* pl = (uint32_t*)(planes + (int64_t)cur0 * kTilePlaneBytes);
               pl[rowk * 4 + sub] = c0;
               if (triple) {
                 pl[kTilePlaneBytes / 4 + rowk * 4 + sub] = c1;
                 pl[2 * kTilePlaneBytes / 4 + rowk * 4 + sub] = c2;
               }
-            } else {
-              flags |= 1;
             }
-          }
-          if (chunk1 && cur1 >= 0) {
-            if (cur1 != kNoPlane) {
+            if (plane1 && cur1 != kNoPlane) {
               uint32_t* pl = (uint32_t*)(planes + (int64_t)cur1 * kTilePlaneBytes);
               pl[rowk * 4 + sub] = c1;
-            } else {
-              flags |= 1;
             }
           }
         }
+        WaveSync();
+      }
+      // the other columns of the group
+      const int c = g + lane;
+      const uint64_t below = T & ((1ull << lane) - 1);
+      int v = v_in;
+      if (below) v = L.vend[kWave - 1 - __builtin_clzll(below)];
+      const bool rest = c < tr.ntc && ((T >> lane) & 1) == 0 && v != 0;
+      if (__ballot(rest) == 0) continue;
+      uint32_t f = 0, s2 = 0, t = 0;
+      if (rest) covers(v, &f, &s2, &t);
+      const bool is_full = !triple && f == 255 && s2 == 0;
+      const bool plane0 = rest && !is_full && (triple ? (f | s2 | t) != 0 : f != 0);
+      const bool plane1 = rest && !triple && s2 != 0;
+      if (rest && is_full) atomicOr(&L.full[c], 1 << rowk);
+      if (__ballot(plane0 || plane1) == 0) continue;
+      const int cc = rest ? c : 0;
+      const int wr = (plane0 ? 1 << rowk : 0) | (plane1 ? 1 << (16 + rowk) : 0);
+      if (wr) atomicOr(&L.rows[cc], wr);
+      const bool need0 = plane0 && L.slot0[cc] < 0, need1 = plane1 && L.slot1[cc] < 0;
+      if (__ballot(need0 || need1) != 0) take_planes(need0, need1, cc);
+      if (kWrite) {
+        const int cur0 = L.slot0[cc], cur1 = L.slot1[cc];
+        auto put = [&](int slot, uint32_t b) {
+          const int w = (int)(b * 0x01010101u);
+          ((int4*)(planes + (int64_t)slot * kTilePlaneBytes))[rowk] = make_int4(w, w, w, w);
+        };
+        if (plane0 && cur0 != kNoPlane) {
+          put(cur0, f);
+          if (triple) {
+            put(cur0 + 1, s2);
+            put(cur0 + 2, t);
+          }
+        }
+        if (plane1 && cur1 != kNoPlane) put(cur1, s2);
       }
     }
-    // clear the end-of-row delta entry
-    if (lane == 0) L.d[W] = 0;
     WaveSync();
   };
 
@@ -1054,12 +1126,6 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
         const bool close_prev =
             prev_right > FixedFloorToInt(left) || prev_right > FixedFloorToInt(l.y);
         const bool no_real = full == 0xFF && (close_prev || r.w != 0);
-        if (act) {
-          const int lo = FixedFloorToInt(Min32(Min32(left, next_left), Min32(right, next_right)));
-          const int hi = FixedCeilToInt(Max32(Max32(left, next_left), Max32(right, next_right)));
-          dmin = Min32(dmin, Max32(lo - ox, 0));
-          dmax = Max32(dmax, Min32(hi - ox, W));
-        }
         BlitIntervals(sink, L.blit, act, left, right, next_left, next_right, l.z, r.z, full,
                       no_real);
       }
@@ -1348,7 +1414,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
     }
     // ---- row completion ------------------------------------------------------
     y = next_y;
-    if (kBlit && (y & 0xFFFF) == 0) flush_row(row);
+    if (draw && (y & 0xFFFF) == 0) flush_row(row);
     if (sample) {
       tp4 = wall_clock64();
       ph[3] += tp4 - tp3;
@@ -1374,6 +1440,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
       if (lane == 0) snap_at(next_b)->y = kMaxS32;
   }
   n_tiles = WaveSum(n_tiles);
+  n_planes = WaveSum(n_planes);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) flags |= __shfl_xor(flags, o, kWave);
   if (lane == 0) {
@@ -1396,6 +1463,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
       c->right = pb.r;
       c->bottom = pb.b;
       atomicAdd(&c->tiles, n_tiles);
+      atomicAdd(&c->planes, n_planes);
       atomicMax(&c->max_active, max_active);
       atomicOr(&c->flags, flags);
       atomicAdd(&c->steps, guard);
@@ -1410,7 +1478,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
       c->right = pb.r;
       c->bottom = pb.b;
       c->tiles = n_tiles;
-      c->planes = next_slot;
+      c->planes = n_planes;
       c->max_active = max_active;
       c->flags = flags;
       c->steps = guard;

@@ -1932,9 +1932,9 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   auto prepare_write = [&](const std::vector<int32_t>* js) -> hipr_result {
     if (!js) {
       hipLaunchKernelGGL(FillKernel, dim3(1024), dim3(256), 0, st, ctx->map0.as<int32_t>(),
-                         total_map, -1);
+                         total_map, kNoTile);
       hipLaunchKernelGGL(FillKernel, dim3(1024), dim3(256), 0, st, ctx->map1.as<int32_t>(),
-                         total_map, -1);
+                         total_map, kNoTile);
       hipLaunchKernelGGL(FillKernel, dim3(256), dim3(256), 0, st, (int32_t*)ctx->wcov.p,
                          (int64_t)nj * (int64_t)(sizeof(JobCov) / 4), 0);
       hipLaunchKernelGGL(FillKernel, dim3(1), dim3(kWave), 0, st, ctx->pool_ctr.as<int32_t>(),
@@ -3010,7 +3010,7 @@ HIPR_API hipr_result hipr_surface_get_tile_bins(hipr_surface s, int64_t* offsets
       for (int c = 0; c < t[2]; c++) {
         int64_t i = s->job_mbase[j] + (int64_t)r * t[2] + c;
         int32_t code = ((t[1] + r) * t[4] + (t[0] + c)) << 1;
-        if (m0[i] >= 0) {
+        if (m0[i] != kNoTile) {
           if (bins && k < cap) bins[k] = code;
           k++;
         }
