@@ -3,7 +3,7 @@
 // blit_trapezoid_row / blit_aaa_trapezoid_row and their alpha helpers
 // (src/render/sw/sw_raster.cc:138-544), evaluated per pixel in closed form and
 // spread over the lanes of a wave.
-// Coverage goes into one LDS delta row, prefix-summed when the pixel row is
+// Coverage goes into LDS delta rows, prefix-summed when the pixel rows are
 // complete.  Each 32-bit entry carries two fields whose prefix sums are
 // non-negative and below 2^16, so one integer prefix sum S decodes as
 // A = S & 0xFFFF, D = S >> 16:
@@ -24,7 +24,7 @@ typedef uint8_t Alpha;
 
 constexpr int kDirectCount = 1 << 12;  // one direct span, in the D field
 
-// The row covers the visible pixels [left, left + width) of the path's
+// A row covers the visible pixels [left, left + width) of the path's
 // canvas.  A span's two delta entries are clamped into [0, width]: deltas left
 // of the canvas fold into entry 0 and deltas right of it into entry `width`,
 // which no visible pixel's prefix sum reads, so every visible pixel sums the
@@ -32,22 +32,23 @@ constexpr int kDirectCount = 1 << 12;  // one direct span, in the D field
 struct RowSink {
   int32_t* d;       // the delta entry of the first visible column
   uint32_t* touch;  // a bit per tile column, from the first visible column's
-  int32_t left;   // pixel x of delta index 0 (the first visible column)
-  int32_t width;  // visible columns; entry `width` is the end-of-row entry
+  int32_t pitch;    // delta entries of a row (16 per tile column and 16 more)
+  int32_t left;     // pixel x of delta index 0 (the first visible column)
+  int32_t width;    // visible columns; entry `width` is the end-of-row entry
   // Direct spans of cover 0 blend nothing in src-over, and are dropped; a
   // job whose blend mode does change pixels under a transparent source keeps
   // them (they still count as a direct span of the pixel).
   bool keep_zero;
-  // Adds v to the delta at pixel x (clamped into the row).
-  __device__ __forceinline__ void Add(int x, int v) {
+  // Adds v to row r's delta at pixel x (clamped into the row).
+  __device__ __forceinline__ void Add(int r, int x, int v) {
     if (v == 0) return;
     const int i = x - left;
-    atomicAdd(&d[i < 0 ? 0 : (i > width ? width : i)], v);
+    atomicAdd(&d[r * pitch + (i < 0 ? 0 : (i > width ? width : i))], v);
   }
-  // Marks the tile columns of the deltas at pixels a .. b (clamped into the
-  // row) as touched.
-  __device__ __forceinline__ void Touch(int a, int b) {
-    const int c0 = left >> 4;
+  // Marks the tile columns of row r's deltas at pixels a .. b (clamped into
+  // the row) as touched.
+  __device__ __forceinline__ void Touch(int r, int a, int b) {
+    const int c0 = (left >> 4) - r * (pitch >> 4);
     const int lo = (Min32(Max32(a, left), left + width) >> 4) - c0;
     const int hi = (Min32(Max32(b, left), left + width) >> 4) - c0;
     for (int w = lo >> 5; w <= hi >> 5; w++) {
@@ -56,12 +57,13 @@ struct RowSink {
       atomicOr(&touch[w], from & to);
     }
   }
-  // A one-pixel span of cover v at a visible pixel.
-  __device__ __forceinline__ void Pixel(bool direct, int x, int v) {
+  // A one-pixel span of cover v at a visible pixel of row r.
+  __device__ __forceinline__ void Pixel(int r, bool direct, int x, int v) {
     if (v == 0 && !(direct && keep_zero)) return;
     const int inc = direct ? (kDirectCount + v) << 16 : v;
-    atomicAdd(&d[x - left], inc);
-    atomicAdd(&d[x - left + 1], -inc);
+    int32_t* e = &d[r * pitch + x - left];
+    atomicAdd(e, inc);
+    atomicAdd(e + 1, -inc);
   }
 };
 
@@ -161,29 +163,33 @@ __device__ __forceinline__ int CountBelow(uint64_t m, int base = 0) {
                                         __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)base));
 }
 
-// LDS of BlitIntervals: two int4 per trapezoid with per-pixel work, and one
-// mark per work item of a pass.
+// LDS of BlitEdges: two int4 per lane with per-pixel work, and one mark per
+// work item of a pass.
 struct BlitScratch {
   int4* items;   // 2 x 64
   int32_t* mark; // 64
 };
 constexpr int kBlitScratchInts = 2 * kWave * 4 + kWave;
 
-// blit_trapezoid_row (sw_raster.cc:457-544) for up to 64 trapezoids of one
-// step, one per lane (`act`).
+// blit_trapezoid_row (sw_raster.cc:457-544) for up to 32 trapezoids, two lanes
+// each (`act`; `side` 0 its left edge, 1 its right edge), on delta row `r` of
+// their lanes.
 //
-// A trapezoid is a run of `full` pixels between a left and a right edge.  An
-// edge that stays within one or two pixels is done by the trapezoid's own
-// lane as deltas.  A flatter one covers a row of pixels in part, each with
-// its own cover (TrapezoidPixel), as does every pixel of a trapezoid whose
-// edges share pixels.  Those pixels, a few for most trapezoids and hundreds
+// A trapezoid is a run of `full` pixels between a left and a right edge, each
+// of which covers R pixels in part.  The right edge is the left edge's mirror
+// image, in every formula and to the bit (distances are taken from the outer
+// pixel boundary), so one lane per edge runs one code path where one lane per
+// trapezoid ran two.  An edge that stays within one or two pixels is done by
+// its lane as deltas.  A flatter one gives every pixel its own cover
+// (TrapezoidPixel), as do all pixels of a trapezoid whose edges share pixels
+// (drawn from side 0).  Those pixels, a few for most trapezoids and hundreds
 // for a nearly horizontal edge, are laid end to end and handed out one per
 // lane, so a wave takes ceil(total / 64) passes over them however unevenly
-// they are spread; looping over them per lane took as many passes as the
-// longest one has pixels (measured with the change in hipr_walk.hpp).
-__device__ __forceinline__ void BlitIntervals(RowSink& s, const BlitScratch& L, bool act, Fixed ul,
-                                              Fixed ur, Fixed ll, Fixed lr, Fixed lDY, Fixed rDY,
-                                              Alpha full, bool no_real) {
+// they are spread; looping over them per lane takes as many passes as the
+// longest one has pixels.
+__device__ __forceinline__ void BlitEdges(RowSink& s, const BlitScratch& L, bool act, int side,
+                                          int r, Fixed ul, Fixed ur, Fixed ll, Fixed lr, Fixed lDY,
+                                          Fixed rDY, Alpha full, bool no_real) {
   const int lane = Lane();
   bool go = act && ul <= ur;
   if (ll > lr) ll = lr = ApproxIntersection(ul, ll, ur, lr);
@@ -205,63 +211,47 @@ __device__ __forceinline__ void BlitIntervals(RowSink& s, const BlitScratch& L, 
     return v != 0 || s.keep_zero ? (kDirectCount + v) << 16 : 0;
   };
   auto part = [&](Alpha a) -> int { return inc(direct ? a : PartialAlphaA(a, full)); };
-  const int vis_end = s.left + s.width;
-  int cnt_a = 0, cnt = 0;
-  if (go) {
-    const Fixed join_left = FixedCeilToFixed(ll), join_rite = FixedFloorToFixed(ur);
-    const int x0 = ul >> 16;
-    if (join_left <= join_rite) {
-      const int JL = join_left >> 16, JR = join_rite >> 16;
-      int last = 0, first = 0;  // increments left of JL and right of JR
-      if (ul < join_left) {
-        const int len = FixedCeilToInt(join_left - ul);
-        if (len == 1) {
-          last = part(TrapezoidToAlpha(join_left - ul, join_left - ll));
-          s.Add(x0, last);
-        } else if (len == 2) {
-          const Fixed f = join_left - kFixed1 - ul;
-          const Fixed sec = ll - ul - f;
-          const int i1 = inc(PartialTriangleToAlpha(f, lDY));
-          last = inc((Alpha)(full - PartialTriangleToAlpha(sec, lDY)));
-          s.Add(x0, i1);
-          s.Add(x0 + 1, last - i1);
-        } else {
-          cnt_a = Max32(0, Min32(JL, vis_end) - Max32(x0, s.left));
-          cnt = cnt_a;
-        }
-      }
-      if (lr > join_rite) {
-        const int len = FixedCeilToInt(lr - join_rite);
-        if (len == 1) {
-          first = part(TrapezoidToAlpha(ur - join_rite, lr - join_rite));
-          s.Add(JR + 1, -first);
-        } else if (len == 2) {
-          const Fixed f = join_rite + kFixed1 - ur;
-          const Fixed sec = lr - ur - f;
-          first = inc((Alpha)(full - PartialTriangleToAlpha(f, rDY)));
-          const int i2 = inc(PartialTriangleToAlpha(sec, rDY));
-          s.Add(JR + 1, i2 - first);
-          s.Add(JR + 2, -i2);
-        } else {
-          cnt += Max32(0, Min32(FixedCeilToInt(lr), vis_end) - Max32(JR, s.left));
-        }
-      }
-      const int run = join_left < join_rite ? inc(full) : 0;
-      s.Add(JL, run - last);
-      s.Add(JR, first - run);
-      s.Touch(x0, JL);
-      s.Touch(JR, FixedCeilToInt(lr));
+  int cnt = 0;
+  const Fixed join_left = FixedCeilToFixed(ll), join_rite = FixedFloorToFixed(ur);
+  const int x0 = ul >> 16;
+  if (go && join_left <= join_rite) {
+    const int JL = join_left >> 16, JR = join_rite >> 16;
+    // the edge's pixels [from, from + R) and, from its outer end, where it
+    // enters (l) and leaves (rr) them
+    const int from = side ? JR : x0;
+    const int R = side ? FixedCeilToInt(lr) - JR : JL - x0;
+    Fixed l = (side ? ur : ul) - IntToFixed(from), rr = (side ? lr : ll) - IntToFixed(from);
+    if (side) {
+      const Fixed t = IntToFixed(R) - rr;
+      rr = IntToFixed(R) - l;
+      l = t;
+    }
+    const Fixed dY = side ? rDY : lDY;
+    int inner = 0, outer = 0;  // increments of the pixels next to the run
+    if (R == 1) {
+      inner = part(TrapezoidToAlpha(kFixed1 - l, kFixed1 - rr));
+    } else if (R == 2) {
+      outer = inc(PartialTriangleToAlpha(kFixed1 - l, dY));
+      inner = inc((Alpha)(full - PartialTriangleToAlpha(rr - kFixed1, dY)));
     } else {
-      const int R = FixedCeilToInt(lr);
-      s.Touch(x0, R);
-      if (R - x0 == 1) {
-        const int v = part(TrapezoidToAlpha(ur - ul, lr - ll));
-        s.Add(x0, v);
-        s.Add(R, -v);
-      } else {
-        cnt_a = Max32(0, Min32(R, vis_end) - Max32(x0, s.left));
-        cnt = cnt_a;
-      }
+      cnt = Max32(0, Min32(from + R, s.left + s.width) - Max32(from, s.left));
+    }
+    const int run = JL < JR ? inc(full) : 0;
+    const int at = side ? JR : JL, d = side ? 1 : -1;
+    const int sg = side ? -1 : 0;  // negates the right edge's increments
+    s.Add(r, at, ((run - inner) ^ sg) - sg);
+    s.Add(r, at + d, ((inner - outer) ^ sg) - sg);
+    s.Add(r, at + 2 * d, (outer ^ sg) - sg);
+    s.Touch(r, from, from + R);
+  } else if (go && side == 0) {
+    const int R = FixedCeilToInt(lr);
+    s.Touch(r, x0, R);
+    if (R - x0 == 1) {
+      const int v = part(TrapezoidToAlpha(ur - ul, lr - ll));
+      s.Add(r, x0, v);
+      s.Add(r, R, -v);
+    } else {
+      cnt = Max32(0, Min32(R, s.left + s.width) - Max32(x0, s.left));
     }
   }
   const uint64_t have = __ballot(cnt > 0);
@@ -272,12 +262,12 @@ __device__ __forceinline__ void BlitIntervals(RowSink& s, const BlitScratch& L, 
   if (cnt > 0) {
     int4* it = L.items + 2 * CountBelow(have);
     it[0] = make_int4(ul, ur, ll, lr);
-    it[1] = make_int4(lDY, rDY, (cnt_a << 1) | (direct ? 1 : 0), start);
+    it[1] = make_int4(lDY, rDY, (r << 2) | (side << 1) | (direct ? 1 : 0), start);
   }
-  int before = 0;  // trapezoids whose pixels start before this pass
+  int before = 0;  // lanes whose pixels start before this pass
   for (int base = 0; base < total; base += kWave) {
-    // mark where each trapezoid's pixels start; the marks up to a lane count
-    // the trapezoids up to its pixel
+    // mark where each lane's pixels start; the marks up to a pixel count the
+    // lanes up to its own
     L.mark[lane] = 0;
     WaveSync();
     if (cnt > 0 && start >= base && start < base + kWave) L.mark[start - base] = 1;
@@ -287,11 +277,9 @@ __device__ __forceinline__ void BlitIntervals(RowSink& s, const BlitScratch& L, 
     if (t < total) {
       const int own = CountBelow(marks, before) + (int)((marks >> lane) & 1) - 1;
       const int4 a = L.items[2 * own], b = L.items[2 * own + 1];
-      const int o = t - b.w, ca = b.z >> 1;
-      const int x = o < ca ? Max32(a.x >> 16, s.left) + o
-                           : Max32(FixedFloorToInt(a.y), s.left) + (o - ca);
+      const int x = Max32(FixedFloorToInt((b.z & 2) != 0 ? a.y : a.x), s.left) + (t - b.w);
       const Alpha v = TrapezoidPixel(x, a.x, a.y, a.z, a.w, b.x, b.y, full);
-      s.Pixel((b.z & 1) != 0, x, v);
+      s.Pixel(b.z >> 2, (b.z & 1) != 0, x, v);
     }
     before += __popcll(marks);
     WaveSync();

@@ -54,10 +54,16 @@ HD Fixed FixedMul(Fixed a, Fixed b) { return (Fixed)(((int64_t)a * b) >> 16); }
 HD Fixed LShift32(int32_t v, int s) { return (int32_t)((uint32_t)v << s); }
 HD Fixed FDot6ToFixed(FDot6 x) { return LShift32(x, 10); }
 HD Fixed FDot6ToFixedDiv2(FDot6 x) { return LShift32(x, 16 - 6 - 1); }
+// (numer << 16) / denom, truncated and clamped.  The operands are exact in
+// double, and truncating the rounded quotient is exact: |numer << 16| < 2^48,
+// so the rounding moves a quotient by less than 2^-5 / |denom|, and one that
+// is not an integer is at least 1 / |denom| away from every integer.  The
+// device's 64-bit integer division is a loop of a hundred instructions and
+// more; this is about twenty.
 HD Fixed FixedDiv(int32_t numer, int32_t denom) {
-  int64_t q = (int64_t)((uint64_t)(int64_t)numer << 16) / denom;
-  q = q < kMinS32 ? kMinS32 : q;
-  q = q > kMaxS32 ? kMaxS32 : q;
+  double q = (double)numer * 65536.0 / (double)denom;
+  q = q < (double)kMinS32 ? (double)kMinS32 : q;
+  q = q > (double)kMaxS32 ? (double)kMaxS32 : q;
   return (Fixed)q;
 }
 HD FDot6 FixedToFDot6(Fixed x) { return x >> 10; }

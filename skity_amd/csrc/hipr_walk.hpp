@@ -6,7 +6,8 @@
 // (sw_raster.cc:159-247) re-expressed for a 64-lane wave.  The active edge
 // list lives in registers (element p in lane p % 64, slot p / 64) and every
 // sequential list operation of the reference is replaced by the parallel
-// operation with the same result:
+// operation with the same result, and rows without an event are taken up to 16
+// at a time:
 //   * winding sums and interval roles: wave prefix sums in list order;
 //   * the left edge of an interval / the previous right edge: max-scans;
 //   * the per-edge x re-insertion after a step keeps the survivors stably
@@ -89,7 +90,8 @@ struct WalkParams {
   int32_t* map0;
   int32_t* map1;
   JobCov* cov;
-  int32_t lds_width;        // row buffer capacity in pixels
+  int32_t lds_width;        // widest row in pixels
+  int32_t row_ints;         // row delta capacity (multiple of 16)
   int32_t* queue;           // persistent form: item counter (starts at 0), else null
 };
 
@@ -184,17 +186,17 @@ struct WalkLds {
   int32_t* slot0;  // per tile column of the current band
   int32_t* slot1;
   int32_t* rows;   // per tile column: rows written, plane 0 (bits 0-15), plane 1 (16-31)
-  int32_t* full;   // per tile column: rows whose 16 pixels all have the cover 255
+  int32_t* full;   // per tile column 16 bits: rows whose 16 pixels all have the cover 255
   int32_t* sX;     // permutation scratch (CAP entries each)
   int32_t* sDX;
   int32_t* sDY;
   int32_t* sLY;
   int32_t* sM;
-  // left and right edges of the step's intervals {x, next x, dy, the next
-  // edge is too close}; they share the permutation scratch, which is free
-  // while the intervals are drawn
-  int4* iL;        // CAP / 2 entries each
-  int4* iR;
+  // left and right edges of the step's intervals; they share the permutation
+  // scratch, which is free while the intervals are drawn
+  int4* iL;        // {x, step, dy, -}; CAP / 2 entries each
+  int4* iR;        // {x, step, dy, kNext*}
+  int2* iN;        // the next edge's {x, dx}
   BlitScratch blit;
   // row flush (in the blit scratch): the touched tile columns of a group of
   // 64, and each one's value at its last pixel
@@ -202,14 +204,23 @@ struct WalkLds {
   int32_t* vend;
 };
 // LDS words of a K-slot walk whose rows are up to `w` pixels wide (w a
-// multiple of 16), the rows starting and ending anywhere in their tiles.
-__host__ __device__ inline int WalkTouchInts(int w) {
-  return 2 * ((w / kTile + 2 + kWave - 1) / kWave);
+// multiple of 16), the rows starting and ending anywhere in their tiles, with
+// room for `row_ints` row deltas (at least one row's, WalkRowInts).
+__host__ __device__ inline int WalkRowInts(int w) { return w + 3 * kTile; }
+__host__ __device__ inline int WalkTouchInts(int row_ints) {
+  return 2 * ((row_ints / kTile + kWave) / kWave);
 }
-__host__ __device__ inline int WalkLdsInts(int K, int w) {
-  return kBlitScratchInts + 5 * K * kWave + (w + 2 * kTile) + WalkTouchInts(w) +
-         4 * (w / kTile + 2);
+// The 32- and 64-slot walks take one row at a time and keep no next edges
+// (iN), so their blit scratch fits into the permutation scratch: a 64-slot
+// walk of a 16,384-pixel row just fits the 160 KB of a CU.
+constexpr int kWideSlots = 32;
+__host__ __device__ inline int WalkLdsInts(int K, int w, int row_ints) {
+  return (K >= kWideSlots ? 0 : kBlitScratchInts) + 5 * K * kWave + row_ints +
+         WalkTouchInts(row_ints) + 3 * (w / kTile + 2) + (w / kTile + 3) / 2;
 }
+// What follows a closing edge in the list: nothing, an edge whose distance
+// the interval checks, or one that is known to be too close.
+enum : int32_t { kNextNone = 0, kNextCheck = 1, kNextClose = 2 };
 
 // Bitonic sort (ascending) of N = 64 * 2^j keys held as element
 // p = slot * 64 + lane; keys at p >= N are not touched (N <= 64 * K).
@@ -316,31 +327,39 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
   // the band ends where the next band's snapshot was taken
   const Fixed stop_y = (kWrite && rband + 1 < nb) ? snap_at(rband + 1)->y : kMaxS32;
   WalkLds L;
-  L.blit.items = (int4*)lds;
-  L.blit.mark = lds + 2 * kWave * 4;
-  L.sX = lds + kBlitScratchInts;
+  constexpr bool kWide = K >= kWideSlots;
+  L.sX = lds + (kWide ? 0 : kBlitScratchInts);
   L.sDX = L.sX + CAP;
   L.sDY = L.sDX + CAP;
   L.sLY = L.sDY + CAP;
   L.sM = L.sLY + CAP;
   L.iL = (int4*)L.sX;
   L.iR = L.iL + CAP / 2;
+  L.iN = (int2*)(L.iR + CAP / 2);
   L.d = L.sM + CAP;
-  L.touch = (uint32_t*)(L.d + P.lds_width + 2 * kTile);
-  L.slot0 = (int32_t*)L.touch + WalkTouchInts(P.lds_width);
+  L.touch = (uint32_t*)(L.d + P.row_ints);
+  L.slot0 = (int32_t*)L.touch + WalkTouchInts(P.row_ints);
   L.slot1 = L.slot0 + (P.lds_width / kTile + 2);
   L.rows = L.slot1 + (P.lds_width / kTile + 2);
   L.full = L.rows + (P.lds_width / kTile + 2);
-  L.list = lds;
-  L.vend = lds + kWave;
-  for (int i = lane; i < tr.ntc * (kTile / 4); i += kWave) ((int4*)L.d)[i] = make_int4(0, 0, 0, 0);
+  int32_t* blit = kWide ? L.sM : lds;
+  L.blit.items = (int4*)blit;
+  L.blit.mark = blit + 2 * kWave * 4;
+  L.list = blit;
+  L.vend = blit + kWave;
+  // Delta rows: a row takes its tile columns and one more, which holds the
+  // end-of-row entry when the row ends on a tile boundary; up to 16 rows.
+  const int ncol = tr.ntc + 1;
+  const int row_cap = kWide ? 1 : Min32(P.row_ints / (ncol * kTile), kTile);
+  for (int i = lane; i < row_cap * ncol * (kTile / 4); i += kWave)
+    ((int4*)L.d)[i] = make_int4(0, 0, 0, 0);
   for (int i = lane; i < tr.ntc; i += kWave) {
     L.slot0[i] = -1;
     L.slot1[i] = -1;
     L.rows[i] = 0;
-    L.full[i] = 0;
   }
-  for (int i = lane; i < WalkTouchInts(P.lds_width); i += kWave) L.touch[i] = 0;
+  for (int i = lane; i < (tr.ntc + 1) / 2; i += kWave) L.full[i] = 0;
+  for (int i = lane; i < WalkTouchInts(P.row_ints); i += kWave) L.touch[i] = 0;
   WaveSync();
 
   const EdgeRec* E = P.wedges + P.edge_base[j];
@@ -357,7 +376,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
   // reference's zero-cover direct spans: its tiles take three planes (direct
   // covers, accumulated covers, and a byte per pixel marking a direct span).
   const bool triple = (job.flags & kJobKeepZero) != 0;
-  RowSink sink{L.d + (ox & (kTile - 1)), L.touch, ox, W, triple};
+  RowSink sink{L.d + (ox & (kTile - 1)), L.touch, ncol * kTile, ox, W, triple};
 
   // Active list registers.
   Fixed X[K], DX[K], DY[K], LY[K];
@@ -443,7 +462,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
       int fm = 0;
       if (ok) {
         written = (uint32_t)L.rows[c];
-        fm = L.full[c];
+        fm = (L.full[c >> 1] >> (16 * (c & 1))) & 0xFFFF;
       }
       const bool has0 = (written & 0xFFFF) != 0 || fm != 0, has1 = (written >> 16) != 0;
       n_tiles += has0 ? 1 : 0;
@@ -477,7 +496,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
         L.slot0[c] = -1;
         L.slot1[c] = -1;
         L.rows[c] = 0;
-        L.full[c] = 0;
+        if ((c & 1) == 0) L.full[c >> 1] = 0;  // (c + 1 was read with c)
       }
     }
     WaveSync();
@@ -505,21 +524,36 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
     if (cnt >= 2) flags |= 4;
   };
 
-  // Resolve pixel row r and emit its tile rows.  Only the tile columns that
-  // hold deltas are summed, 16 of them at a time (four lanes of four pixels
-  // each, in column order, so one prefix sum runs through them); the columns
+  // Resolve the `rows` pixel rows from r on (delta rows 0 .. rows - 1, all in
+  // one band) and emit their tile rows.  Only the tile columns that hold
+  // deltas are summed, 16 of them at a time (four lanes of four pixels each,
+  // in column order, so one prefix sum runs through them); the columns
   // between take the value at the end of the touched column before them, one
-  // lane per column.
-  auto flush_row = [&](int r) {
+  // lane per column.  The rows lie end to end: a row's deltas add up to zero,
+  // so the sum starts each row at zero.
+  auto flush_rows = [&](int r, int rows) {
     WaveSync();
     const int rb = r >> 4;
     if (rb != band) {
       finish_band();
       band = rb;
     }
-    const int rowk = r & 15;
+    const int rowk0 = r & 15;
+    const int cols = rows * ncol;
+    // column -> row and tile column (col < 2^11, and the quotient is at least
+    // 1 / (2 ncol) away from an integer)
+    const float inv = rows > 1 ? __builtin_amdgcn_rcpf((float)ncol) : 0.f;
+    auto place = [&](int col, int* row, int* tcol) {
+      *row = 0;
+      *tcol = col;
+      if (rows > 1) {
+        const int q = (int)(((float)col + 0.5f) * inv);
+        *row = q;
+        *tcol = col - __mul24(q, ncol);
+      }
+    };
     int carry = 0;
-    for (int g = 0; g < tr.ntc; g += kWave) {
+    for (int g = 0; g < cols; g += kWave) {
       const uint32_t* tw = L.touch + 2 * (g / kWave);
       const uint64_t T = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)tw[0]) |
                          (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)tw[1]) << 32;
@@ -532,13 +566,15 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
         const int nt = __popcll(T);
         for (int b = 0; b < nt; b += kWave / 4) {
           const int ti = b + (lane >> 2), sub = lane & 3;
-          // (a bit past the last column is the end-of-row entry's)
-          const int col = ti < nt ? L.list[ti] : kWave;
-          const int tcol = g + col;
-          const bool ok = col < kWave && tcol < tr.ntc;
+          const bool held = ti < nt;
+          const int col = held ? L.list[ti] : 0;
+          int jrow, tcol;
+          place(g + col, &jrow, &tcol);
+          const bool ok = held && tcol < tr.ntc;  // not the end-of-row column
+          const int rowk = rowk0 + jrow;
           int4 dv = make_int4(0, 0, 0, 0);
-          if (ok) {
-            int4* dp = (int4*)(L.d + tcol * kTile + 4 * sub);
+          if (held) {
+            int4* dp = (int4*)(L.d + (g + col) * kTile + 4 * sub);
             dv = *dp;
             *dp = make_int4(0, 0, 0, 0);
           }
@@ -546,7 +582,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
           const int incl = ScanSum(t3);
           const int e = incl - t3 + carry;
           carry += __builtin_amdgcn_readlane(incl, kWave - 1);
-          if (ok && sub == 3) L.vend[col] = e + t3;
+          if (held && sub == 3) L.vend[col] = e + t3;
           uint32_t c0 = 0, c1 = 0, c2 = 0, f, s2, t;
           covers(e + dv.x, &f, &s2, &t);
           c0 = f, c1 = s2, c2 = t;
@@ -569,15 +605,20 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
           const bool plane0 = (st & 5) == 5, plane1 = (st & 2) != 0;
           const int cc = ok ? tcol : 0;
           if (sub == 0 && ok) {
-            if ((st & 5) == 1) atomicOr(&L.full[cc], 1 << rowk);
+            if ((st & 5) == 1) atomicOr(&L.full[cc >> 1], 1 << (16 * (cc & 1) + rowk));
             const int wr = (plane0 ? 1 << rowk : 0) | (plane1 ? 1 << (16 + rowk) : 0);
             if (wr) atomicOr(&L.rows[cc], wr);
           }
           int cur0 = L.slot0[cc], cur1 = L.slot1[cc];
-          const bool need0 = sub == 0 && plane0 && cur0 < 0;
-          const bool need1 = sub == 0 && plane1 && cur1 < 0;
+          bool need0 = sub == 0 && plane0 && cur0 < 0;
+          bool need1 = sub == 0 && plane1 && cur1 < 0;
           // most columns already hold their planes: allocate only when needed
           if (__ballot(need0 || need1) != 0) {
+            // several rows may meet the same column here: one of them asks
+            if (rows > 1) {
+              if (need0) need0 = atomicCAS(&L.slot0[cc], -1, -2) == -1;
+              if (need1) need1 = atomicCAS(&L.slot1[cc], -1, -2) == -1;
+            }
             take_planes(need0, need1, cc);
             cur0 = L.slot0[cc];
             cur1 = L.slot1[cc];
@@ -600,24 +641,32 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
         WaveSync();
       }
       // the other columns of the group
-      const int c = g + lane;
       const uint64_t below = T & ((1ull << lane) - 1);
       int v = v_in;
       if (below) v = L.vend[kWave - 1 - __builtin_clzll(below)];
-      const bool rest = c < tr.ntc && ((T >> lane) & 1) == 0 && v != 0;
+      int jrow, c;
+      place(g + lane, &jrow, &c);
+      const int rowk = rowk0 + jrow;
+      const bool rest = g + lane < cols && c < tr.ntc && ((T >> lane) & 1) == 0 && v != 0;
       if (__ballot(rest) == 0) continue;
       uint32_t f = 0, s2 = 0, t = 0;
       if (rest) covers(v, &f, &s2, &t);
       const bool is_full = !triple && f == 255 && s2 == 0;
       const bool plane0 = rest && !is_full && (triple ? (f | s2 | t) != 0 : f != 0);
       const bool plane1 = rest && !triple && s2 != 0;
-      if (rest && is_full) atomicOr(&L.full[c], 1 << rowk);
+      if (rest && is_full) atomicOr(&L.full[c >> 1], 1 << (16 * (c & 1) + rowk));
       if (__ballot(plane0 || plane1) == 0) continue;
       const int cc = rest ? c : 0;
       const int wr = (plane0 ? 1 << rowk : 0) | (plane1 ? 1 << (16 + rowk) : 0);
       if (wr) atomicOr(&L.rows[cc], wr);
-      const bool need0 = plane0 && L.slot0[cc] < 0, need1 = plane1 && L.slot1[cc] < 0;
-      if (__ballot(need0 || need1) != 0) take_planes(need0, need1, cc);
+      bool need0 = plane0 && L.slot0[cc] < 0, need1 = plane1 && L.slot1[cc] < 0;
+      if (__ballot(need0 || need1) != 0) {
+        if (rows > 1) {
+          if (need0) need0 = atomicCAS(&L.slot0[cc], -1, -2) == -1;
+          if (need1) need1 = atomicCAS(&L.slot1[cc], -1, -2) == -1;
+        }
+        take_planes(need0, need1, cc);
+      }
       if (kWrite) {
         const int cur0 = L.slot0[cc], cur1 = L.slot1[cc];
         auto put = [&](int slot, uint32_t b) {
@@ -977,8 +1026,9 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
   }
 
   const Fixed stop_fixed = IntToFixed(pb.b);
-  int guard = 0;
-  // Phase times (10 ns units) of every 16th step: reading the clock waits for
+  int guard = 0;  // steps taken
+  uint32_t turn = 0;
+  // Phase times (10 ns units) of every 16th turn: reading the clock waits for
   // it and for the LDS operations in flight, which took a third of a small
   // step when every step did it five times.
   uint64_t ph[5] = {0, 0, 0, 0, 0};
@@ -1017,7 +1067,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
       flags |= 32;
       break;
     }
-    const bool sample = (guard & 15) == 1;
+    const bool sample = (turn++ & 15) == 0;
     max_active = Max32(max_active, n);
     Fixed next_y = Min32(nny, FixedCeilToFixed(y + 1));
     int y_shift = 0;
@@ -1032,6 +1082,52 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
     const int S = (n + kWave - 1) / kWave;
     // rows off the canvas are stepped but not drawn
     const bool draw = kBlit && row >= cy0 && row < cy1;
+    // ---- several rows at once ----------------------------------------------------
+    // From a whole row on, until the first event (an edge ends or begins),
+    // every step is one whole row as long as no two edges cross, and the list
+    // stays as it is: row i is x + i dx.  Each neighbouring pair moves apart
+    // or together linearly, so a list in order now and after `rows` rows is in
+    // order on all rows between, and the steps up to there are taken as one.
+    // A list of few edges, most of them, takes 16 rows (a band, as many delta
+    // rows as fit) in little more than the time of one.
+    int rows = 1;
+    if ((y & 0xFFFF) == 0) {
+      int most = Min32((nny - 1) >> 16, stop_fixed >> 16) - row;
+      if (kWrite && stop_y != kMaxS32) most = Min32(most, (stop_y >> 16) - row);
+      if (!kWrite && next_b < nb) {
+        // not past the row of the next snapshot
+        const int at = Max32(BandStartRow(pb, nb, next_b), (row + kTile) & ~(kTile - 1));
+        most = Min32(most, at - row);
+      }
+      if (draw) {
+        most = Min32(most, Min32(row_cap, kTile - (row & (kTile - 1))));
+        most = Min32(most, cy1 - row);
+      } else {
+        most = Min32(most, kWave - 1);
+        if (kBlit && row < cy0) most = Min32(most, cy0 - row);
+      }
+      if (most > 1) {
+        // no overflow on the way: |x| < 2^30, |63 dx| < 2^29
+        bool off = false;
+        Fixed cx = kMinS32, cj = kMinS32;
+#pragma unroll
+        for (int s = 0; s < K; s++) {
+          if (s >= S) break;
+          const bool valid = s * kWave + lane < n;
+          const Fixed x0 = X[s], xj = x0 + __mul24(DX[s], most);
+          const Fixed p0 = ShiftUp(x0, cx), pj = ShiftUp(xj, cj);
+          off |= valid && (p0 > x0 || pj > xj || (uint32_t)(DX[s] + (1 << 23)) >= (1u << 24) ||
+                           (uint32_t)(x0 + (1 << 30)) >= (1u << 31));
+          cx = __builtin_amdgcn_readlane(x0, kWave - 1);
+          cj = __builtin_amdgcn_readlane(xj, kWave - 1);
+        }
+        if (__ballot(off) == 0) {
+          rows = most;
+          next_y = y + rows * kFixed1;
+          guard += rows - 1;
+        }
+      }
+    }
 
     uint64_t tp0 = 0, tp1 = 0, tp2 = 0, tp3 = 0, tp4 = 0;
     if (sample) tp0 = wall_clock64();
@@ -1056,8 +1152,8 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
         const int rem = n - s * kWave;
         const uint64_t bval = rem >= kWave ? ~0ull : (1ull << rem) - 1;
         const bool valid = lane < rem;
-        const Fixed xo = X[s], dx = DX[s];
-        const Fixed xn = xo + (dx >> y_shift);
+        const Fixed xo = X[s], dx = DX[s], step = dx >> y_shift;
+        const Fixed xn = rows > 1 ? xo + __mul24(dx, rows) : xo + step;
         if (draw) {
           const bool neg = (M[s] & 1) != 0;
           const uint64_t bneg = __ballot(neg) & bval, bpos = bval & ~bneg;
@@ -1076,10 +1172,17 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
             }
           }
           if (__builtin_amdgcn_inverse_ballot_w64(bl))
-            L.iL[CountBelow(bl, nl)] = make_int4(xo, xn, DY[s], 0);
+            L.iL[CountBelow(bl, nl)] = make_int4(xo, step, DY[s], 0);
           if (__builtin_amdgcn_inverse_ballot_w64(br)) {
-            const bool close = lane + 1 < rem && (xn + kFixed1 >= nxo - Abs32(ndx));
-            L.iR[CountBelow(br, nr)] = make_int4(xo, xn, DY[s], close ? 1 : 0);
+            const int at = CountBelow(br, nr);
+            int next = lane + 1 < rem ? kNextCheck : kNextNone;
+            if (kWide) {
+              if (next != kNextNone)
+                next = xn + kFixed1 >= nxo - Abs32(ndx) ? kNextClose : kNextNone;
+            } else {
+              L.iN[at] = make_int2(nxo, ndx);
+            }
+            L.iR[at] = make_int4(xo, step, DY[s], next);
           }
           nl += __popcll(bl);
           nr += __popcll(br);
@@ -1106,28 +1209,53 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
         // The left edge's list predecessor is not tracked; the span is
         // emitted as accumulated coverage.
         flags |= 8;
-        if (lane == 0) L.iR[nr] = make_int4(right_clip, right_clip, 0, 1);
+        if (lane == 0) {
+          L.iR[nr] = make_int4(right_clip, 0, 0, kNextClose);
+          if (!kWide) L.iN[nr] = make_int2(0, 0);
+        }
         nr++;
       }
       WaveSync();
-      for (int k0 = 0; k0 < nr; k0 += kWave) {
-        const int k = k0 + lane;
-        const bool act = k < nr;
+      // two lanes (left and right edge) per interval and row
+      const int total = nr * rows;
+      // (rows > 1: t / nr by a product; t < 2^13, and a quotient is at least
+      // 1 / (2 nr) away from an integer)
+      const float inv = rows > 1 ? __builtin_amdgcn_rcpf((float)nr) : 0.f;
+      for (int t0 = 0; t0 < total; t0 += kWave / 2) {
+        const int t = t0 + (lane >> 1);
+        const bool act = t < total;
+        int jr = 0, k = t;
+        if (rows > 1) {
+          jr = (int)(((float)t + 0.5f) * inv);
+          k = t - __mul24(jr, nr);
+        }
         int4 l = make_int4(0, 0, 0, 0), r = l, q = l;
+        int2 nx = make_int2(0, 0);
         if (act) {
           l = L.iL[k];
           r = L.iR[k];
+          if (!kWide) nx = L.iN[k];
           if (k > 0) q = L.iR[k - 1];
         }
-        const Fixed left = Max32(l.x, left_clip), next_left = Max32(left_clip, l.y);
-        const Fixed right = Min32(right_clip, r.x), next_right = Min32(right_clip, r.y);
-        const int prev_right = k > 0 ? FixedCeilToInt(Max32(Min32(right_clip, q.x), q.y))
+        if (rows > 1) {
+          l.x += __mul24(l.y, jr);
+          r.x += __mul24(r.y, jr);
+          q.x += __mul24(q.y, jr);
+          nx.x += __mul24(nx.y, jr);
+        }
+        const Fixed lxn = l.x + l.y, rxn = r.x + r.y;
+        const Fixed left = Max32(l.x, left_clip), next_left = Max32(left_clip, lxn);
+        const Fixed right = Min32(right_clip, r.x), next_right = Min32(right_clip, rxn);
+        const int prev_right = k > 0 ? FixedCeilToInt(Max32(Min32(right_clip, q.x), q.x + q.y))
                                      : FixedFloorToInt(left_clip);
         const bool close_prev =
-            prev_right > FixedFloorToInt(left) || prev_right > FixedFloorToInt(l.y);
-        const bool no_real = full == 0xFF && (close_prev || r.w != 0);
-        BlitIntervals(sink, L.blit, act, left, right, next_left, next_right, l.z, r.z, full,
-                      no_real);
+            prev_right > FixedFloorToInt(left) || prev_right > FixedFloorToInt(lxn);
+        const bool close_next =
+            r.w == kNextClose ||
+            (r.w == kNextCheck && (rxn + kFixed1 >= nx.x - Abs32(nx.y)));
+        const bool no_real = full == 0xFF && (close_prev || close_next);
+        BlitEdges(sink, L.blit, act, lane & 1, jr, left, right, next_left, next_right, l.z, r.z,
+                  full, no_real);
       }
       WaveSync();
     }
@@ -1414,7 +1542,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
     }
     // ---- row completion ------------------------------------------------------
     y = next_y;
-    if (draw && (y & 0xFFFF) == 0) flush_row(row);
+    if (draw && (y & 0xFFFF) == 0) flush_rows(row, rows);
     if (sample) {
       tp4 = wall_clock64();
       ph[3] += tp4 - tp3;

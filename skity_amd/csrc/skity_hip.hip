@@ -1113,8 +1113,20 @@ constexpr int kBandMinEdges = 4 * kWave + 1;
 constexpr int kBandMinRows = 512;
 constexpr int kBandSlots = 512;
 
-size_t WalkLdsBytes(int K, int lds_width) {
-  return (size_t)WalkLdsInts(K, lds_width) * sizeof(int32_t);
+size_t WalkLdsBytes(int K, int lds_width, int row_ints) {
+  return (size_t)WalkLdsInts(K, lds_width, row_ints) * sizeof(int32_t);
+}
+
+// Delta row words of a walk wave: at least one row of the frame's widest path.
+// More rows let the walk take more rows at once on narrower paths, and cost
+// resident waves, so a frame gets what its walks leave of the LDS: 160 KB a CU
+// over the walks per CU, up to 8,192 words (16 rows of 500 pixels) and at
+// least 2,048 (16 rows of 112).
+int WalkRowCapacity(hipr_context ctx, int lds_width, int64_t walks) {
+  const int64_t per_cu = (walks + std::max(ctx->n_cus, 1) - 1) / std::max(ctx->n_cus, 1);
+  int64_t ints = 160 * 1024 / 4 / std::max<int64_t>(per_cu, 1) - 3072;
+  ints = std::min<int64_t>(std::max<int64_t>(ints, 2048), 8192) & ~(int64_t)(kTile - 1);
+  return (int)std::max<int64_t>(ints, WalkRowInts(lds_width));
 }
 
 hipr_result WalkLdsCheck(hipr_context ctx, int K, size_t lds) {
@@ -1130,7 +1142,7 @@ template <int K, int kMode>
 hipr_result LaunchWalk(hipr_context ctx, WalkParams P, hipStream_t st, bool timed,
                        int32_t* queue, double share) {
   if (P.n_walk == 0) return HIPR_SUCCESS;
-  size_t lds = WalkLdsBytes(K, P.lds_width);
+  size_t lds = WalkLdsBytes(K, P.lds_width, P.row_ints);
   if (hipr_result r = WalkLdsCheck(ctx, K, lds)) return r;
   unsigned grid = (unsigned)P.n_walk;
   P.queue = queue;
@@ -1159,7 +1171,9 @@ hipr_result LaunchWalkWide(hipr_context ctx, int K, int kmode, WalkParams P, hip
                            bool timed) {
   if (P.n_walk == 0) return HIPR_SUCCESS;
   if (kmode == kWalkSchedule) return HIPR_ERROR_INVALID_ARGUMENT;  // wide jobs are unbanded
-  size_t lds = WalkLdsBytes(K, P.lds_width);
+  // (their lists fill the LDS: one delta row)
+  P.row_ints = WalkRowInts(P.lds_width);
+  size_t lds = WalkLdsBytes(K, P.lds_width, P.row_ints);
   if (hipr_result r = WalkLdsCheck(ctx, K, lds)) return r;
   P.queue = nullptr;
   const int stage = kmode == kWalkCount ? HIPR_STAGE_WALK_COUNT : HIPR_STAGE_WALK;
@@ -1635,6 +1649,7 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   wp.canvases = ctx->canvases.as<Canvas>();
   wp.cov = ctx->cov.as<JobCov>();
   wp.lds_width = lds_width;
+  wp.row_ints = WalkRowCapacity(ctx, lds_width, nwalk);
   wp.map_base = ctx->map_base.as<int64_t>();
   // ---- stage (b): walk ----
   // The walk keeps the active edge list in registers.  The sort bounded each
