@@ -236,7 +236,9 @@ typedef struct hipr_stats {
                              overflow pool, or re-run when it ran out)      */
 } hipr_stats;
 
-/* Execution options.  mode 0 = plain exact two-pass (count, scan, write);
+/* Execution options.  mode 0 = plain exact: edges are counted, then written;
+ * tile planes are reserved for every tile a path could cover where that takes
+ * at most 4 GiB (one walk), else counted and then written (two walks);
  * mode 1 = pre-sized single pass from the caller-supplied per-path estimates
  * (estimates != NULL), falling back to the exact two-pass method for every
  * path whose estimate was too small; mode 2 = pre-sized from the context's
@@ -251,8 +253,9 @@ typedef struct hipr_options {
   const int32_t* tile_estimates;  /* n_paths or NULL */
   int32_t blur_impl;              /* HIPR_BLUR_IMPL_*; 0 = MFMA */
   int32_t band_rows;              /* rows per walk band: 0 = default (128
-                                     exact, 64 estimate modes), < 0 = one
-                                     band per path */
+                                     where the planes are counted, else 64),
+                                     < 0 = one band per path; exact mode
+                                     counts the planes unless it is 0 */
   int32_t band_min_edges;         /* estimate modes: band only the paths whose
                                      active-edge bound reaches this; 0 = default
                                      (257: the 8- and 16-slot walks), < 0 =

@@ -1102,16 +1102,18 @@ constexpr int kBandRowsEstimates = 64;
 // (Banding every path costs more schedule work than it saves; the
 // autotuner tries other thresholds.)
 constexpr int kBandMinEdges = 4 * kWave + 1;
-// ... and so are paths whose scan bounds span this many rows: a large
-// outline with a short active list (the tiger at 4096^2: 2,000-4,000 steps
-// per path) is as long a sequential walk, and its schedule pass costs a
-// fraction of the write it splits (tiger.skp at 4096^2, learned: walk
-// 34.5 -> 10 ms when every path is banded at 64 rows).  In a frame of many
-// paths they are not the critical path, and banding all of them costs more
-// than it saves (curves + strokes at 2048^2, learned: 175 -> 231 ms), hence
-// the frame-relative threshold below.
-constexpr int kBandMinRows = 512;
-constexpr int kBandSlots = 512;
+// ... and so are paths whose scan bounds span at least this many rows, and
+// more than the frame's rows spread over the walks that fit the device at
+// once (two per SIMD): a large outline with a short active list is as long a
+// sequential walk, its schedule pass takes a fraction of the write it splits,
+// and a frame of few walks leaves the waves for its bands.  In a frame of
+// many paths they are not the critical path, and banding all of them costs
+// more than it saves (curves + strokes at 2048^2, learned: 175 -> 231 ms).
+constexpr int kBandMinRows = 128;
+constexpr int kBandSlots = 2048;
+// Exact form: planes for every tile a path could cover, up to this many (4
+// GiB), make the count pass unnecessary.
+constexpr int64_t kUncountedPlanes = 16 << 20;
 
 size_t WalkLdsBytes(int K, int lds_width, int row_ints) {
   return (size_t)WalkLdsInts(K, lds_width, row_ints) * sizeof(int32_t);
@@ -1663,6 +1665,24 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
                          st));
   HIP_TRY(hipStreamSynchronize(st));
   const std::vector<int32_t>& all = pl->walk_jobs;
+  // Planes a job can use at most: two per visible tile, a keep-zero job three
+  // (every tile row belongs to one band).
+  auto most_planes = [&](int32_t j) -> int64_t {
+    const Canvas& cv = f.canvases[f.jobs[j].canvas];
+    const TileRange tr = JobTiles(JobScanBounds(ctx->h_geo[j]), cv.width, cv.height);
+    return (int64_t)tr.ntc * tr.ntr * ((f.jobs[j].flags & kJobKeepZero) ? 3 : 2);
+  };
+  // Exact form, uncounted: where the planes every job could use fit a bounded
+  // buffer, they are reserved (a plane that is not used is not touched) and
+  // the write pass takes what it needs, without the count pass, which is as
+  // long a walk as the write.  The row bands then come from a schedule pass,
+  // as in the estimate forms.  A caller that sets the band rows gets the
+  // counted form.
+  int64_t most_total = 0;
+  for (int32_t j : all) most_total += std::max<int64_t>(most_planes(j), 1);
+  const bool uncounted =
+      mode == 0 && !(opt && opt->band_rows != 0) && most_total <= kUncountedPlanes;
+  const bool counted = mode == 0 && !uncounted;
   std::vector<int32_t> small, wide;
   std::vector<int8_t> tier(nj, 4);  // slots of each job's walk
   for (int32_t j : all) {
@@ -1679,21 +1699,21 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   // Row bands: each job's rows are split into bands walked concurrently by
   // the write pass; the count or schedule pass records where they start.
   const int band_rows = opt && opt->band_rows != 0 ? std::max(opt->band_rows, 0)
-                        : mode == 0                    ? kBandRowsExact
+                        : counted                      ? kBandRowsExact
                                                        : kBandRowsEstimates;
-  // In the estimate modes banding costs a schedule pass, so only the paths
+  // Without a count pass banding costs a schedule pass, so only the paths
   // with the widest active lists (the longest walks) are banded.
-  const int band_min =
-      mode == 0 ? 0
-      : (opt && opt->band_min_edges != 0) ? std::max(opt->band_min_edges, 0)
-                                          : kBandMinEdges;
-  // (estimate modes, default split only) paths this tall are banded too:
-  // at least kBandMinRows, and taller than the frame's rows spread over
-  // kBandSlots concurrent walks, so that only paths that would outlast the
-  // rest of the walk are split (a frame of many paths keeps its unbanded
-  // walks; one of a few large outlines bands them)
+  const bool own_split = mode != 0 && opt && opt->band_min_edges != 0;
+  const int band_min = counted     ? 0
+                       : own_split ? std::max(opt->band_min_edges, 0)
+                                   : kBandMinEdges;
+  // (default split only) paths this tall are banded too: at least
+  // kBandMinRows, and taller than the frame's rows spread over kBandSlots
+  // concurrent walks, so that only paths that would outlast the rest of the
+  // walk are split (a frame of many paths keeps its unbanded walks; one of a
+  // few large outlines bands them)
   int band_min_rows = 0;
-  if (mode != 0 && !(opt && opt->band_min_edges != 0)) {
+  if (!counted && !own_split) {
     int64_t total_rows = 0;
     for (int32_t j : all) {
       const PixBounds b = JobScanBounds(ctx->h_geo[j]);
@@ -1965,7 +1985,13 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
     return HIPR_SUCCESS;
   };
   JobCov* hw = ctx->h_wcov;
-  if (mode == 0) {
+  if (uncounted) {
+    test.resize(nj, 0);
+    for (int32_t j : all) {
+      pcap[j] = (int32_t)std::max<int64_t>(most_planes(j), 1);
+      test[j] = pcap[j];
+    }
+  } else if (counted) {
     // count pass over every job (recording the band snapshots), then planes
     // sized exactly
     if ((r = walk_pass(kWalkCount, small, wide)) != HIPR_SUCCESS) return r;
@@ -1975,17 +2001,9 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
     if ((r = move_overflowed(ctx->h_cov, nullptr)) != HIPR_SUCCESS) return r;
     for (int32_t j : all) pcap[j] = ctx->h_cov[j].planes;
   } else {
-    // planes from the estimates, at most what the job can use: three planes
-    // (a keep-zero triple) per visible tile, and per band that meets the
-    // tile
-    for (int32_t j : all) {
-      const Canvas& cv = f.canvases[f.jobs[j].canvas];
-      const TileRange tr = JobTiles(JobScanBounds(ctx->h_geo[j]), cv.width, cv.height);
-      const int64_t bands_per_tile =
-          nbands[j] > 1 ? 1 + (kTile + std::max(band_rows, 1) - 1) / std::max(band_rows, 1) : 1;
-      const int64_t most = 3 * (int64_t)tr.ntc * tr.ntr * bands_per_tile;
-      pcap[j] = (int32_t)std::max<int64_t>(std::min<int64_t>(test[j], most), 1);
-    }
+    // planes from the estimates, at most what the job can use
+    for (int32_t j : all)
+      pcap[j] = (int32_t)std::max<int64_t>(std::min<int64_t>(test[j], most_planes(j)), 1);
   }
   assign_planes(all);
   // Estimate modes: a shared pool after the estimated ranges serves the
@@ -2006,7 +2024,7 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   wp.planes = ctx->planes.as<uint8_t>();
   wp.cov = ctx->wcov.as<JobCov>();
   if ((r = prepare_write(nullptr)) != HIPR_SUCCESS) return r;
-  if (mode == 0) {
+  if (counted) {
     if ((r = walk_pass(kWalkWrite, small, wide)) != HIPR_SUCCESS) return r;
   } else {
     // The banded (longest) walks need a schedule pass before their write
@@ -2037,7 +2055,7 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
       return r;
   }
   if ((r = read_cov(&ctx->wcov, hw)) != HIPR_SUCCESS) return r;
-  if (mode == 0) {
+  if (counted) {
     if ((r = limit_error(hw, all, 1 | 2 | 16 | 32)) != HIPR_SUCCESS) return r;
   } else {
     if ((r = limit_error(hw, wide, 2)) != HIPR_SUCCESS) return r;
