@@ -34,6 +34,8 @@ namespace hipr {
 constexpr int kTilePlaneBytes = kTile * kTile;
 // Tile slot of an allocation that found no plane (capacity and pool spent).
 constexpr int32_t kNoPlane = 0x7FFFFFFF;
+// Planes the bands of a job take at a time (a multiple of three).
+constexpr int kPlaneChunk = 48;
 // Map entries: a plane number, or no coverage, or a tile whose every pixel
 // has the first cover 255, which needs no plane.
 constexpr int32_t kNoTile = -1;
@@ -268,9 +270,9 @@ __device__ void BitonicSortSlots(int64_t (&key)[K], int N, int lane) {
 }
 
 // Write pass (kWalkWrite): one wave per (job, band) item; the job's map
-// starts at kNoTile (filled before the launch), its JobCov at zero, and planes
-// are taken from the job's counter (JobCov::alloc) with atomics, so the bands
-// of a job run concurrently.  Count and schedule passes: one wave per job, band
+// starts at kNoTile (filled before the launch), its JobCov at zero, and the
+// bands of a job, which run concurrently, take planes from the job's counter
+// (JobCov::alloc).  Count and schedule passes: one wave per job, band
 // 0, walking every row and recording the band snapshots.
 template <int K, int kMode>
 __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* lds) {
@@ -385,6 +387,8 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
   for (int t = 0; t < K; t++) X[t] = DX[t] = DY[t] = LY[t] = M[t] = 0;
   int n = 0;
   int n_planes = 0;   // planes of this lane's tiles (a solid tile counts one)
+  int next_slot = 0;  // next plane of the job's range
+  int chunk_end = 0;  // end of the chunk taken (several bands)
   int band = -1;      // current 16-row band
 
   // ---- helpers ---------------------------------------------------------------
@@ -406,38 +410,56 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
   // Takes planes for the tile columns `c` of the lanes that need one: plane 0
   // (three of them for a keep-zero job) and / or plane 1 of the column.
   // Count pass: nothing to take, the slots are only marked as held.
+  // A job walked by one wave counts its planes itself; the bands of a job
+  // share its range and take it kPlaneChunk planes at a time (the host adds
+  // that much per band), so that a flush hardly ever waits for an atomic's
+  // answer.
   auto take_planes = [&](bool need0, bool need1, int c) {
     int a0 = 0, a1 = 0;
     if (kWrite) {
       const int req = triple ? (need0 ? 3 : 0) : (need0 ? 1 : 0) + (need1 ? 1 : 0);
       const int rincl = ScanSum(req);
       const int rtot = __builtin_amdgcn_readlane(rincl, kWave - 1);
-      // the bands of a job share its plane range
-      int got = 0;
-      if (lane == 0) got = atomicAdd(&P.cov[j].alloc, rtot);
-      const int slot_base = __builtin_amdgcn_readlane(got, 0);
-      a0 = slot_base + rincl - req;
+      const int at = rincl - req;
+      a0 = next_slot + at;
       a1 = a0 + (need0 ? 1 : 0);
+      if (nb > 1 && next_slot + rtot > chunk_end) {
+        // the rest of the chunk, then a new one (chunks and triples are both
+        // multiples of three)
+        const int more = next_slot + rtot - chunk_end;
+        const int grab = (more + kPlaneChunk - 1) / kPlaneChunk * kPlaneChunk;
+        int got = 0;
+        if (lane == 0) got = atomicAdd(&P.cov[j].alloc, grab);
+        got = __builtin_amdgcn_readlane(got, 0);
+        if (a0 >= chunk_end) a0 += got - chunk_end;
+        if (a1 >= chunk_end) a1 += got - chunk_end;
+        next_slot = got + more;
+        chunk_end = got + grab;
+      } else {
+        next_slot += rtot;
+      }
       // absolute plane numbers, from the job's range or (past its capacity)
       // from the pool
-      const int over_from = slot_base > pcap ? slot_base : pcap;
-      const int over = slot_base + rtot - over_from;
-      int pool0 = 0;
-      if (over > 0) {
+      const bool over0 = need0 && a0 + (triple ? 2 : 0) >= pcap, over1 = need1 && a1 >= pcap;
+      int p0 = (int)(pbase + a0), p1 = (int)(pbase + a1);
+      if (__ballot(over0 || over1) != 0) {
+        // a triple must be contiguous: it never comes from the pool (a
+        // job that outgrows its range that way is walked again exactly)
+        const int ov = triple ? 0 : (over0 ? 1 : 0) + (over1 ? 1 : 0);
+        const int oincl = ScanSum(ov);
+        const int otot = __builtin_amdgcn_readlane(oincl, kWave - 1);
         int pg = 0;
-        if (lane == 0) pg = atomicAdd(P.pool_ctr, over);
-        pool0 = __builtin_amdgcn_readlane(pg, 0);
+        if (lane == 0 && otot > 0) pg = atomicAdd(P.pool_ctr, otot);
+        int pi = __builtin_amdgcn_readlane(pg, 0) + oincl - ov;
+        if (over0) {
+          p0 = !triple && pi < P.pool_cap ? P.pool_base + pi : kNoPlane;
+          pi++;
+        }
+        if (over1) p1 = pi < P.pool_cap ? P.pool_base + pi : kNoPlane;
+        if ((over0 && p0 == kNoPlane) || (over1 && p1 == kNoPlane)) flags |= 1;
       }
-      auto to_abs = [&](int sl) -> int {
-        if (sl < pcap) return (int)(pbase + sl);
-        int pi = pool0 + (sl - over_from);
-        return pi < P.pool_cap ? P.pool_base + pi : kNoPlane;
-      };
-      // a triple must be contiguous: it never comes from the pool (a
-      // job that outgrows its range that way is walked again exactly)
-      a0 = triple ? (a0 + 2 < pcap ? (int)(pbase + a0) : kNoPlane) : to_abs(a0);
-      a1 = to_abs(a1);
-      if ((need0 && a0 == kNoPlane) || (need1 && a1 == kNoPlane)) flags |= 1;
+      a0 = p0;
+      a1 = p1;
     }
     if (need0) L.slot0[c] = a0;
     if (need1) L.slot1[c] = a1;
@@ -583,15 +605,30 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
           const int e = incl - t3 + carry;
           carry += __builtin_amdgcn_readlane(incl, kWave - 1);
           if (held && sub == 3) L.vend[col] = e + t3;
-          uint32_t c0 = 0, c1 = 0, c2 = 0, f, s2, t;
-          covers(e + dv.x, &f, &s2, &t);
-          c0 = f, c1 = s2, c2 = t;
-          covers(e + t1, &f, &s2, &t);
-          c0 |= f << 8, c1 |= s2 << 8, c2 |= t << 8;
-          covers(e + t2, &f, &s2, &t);
-          c0 |= f << 16, c1 |= s2 << 16, c2 |= t << 16;
-          covers(e + t3, &f, &s2, &t);
-          c0 |= f << 24, c1 |= s2 << 24, c2 |= t << 24;
+          // Most rows have only one kind of span in 16 columns: steps of less
+          // than a row accumulate, and a step of a whole row sends its spans
+          // directly unless edges are close.
+          const int v0 = e + dv.x, v1 = e + t1, v2 = e + t2, v3 = e + t3;
+          const uint32_t any = (uint32_t)(v0 | v1 | v2 | v3);
+          uint32_t c0 = 0, c1 = 0, c2 = 0;
+          if (!triple && __ballot((any >> 16) != 0) == 0) {
+            c0 = (uint32_t)Min32(v0, 255) | (uint32_t)Min32(v1, 255) << 8 |
+                 (uint32_t)Min32(v2, 255) << 16 | (uint32_t)Min32(v3, 255) << 24;
+          } else if (!triple && __ballot((any & 0xEF00FFFFu) != 0) == 0) {
+            // direct covers up to 255, one span at a pixel
+            c0 = ((uint32_t)v0 >> 16 & 0xFF) | ((uint32_t)v1 >> 8 & 0xFF00) |
+                 ((uint32_t)v2 & 0xFF0000) | ((uint32_t)v3 << 8 & 0xFF000000);
+          } else {
+            uint32_t f, s2, t;
+            covers(v0, &f, &s2, &t);
+            c0 = f, c1 = s2, c2 = t;
+            covers(v1, &f, &s2, &t);
+            c0 |= f << 8, c1 |= s2 << 8, c2 |= t << 8;
+            covers(v2, &f, &s2, &t);
+            c0 |= f << 16, c1 |= s2 << 16, c2 |= t << 16;
+            covers(v3, &f, &s2, &t);
+            c0 |= f << 24, c1 |= s2 << 24, c2 |= t << 24;
+          }
           // the tile row's state over its four lanes: bit 0 a cover in plane
           // 0, bit 1 one in plane 1, bit 2 not full
           int st = 0;

@@ -1775,6 +1775,8 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   };
   auto assign_planes = [&](const std::vector<int32_t>& js) {
     for (int32_t j : js) {
+      // the last chunk of each band may be left over in part
+      if (nbands[j] > 1) pcap[j] += nbands[j] * kPlaneChunk;
       pbase[j] = plane_total;
       plane_total += pcap[j];
     }
