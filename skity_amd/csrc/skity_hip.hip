@@ -1206,18 +1206,25 @@ struct Frame {
   hipr_stats stats{};
 };
 
-// Stroke outlines of the frame's stroke jobs.  Exact form: a count pass,
-// then a write pass into exact ranges.  Estimate forms (`single_pass`): one
-// write pass into ranges sized from each job's quad-path segment count
-// (an outline has at most ~12 verbs, ~19 points and ~0.7 conic weights per
-// segment on the workloads measured); a job whose outline outgrew its range
-// reports its exact sizes and is written again into an exact range.
-hipr_result RunStrokes(Frame& f, bool single_pass) {
+// Stroke outlines of the frame's stroke jobs: one write pass into ranges sized
+// from each job's quad-path segment count (an outline has at most ~12 verbs,
+// ~19 points and ~0.7 conic weights per segment on the workloads measured; in
+// the exact form six weights, what round joins of a polyline take); a
+// job whose outline outgrew its range reports its exact sizes and is written
+// again into an exact range (counted as a fallback in the estimate forms).
+// Exact form of a frame of more than kStrokeQuadsReserved segments: a count
+// pass, then a write pass into exact ranges; below that the ranges are small
+// (440 B a segment) and the count pass, as long as the write, is saved.
+constexpr int64_t kStrokeQuadsReserved = 1 << 20;
+hipr_result RunStrokes(Frame& f, bool estimates) {
   hipr_context ctx = f.ctx;
   hipr_prepared_s* pl = f.pl;
   int ns = (int)pl->stroke_jobs.size();
   if (ns == 0) return HIPR_SUCCESS;
   hipStream_t st = f.st;
+  int64_t quads = 0;
+  for (int32_t q : pl->stroke_quads) quads += q;
+  const bool single_pass = estimates || (!pl->stroke_quads.empty() && quads <= kStrokeQuadsReserved);
   if (ctx->stroke_out.Ensure(sizeof(StrokeOut) * ns) != hipSuccess)
     return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
   GeomSrc gs{pl->verbs.as<uint8_t>(), pl->pts.as<float>(), pl->weights.as<float>()};
@@ -1293,7 +1300,7 @@ hipr_result RunStrokes(Frame& f, bool single_pass) {
     StrokeOut so{};
     so.nv = (int32_t)std::min<int64_t>(12 * q + 64, INT32_MAX / 4);
     so.np = (int32_t)std::min<int64_t>(20 * q + 64, INT32_MAX / 4);
-    so.nw = (int32_t)std::min<int64_t>(q + 16, INT32_MAX / 4);
+    so.nw = (int32_t)std::min<int64_t>(estimates ? q + 16 : 6 * q + 64, INT32_MAX / 4);
     so.inner_nv = so.nv;
     so.inner_np = so.np;
     so.inner_nw = so.nw;
@@ -1326,7 +1333,7 @@ hipr_result RunStrokes(Frame& f, bool single_pass) {
     redo_out.push_back(so);
   }
   if (redo_list.empty()) return HIPR_SUCCESS;
-  f.stats.fallbacks += (int64_t)redo_list.size();
+  if (estimates) f.stats.fallbacks += (int64_t)redo_list.size();
   if ((r = ensure_outlines(true)) != HIPR_SUCCESS) return r;
   if ((r = Upload(&ctx->stroke_redo, redo_list.data(), redo_list.size(), st)) != HIPR_SUCCESS ||
       (r = Upload(&ctx->stroke_redo_out, redo_out.data(), redo_out.size(), st)) != HIPR_SUCCESS)
