@@ -1654,7 +1654,8 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
   }
 }
 
-// The walk kernel.  Without a queue, workgroup i walks item i (the
+// The slot walk's kernel (paths of more than 64 active edges; up to 64 walk as
+// a team of one wave, hipr_walk_team.hpp).  Without a queue, workgroup i walks item i (the
 // dispatcher hands out items in list order).  With a queue (persistent
 // form), a grid sized to the resident waves takes items from an atomic
 // counter until the list is exhausted; every wave leaves when the counter

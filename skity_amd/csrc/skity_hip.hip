@@ -33,6 +33,7 @@
 #include "hipr_sort.hpp"
 #include "hipr_stroke.hpp"
 #include "hipr_walk.hpp"
+#include "hipr_walk_team.hpp"
 
 using namespace hipr;
 
@@ -305,13 +306,15 @@ GradDev MakeGradDev(const hipr_gradient& g, const Aff& ctm) {
 
 }  // namespace
 
+constexpr int kSideStreams = 3;
+
 struct hipr_context_s {
   int refs = 1;  // the handle itself + live surfaces and prepared scenes
   int device = 0;
   hipStream_t stream = nullptr;
-  hipStream_t side = nullptr;  // walk tiers run here and on side2, beside the main stream
-  hipStream_t side2 = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_join2 = nullptr;
+  // walk tiers run here, beside the main stream
+  hipStream_t side[kSideStreams] = {};
+  hipEvent_t ev_fork = nullptr, ev_join[kSideStreams] = {};
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   // per-draw device buffers (grow-only)
   DevBuf canvases, layer_canvases, geo, cov, edge_base, edge_cap, edges, wedges, gkeys;
@@ -326,8 +329,6 @@ struct hipr_context_s {
   DevBuf pool_ctr;                        // overflow plane pool counter
   int n_cus = 0;                          // compute units of the device
   int max_lds = 0;                        // LDS bytes one workgroup may take
-  std::vector<hipGraph_t> graphs;         // graphs of the walk passes in flight
-  std::vector<hipGraphExec_t> graph_execs;
   DevBuf stroke_out, o_verbs, o_pts, o_w, s_verbs, s_pts, s_w;
   DevBuf layers, blur_rows, blur_cols, blur_rb, blur_cb, blur_tmp, blur_jobs, blur_lines;
   DevBuf blur_raw, blur_styles;  // unblurred layers and jobs of the style pass
@@ -1140,31 +1141,82 @@ hipr_result WalkLdsCheck(hipr_context ctx, int K, size_t lds) {
   return HIPR_SUCCESS;
 }
 
-template <int K, int kMode>
-hipr_result LaunchWalk(hipr_context ctx, WalkParams P, hipStream_t st, bool timed,
-                       int32_t* queue, double share) {
+// Waves a schedule pass by teams may take of the device (half of the waves
+// that fit beside each other), 300 paths: lists of up to 400 edges 35 ms
+// against 55 ms by slots.
+constexpr int64_t kTeamWaves = 1024;
+
+// Launches `kernel` (a slot walk, or a team of `waves` waves) over P's items.
+hipr_result LaunchWalk(hipr_context ctx, void (*kernel)(WalkParams), int waves, size_t lds,
+                       int stage, WalkParams P, hipStream_t st, bool timed, int32_t* queue,
+                       double share) {
   if (P.n_walk == 0) return HIPR_SUCCESS;
-  size_t lds = WalkLdsBytes(K, P.lds_width, P.row_ints);
-  if (hipr_result r = WalkLdsCheck(ctx, K, lds)) return r;
+  if (hipr_result r = WalkLdsCheck(ctx, waves, lds)) return r;
   unsigned grid = (unsigned)P.n_walk;
   P.queue = queue;
   if (queue) {
-    // persistent form: as many waves as fit at once (this tier's share)
+    // persistent form: as many workgroups as fit at once (this tier's share)
     int per_cu = 0;
-    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, WalkKernel<K, kMode>, kWave,
-                                                         lds));
+    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)kernel,
+                                                         waves * kWave, lds));
     int64_t cap = (int64_t)std::max(per_cu, 1) * std::max(ctx->n_cus, 1);
     cap = std::max<int64_t>(1, (int64_t)((double)cap * share));
     grid = (unsigned)std::min<int64_t>(P.n_walk, cap);
   }
-  const int stage = kMode == kWalkCount   ? HIPR_STAGE_WALK_COUNT
-                    : kMode == kWalkWrite ? HIPR_STAGE_WALK
-                                          : HIPR_STAGE_WALK_SCHEDULE;
   hipEvent_t b = timed ? StageBegin(ctx, st) : nullptr;
-  hipLaunchKernelGGL((WalkKernel<K, kMode>), dim3(grid), dim3(kWave), lds, st, P);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(waves * kWave), lds, st, P);
   HIP_TRY(hipGetLastError());
   if (timed) StageEnd(ctx, stage, b, st);
   return HIPR_SUCCESS;
+}
+
+// The walk kernel of a tier (jobs of up to 64 * tier active edges) in a mode:
+// for up to 64 edges a team of one wave, above that one wave with its list in
+// register slots, or (schedule passes of few paths) a team.  A team takes the
+// steps of one path faster, but its waves wait for each other: the write pass
+// of curves + strokes, 4,096 paths, took 210 ms by teams and 89 ms by slots.
+struct WalkShape {
+  void (*kernel)(WalkParams);
+  int waves;
+  bool team;
+};
+WalkShape ShapeOf(int tier, int mode, int64_t items) {
+  if (tier == 1)
+    return {mode == kWalkCount   ? TeamWalkKernel<1, kWalkCount>
+            : mode == kWalkWrite ? TeamWalkKernel<1, kWalkWrite>
+                                 : TeamWalkKernel<1, kWalkSchedule>,
+            1, true};
+  if (mode == kWalkSchedule && tier >= 8 && items * tier <= kTeamWaves)
+    return {tier == 8 ? TeamWalkKernel<8, kWalkSchedule> : TeamWalkKernel<16, kWalkSchedule>, tier,
+            true};
+  if (mode == kWalkSchedule)
+    return {tier == 2   ? WalkKernel<2, kWalkSchedule>
+            : tier == 4 ? WalkKernel<4, kWalkSchedule>
+            : tier == 8 ? WalkKernel<8, kWalkSchedule>
+                        : WalkKernel<16, kWalkSchedule>,
+            1, false};
+  if (mode == kWalkCount)
+    return {tier == 2   ? WalkKernel<2, kWalkCount>
+            : tier == 4 ? WalkKernel<4, kWalkCount>
+            : tier == 8 ? WalkKernel<8, kWalkCount>
+                        : WalkKernel<16, kWalkCount>,
+            1, false};
+  return {tier == 2   ? WalkKernel<2, kWalkWrite>
+          : tier == 4 ? WalkKernel<4, kWalkWrite>
+          : tier == 8 ? WalkKernel<8, kWalkWrite>
+                      : WalkKernel<16, kWalkWrite>,
+          1, false};
+}
+hipr_result LaunchTier(hipr_context ctx, int tier, int mode, const WalkParams& P, hipStream_t st,
+                       bool timed, int32_t* queue, double share) {
+  const WalkShape w = ShapeOf(tier, mode, P.n_walk);
+  const size_t lds =
+      w.team ? (size_t)TeamLdsInts(w.waves, P.lds_width, P.row_ints) * sizeof(int32_t)
+             : WalkLdsBytes(tier, P.lds_width, P.row_ints);
+  const int stage = mode == kWalkCount   ? HIPR_STAGE_WALK_COUNT
+                    : mode == kWalkWrite ? HIPR_STAGE_WALK
+                                         : HIPR_STAGE_WALK_SCHEDULE;
+  return LaunchWalk(ctx, w.kernel, w.waves, lds, stage, P, st, timed, queue, share);
 }
 
 // The 32- and 64-slot walks (hipr_walk_wide.hip): one wave per job, never
@@ -1183,15 +1235,6 @@ hipr_result LaunchWalkWide(hipr_context ctx, int K, int kmode, WalkParams P, hip
   HIP_TRY(LaunchWideWalk(K, kmode, (unsigned)P.n_walk, lds, st, P));
   if (timed) StageEnd(ctx, stage, b, st);
   return HIPR_SUCCESS;
-}
-
-// Graphs launched by the walk passes; every pass is followed by a stream
-// synchronisation, so they are released at the start of the next pass.
-void ReleaseGraphs(hipr_context ctx) {
-  for (hipGraphExec_t e : ctx->graph_execs) (void)hipGraphExecDestroy(e);
-  for (hipGraph_t g : ctx->graphs) (void)hipGraphDestroy(g);
-  ctx->graph_execs.clear();
-  ctx->graphs.clear();
 }
 
 // ---- the device pipeline -----------------------------------------------------
@@ -1661,12 +1704,12 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   wp.row_ints = WalkRowCapacity(ctx, lds_width, nwalk);
   wp.map_base = ctx->map_base.as<int64_t>();
   // ---- stage (b): walk ----
-  // The walk keeps the active edge list in registers.  The sort bounded each
-  // job's list by its largest row overlap: jobs within 256 edges take the
-  // 4-slot walk on the main stream, the others the 8-slot (512 edges) or
-  // 16-slot (1024 edges) walk on a side stream, at the same time, and the
-  // rare longer lists the unbanded 32- or 64-slot walk (2048 and 4096
-  // edges).  A longer list is refused (HIPR_ERROR_CAPACITY).
+  // The walk keeps the active edge list in registers, one element per lane.
+  // The sort bounded each job's list by its largest row overlap: a job takes
+  // a team of one wave per 64 edges of its bound (1, 2, 4, 8 or 16 waves), and
+  // the rare list of more than 1,024 edges the unbanded 32- or 64-slot walk of
+  // one wave (2,048 and 4,096 edges).  A longer list is refused
+  // (HIPR_ERROR_CAPACITY).
   std::vector<int32_t> bound(nj, 0);
   HIP_TRY(hipMemcpyAsync(bound.data(), ctx->bound.p, sizeof(int32_t) * nj, hipMemcpyDeviceToHost,
                          st));
@@ -1691,17 +1734,17 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
       mode == 0 && !(opt && opt->band_rows != 0) && most_total <= kUncountedPlanes;
   const bool counted = mode == 0 && !uncounted;
   std::vector<int32_t> small, wide;
-  std::vector<int8_t> tier(nj, 4);  // slots of each job's walk
+  std::vector<int8_t> tier(nj, 1);  // waves (slots) of each job's walk
   for (int32_t j : all) {
     if (bound[j] > kMaxSlots * kWave) {
       std::fprintf(stderr, "skity_hip: draw %d keeps up to %d edges active (limit %d)\n",
                    f.jobs[j].path, bound[j], kMaxSlots * kWave);
       return HIPR_ERROR_CAPACITY;
     }
-    int k = 4;
+    int k = 1;
     while (bound[j] > k * kWave) k *= 2;
     tier[j] = (int8_t)k;
-    (tier[j] == 4 ? small : wide).push_back(j);
+    (tier[j] <= 4 ? small : wide).push_back(j);
   }
   // Row bands: each job's rows are split into bands walked concurrently by
   // the write pass; the count or schedule pass records where they start.
@@ -1823,28 +1866,20 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
       for (int b = 0; b < nbands[o.second]; b++) it.push_back((o.second << kBandBits) | b);
     return it;
   };
-  // One walk pass: the 4-slot jobs on the main stream, the 8- and 16-slot
-  // jobs on the side stream; the main stream waits for both.
-  // One walk pass: the 4-slot jobs on the main stream, the 8- and 16-slot
-  // jobs on the side stream; the main stream waits for both.  The item lists
-  // are uploaded first; the launches (queue reset, fork, tier kernels, join)
-  // are captured into a hipGraph and launched as one unless the caller asks
-  // for direct launches.
   const int run_flags = opt ? opt->flags : 0;
-  const bool use_graph = (run_flags & HIPR_FLAG_NO_GRAPH) == 0;
   const bool persistent = (run_flags & HIPR_FLAG_PERSISTENT) != 0;
-  // A launch plan: walk kernels, each on one of three streams (0 = main);
-  // launches on one stream run in order, the streams concurrently.  The item
-  // lists are uploaded first; the launches (queue reset, fork, kernels, join)
-  // are captured into a hipGraph and launched as one unless the caller asks
-  // for direct launches.
+  // A launch plan: walk kernels, each on the main stream (0) or a side stream;
+  // launches on one stream run in order, the streams concurrently, and the
+  // main stream waits for all.  The item lists are uploaded first.  (The plan
+  // was captured into a hipGraph once; a graph is made for each draw, and
+  // making and launching it took 5 to 10 us more than the launches for a plan
+  // of one kernel and 100 us more for one of two streams.)
   struct WalkLaunch {
     int kmode, K, stream;
     std::vector<int32_t> jobs;
   };
   auto run_plan = [&](const std::vector<WalkLaunch>& plan) -> hipr_result {
     hipr_result rr;
-    ReleaseGraphs(ctx);
     std::vector<int32_t> all_items;
     std::vector<size_t> off, cnt;
     std::vector<double> work;
@@ -1870,86 +1905,107 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
     if (persistent && ctx->queues.Ensure(sizeof(int32_t) * (plan.size() + 1)) != hipSuccess)
       return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
     int32_t* q = persistent ? ctx->queues.as<int32_t>() : nullptr;
-    hipStream_t streams[3] = {st, ctx->side, ctx->side2};
-    hipEvent_t joins[3] = {nullptr, ctx->ev_join, ctx->ev_join2};
-    bool used[3] = {true, false, false};
+    // one stream alone is the main stream
+    int only = -1;
+    for (size_t i = 0; i < plan.size(); i++) {
+      if (!cnt[i]) continue;
+      only = only < 0 || only == plan[i].stream ? plan[i].stream : kSideStreams + 1;
+    }
+    auto stream_of = [&](size_t i) { return plan[i].stream == only ? 0 : plan[i].stream; };
+    bool used[kSideStreams + 1] = {true};
     for (size_t i = 0; i < plan.size(); i++)
-      if (cnt[i]) used[plan[i].stream] = true;
-    const bool timed = !use_graph;
-    auto launches = [&]() -> hipr_result {
-      if (q)
-        hipLaunchKernelGGL(FillKernel, dim3(1), dim3(kWave), 0, st, q, (int64_t)plan.size(), 0);
-      HIP_TRY(hipEventRecord(ctx->ev_fork, st));
-      for (int k = 1; k < 3; k++)
-        if (used[k]) HIP_TRY(hipStreamWaitEvent(streams[k], ctx->ev_fork, 0));
-      for (size_t i = 0; i < plan.size(); i++) {
-        if (!cnt[i]) continue;
-        const WalkLaunch& l = plan[i];
-        WalkParams w = wp;
-        w.walk_list = ctx->sub_list.as<int32_t>() + off[i];
-        w.n_walk = (int32_t)cnt[i];
-        w.cov = l.kmode == kWalkWrite ? ctx->wcov.as<JobCov>() : ctx->cov.as<JobCov>();
-        int32_t* qi = q ? q + i : nullptr;
-        double share = work_all > 0 ? work[i] / work_all : 1.0;
-        hipStream_t ls = streams[l.stream];
-        hipr_result lr;
-#define HIPR_WALK_K(KK)                                                             \
-  (l.kmode == kWalkCount   ? LaunchWalk<KK, kWalkCount>(ctx, w, ls, timed, qi, share) \
-   : l.kmode == kWalkWrite ? LaunchWalk<KK, kWalkWrite>(ctx, w, ls, timed, qi, share) \
-                           : LaunchWalk<KK, kWalkSchedule>(ctx, w, ls, timed, qi, share))
-        lr = l.K == 4    ? HIPR_WALK_K(4)
-             : l.K == 8  ? HIPR_WALK_K(8)
-             : l.K == 16 ? HIPR_WALK_K(16)
-                         : LaunchWalkWide(ctx, l.K, l.kmode, w, ls, timed);
-#undef HIPR_WALK_K
-        if (lr != HIPR_SUCCESS) return lr;
-      }
-      for (int k = 1; k < 3; k++) {
-        if (!used[k]) continue;
-        HIP_TRY(hipEventRecord(joins[k], streams[k]));
-        HIP_TRY(hipStreamWaitEvent(st, joins[k], 0));
-      }
-      return HIPR_SUCCESS;
-    };
-    if (!use_graph) return launches();
-    HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
-    rr = launches();
-    hipGraph_t g = nullptr;
-    hipError_t ce = hipStreamEndCapture(st, &g);
-    if (g) ctx->graphs.push_back(g);
-    if (rr != HIPR_SUCCESS) return rr;
-    HIP_TRY(ce);
-    hipGraphExec_t ge = nullptr;
-    HIP_TRY(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0));
-    ctx->graph_execs.push_back(ge);
+      if (cnt[i]) used[stream_of(i)] = true;
+    // each kernel timed by itself, or the plan as one (a pass that writes
+    // planes counts as the walk)
+    const bool timed = (run_flags & HIPR_FLAG_NO_GRAPH) != 0;
     int stage = HIPR_STAGE_WALK;
-    for (const WalkLaunch& l : plan)
+    bool any_write = false;
+    for (const WalkLaunch& l : plan) {
+      any_write |= l.kmode == kWalkWrite;
       if (l.kmode != kWalkWrite)
         stage = l.kmode == kWalkCount ? HIPR_STAGE_WALK_COUNT : HIPR_STAGE_WALK_SCHEDULE;
-    bool any_write = false;
-    for (const WalkLaunch& l : plan) any_write |= l.kmode == kWalkWrite;
-    if (any_write) stage = HIPR_STAGE_WALK;  // a pass that writes planes counts as the walk
-    hipEvent_t b = StageBegin(ctx, st);
-    HIP_TRY(hipGraphLaunch(ge, st));
-    StageEnd(ctx, stage, b, st);
+    }
+    if (any_write) stage = HIPR_STAGE_WALK;
+    hipEvent_t whole = timed ? nullptr : StageBegin(ctx, st);
+    if (q) hipLaunchKernelGGL(FillKernel, dim3(1), dim3(kWave), 0, st, q, (int64_t)plan.size(), 0);
+    bool forked = false;
+    for (int k = 1; k <= kSideStreams; k++) {
+      if (!used[k]) continue;
+      if (!forked) HIP_TRY(hipEventRecord(ctx->ev_fork, st));
+      forked = true;
+      HIP_TRY(hipStreamWaitEvent(ctx->side[k - 1], ctx->ev_fork, 0));
+    }
+    for (size_t i = 0; i < plan.size(); i++) {
+      if (!cnt[i]) continue;
+      const WalkLaunch& l = plan[i];
+      WalkParams wpl = wp;
+      wpl.walk_list = ctx->sub_list.as<int32_t>() + off[i];
+      wpl.n_walk = (int32_t)cnt[i];
+      wpl.cov = l.kmode == kWalkWrite ? ctx->wcov.as<JobCov>() : ctx->cov.as<JobCov>();
+      int32_t* qi = q ? q + i : nullptr;
+      double share = work_all > 0 ? work[i] / work_all : 1.0;
+      const int sk = stream_of(i);
+      hipStream_t ls = sk == 0 ? st : ctx->side[sk - 1];
+      hipr_result lr;
+      lr = l.K <= kMaxTeam ? LaunchTier(ctx, l.K, l.kmode, wpl, ls, timed, qi, share)
+                           : LaunchWalkWide(ctx, l.K, l.kmode, wpl, ls, timed);
+      if (lr != HIPR_SUCCESS) return lr;
+    }
+    for (int k = 1; k <= kSideStreams; k++) {
+      if (!used[k]) continue;
+      HIP_TRY(hipEventRecord(ctx->ev_join[k - 1], ctx->side[k - 1]));
+      HIP_TRY(hipStreamWaitEvent(st, ctx->ev_join[k - 1], 0));
+    }
+    if (whole) StageEnd(ctx, stage, whole, st);
     return HIPR_SUCCESS;
   };
-  // One walk pass of one mode: the 4-slot jobs on the main stream, the 8-
-  // and 16-slot jobs on a side stream.
+  constexpr int kTiers[] = {64, 32, 16, 8, 4, 2, 1};
+  // Streams: the device runs four hardware queues of this process at once, so
+  // a plan's kernel chains go to four streams, the longest first, each to the
+  // stream with the least before it.  A chain's length is its longest walk,
+  // in rows, a wider list counting more.
+  auto place_chains = [&](std::vector<std::vector<WalkLaunch>> chains) {
+    std::vector<std::pair<double, size_t>> order;
+    for (size_t i = 0; i < chains.size(); i++) {
+      double len = 0;
+      for (int32_t j : chains[i][0].jobs) {
+        const PixBounds pb = JobScanBounds(ctx->h_geo[j]);
+        len = std::max(len, (double)(pb.b - pb.t) * (4 + chains[i][0].K));
+      }
+      order.push_back({-len, i});
+    }
+    std::stable_sort(order.begin(), order.end());
+    double load[kSideStreams + 1] = {};
+    std::vector<WalkLaunch> plan;
+    for (auto& o : order) {
+      int best = 0;
+      for (int k = 1; k <= kSideStreams; k++)
+        if (load[k] < load[best]) best = k;
+      load[best] -= o.first - 1;
+      for (WalkLaunch& l : chains[o.second]) {
+        l.stream = best;
+        plan.push_back(std::move(l));
+      }
+    }
+    return plan;
+  };
+  // One walk pass of one mode, every tier on a stream of its own.
   auto walk_pass = [&](int kmode, const std::vector<int32_t>& sm,
                        const std::vector<int32_t>& wd) -> hipr_result {
-    std::vector<int32_t> j8, j16, j32, j64;
-    for (int32_t j : wd)
-      (tier[j] <= 8 ? j8 : tier[j] == 16 ? j16 : tier[j] == 32 ? j32 : j64).push_back(j);
-    return run_plan({{kmode, 64, 2, j64},
-                     {kmode, 32, 2, j32},
-                     {kmode, 8, 1, j8},
-                     {kmode, 16, 1, j16},
-                     {kmode, 4, 0, sm}});
+    std::vector<std::vector<WalkLaunch>> chains;
+    for (int k : kTiers) {
+      std::vector<int32_t> js;
+      for (int32_t j : wd)
+        if (tier[j] == k) js.push_back(j);
+      for (int32_t j : sm)
+        if (tier[j] == k) js.push_back(j);
+      if (!js.empty()) chains.push_back({{kmode, k, 0, std::move(js)}});
+    }
+    return run_plan(place_chains(std::move(chains)));
   };
-  // A 4-slot job whose list still outgrew 256 edges (flag 2) is counted again
-  // by the 16-slot walk (recording its snapshots there); the bound makes this
-  // a safety net.  `from` holds the flags of the pass that overflowed.
+  // A job of up to four waves whose list still outgrew them (flag 2) is
+  // counted again by a team of 16 (recording its snapshots there); the bound
+  // makes this a safety net.  `from` holds the flags of the pass that overflowed.
   auto move_overflowed = [&](const JobCov* from, std::vector<int32_t>* moved_out) -> hipr_result {
     std::vector<int32_t> moved, keep;
     for (int32_t j : small) (from[j].flags & 2 ? moved : keep).push_back(j);
@@ -2037,31 +2093,34 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
     if ((r = walk_pass(kWalkWrite, small, wide)) != HIPR_SUCCESS) return r;
   } else {
     // The banded (longest) walks need a schedule pass before their write
-    // pass; both run on side streams while the main stream writes the other
-    // jobs, so the schedule pass overlaps the bulk of the writing.
-    std::vector<int32_t> b4, u4, b8, u8, b16, u16, u32, u64;
-    for (int32_t j : small) (nbands[j] > 1 ? b4 : u4).push_back(j);
-    for (int32_t j : wide) {
-      if (tier[j] <= 8) {
-        (nbands[j] > 1 ? b8 : u8).push_back(j);
-      } else if (tier[j] == 16) {
-        (nbands[j] > 1 ? b16 : u16).push_back(j);
-      } else {
-        (tier[j] == 32 ? u32 : u64).push_back(j);
+    // pass; both run on side streams while the other jobs are written.
+    // Unbanded jobs of up to 256 edges that fill the device more than once go
+    // into one launch of 4-slot walks, the longest first: kernels of their own
+    // would run their short jobs beside each other's long ones and end later
+    // (curves + strokes, 4,096 paths: 104 ms in three launches, 89 ms in one).
+    std::vector<std::vector<WalkLaunch>> chains;
+    int64_t plain_small = 0;
+    bool mixed = false;
+    for (int32_t j : small)
+      if (nbands[j] == 1) {
+        plain_small++;
+        mixed |= tier[j] > 1;
       }
+    const bool merge = mixed && plain_small > kBandSlots;
+    for (int k : kTiers) {
+      std::vector<int32_t> banded, plain;
+      for (int32_t j : all) {
+        if (nbands[j] > 1) {
+          if (tier[j] == k) banded.push_back(j);
+        } else if ((merge && tier[j] <= 4 ? 4 : tier[j]) == k) {
+          plain.push_back(j);
+        }
+      }
+      if (!banded.empty())
+        chains.push_back({{kWalkSchedule, k, 0, banded}, {kWalkWrite, k, 0, banded}});
+      if (!plain.empty()) chains.push_back({{kWalkWrite, k, 0, std::move(plain)}});
     }
-    if ((r = run_plan({{kWalkWrite, 64, 1, u64},
-                       {kWalkWrite, 32, 1, u32},
-                       {kWalkSchedule, 8, 2, b8},
-                       {kWalkWrite, 8, 2, b8},
-                       {kWalkSchedule, 16, 2, b16},
-                       {kWalkWrite, 16, 2, b16},
-                       {kWalkWrite, 8, 2, u8},
-                       {kWalkWrite, 16, 2, u16},
-                       {kWalkSchedule, 4, 1, b4},
-                       {kWalkWrite, 4, 1, b4},
-                       {kWalkWrite, 4, 0, u4}})) != HIPR_SUCCESS)
-      return r;
+    if ((r = run_plan(place_chains(std::move(chains)))) != HIPR_SUCCESS) return r;
   }
   if ((r = read_cov(&ctx->wcov, hw)) != HIPR_SUCCESS) return r;
   if (counted) {
@@ -2757,13 +2816,17 @@ HIPR_API hipr_result hipr_context_create(int32_t device, hipr_context* out) {
       hipDeviceGetAttribute(&ctx->max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) !=
           hipSuccess ||
       hipStreamCreate(&ctx->stream) != hipSuccess ||
-      hipStreamCreate(&ctx->side) != hipSuccess || hipStreamCreate(&ctx->side2) != hipSuccess ||
       hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&ctx->ev_join2, hipEventDisableTiming) != hipSuccess ||
       hipEventCreate(&ctx->ev0) != hipSuccess || hipEventCreate(&ctx->ev1) != hipSuccess) {
     delete ctx;
     return HIPR_ERROR_INITIALIZATION_FAILED;
+  }
+  for (int k = 0; k < kSideStreams; k++) {
+    if (hipStreamCreate(&ctx->side[k]) != hipSuccess ||
+        hipEventCreateWithFlags(&ctx->ev_join[k], hipEventDisableTiming) != hipSuccess) {
+      delete ctx;
+      return HIPR_ERROR_INITIALIZATION_FAILED;
+    }
   }
   // The sRGB tables of SRGBGammaColorFilter (color_filter.cc:128-166) from
   // their definition: floor(255 f(i / 255)) with f the sRGB encoding
@@ -2810,7 +2873,6 @@ static void FreeContext(hipr_context ctx) {
                     &ctx->qstate, &ctx->q_base, &ctx->snaps, &ctx->snap_base,
                     &ctx->band_count, &ctx->queues, &ctx->flatten_redo, &ctx->pool_ctr, &ctx->stroke_redo,
                     &ctx->stroke_redo_out, &ctx->blur_raw, &ctx->blur_styles};
-  ReleaseGraphs(ctx);
   for (DevBuf* b : bufs) b->Free();
   DevBuf* mlp[] = {&ctx->mlp_prm, &ctx->mlp_ops, &ctx->mlp_feats, &ctx->mlp_preds,
                    &ctx->mlp_targets, &ctx->mlp_grads, &ctx->mlp_loss, &ctx->mlp_m,
@@ -2821,15 +2883,14 @@ static void FreeContext(hipr_context ctx) {
   if (ctx->h_wcov) (void)hipHostFree(ctx->h_wcov);
   if (ctx->h_so) (void)hipHostFree(ctx->h_so);
   for (hipEvent_t e : ctx->ev_pool) (void)hipEventDestroy(e);
-  (void)hipStreamSynchronize(ctx->side);
   (void)hipEventDestroy(ctx->ev0);
   (void)hipEventDestroy(ctx->ev1);
   (void)hipEventDestroy(ctx->ev_fork);
-  (void)hipEventDestroy(ctx->ev_join);
-  (void)hipEventDestroy(ctx->ev_join2);
-  (void)hipStreamSynchronize(ctx->side2);
-  (void)hipStreamDestroy(ctx->side);
-  (void)hipStreamDestroy(ctx->side2);
+  for (int k = 0; k < kSideStreams; k++) {
+    (void)hipStreamSynchronize(ctx->side[k]);
+    (void)hipStreamDestroy(ctx->side[k]);
+    (void)hipEventDestroy(ctx->ev_join[k]);
+  }
   (void)hipStreamDestroy(ctx->stream);
   delete ctx;
 }
