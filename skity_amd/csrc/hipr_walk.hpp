@@ -1701,6 +1701,31 @@ __global__ void FillKernel(int32_t* __restrict__ p, int64_t n, int32_t v) {
     p[i] = v;
 }
 
+// Before the write pass: both tile maps at kNoTile, the coverage records, the
+// plane pool's counter and the composite's counters at zero.  One launch (four
+// fills and a memset were 20 us of a small frame); bound by the maps' bytes,
+// which go out 16 per lane (the maps begin at an allocation).
+__global__ void PrepareWriteKernel(int32_t* __restrict__ map0, int32_t* __restrict__ map1,
+                                   int64_t n_map, int32_t* __restrict__ cov, int64_t n_cov,
+                                   int32_t* __restrict__ pool_ctr,
+                                   unsigned long long* __restrict__ counters) {
+  const int64_t first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t step = (int64_t)gridDim.x * blockDim.x;
+  const int64_t n4 = n_map / 4;
+  const int4 none = make_int4(kNoTile, kNoTile, kNoTile, kNoTile);
+  for (int64_t i = first; i < n4; i += step) {
+    ((int4*)map0)[i] = none;
+    ((int4*)map1)[i] = none;
+  }
+  if (first < n_map - 4 * n4) {
+    map0[4 * n4 + first] = kNoTile;
+    map1[4 * n4 + first] = kNoTile;
+  }
+  for (int64_t i = first; i < n_cov; i += step) cov[i] = 0;
+  if (first == 0) *pool_ctr = 0;
+  if (first < 2) counters[first] = 0;
+}
+
 // Zeroes the coverage records of the listed jobs (before a write pass redoes
 // them).
 __global__ void ResetCovKernel(const int32_t* __restrict__ list, int n, JobCov* __restrict__ cov) {

@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <memory>
 #include <cmath>
@@ -319,9 +320,10 @@ struct hipr_context_s {
   // per-draw device buffers (grow-only)
   DevBuf canvases, layer_canvases, geo, cov, edge_base, edge_cap, edges, wedges, gkeys;
   DevBuf job_tiles;  // per-job tile ranges for the composite
-  DevBuf plane_base, plane_cap, planes, map_base, map0, map1, sub_list, big_list, bound,
+  DevBuf planes, map0, map1, sub_list, big_list, bound,
       gather_list;
-  DevBuf wcov, qstate, q_base, snaps, snap_base, band_count;  // write-pass coverage, row bands
+  DevBuf wcov, qstate, snaps;  // write-pass coverage, row bands
+  DevBuf tables;                          // per-job offsets of the walk (JobTables)
   DevBuf queues;                          // persistent walk: item counters
   DevBuf srgb;                            // sRGB colour-filter tables (512 bytes)
   DevBuf flatten_redo;                    // jobs whose edges outgrew their estimate
@@ -354,6 +356,10 @@ struct hipr_context_s {
   JobCov* h_cov = nullptr;
   JobCov* h_wcov = nullptr;
   StrokeOut* h_so = nullptr;
+  int32_t* h_bound = nullptr;
+  float* h_pred = nullptr;
+  uint8_t* h_tables = nullptr;
+  unsigned long long* h_counts = nullptr;  // composite counters: blends, pixels
   size_t h_cap = 0;
   uint64_t draw_serial = 0;  // pipeline runs so far (see hipr_surface_s)
 };
@@ -481,21 +487,47 @@ hipr_result LaunchBlurMfma(hipr_context ctx, const std::vector<BlurJob>& rows,
                            const std::vector<BlurJob>& cols, DevBuf* d_rows, DevBuf* d_cols,
                            hipStream_t st, bool timed);
 
+// Per-job offsets of the walk's buffers, one block of n entries each, so that
+// a draw uploads them with one copy (six copies of a few bytes took about 25 us
+// of a 500 us frame).
+struct JobTables {
+  static constexpr size_t kBytes = 4 * sizeof(int64_t) + 2 * sizeof(int32_t);
+  int64_t *map_base, *plane_base, *q_base, *snap_base;
+  int32_t *plane_cap, *band_count;
+  JobTables(void* p, size_t n) {
+    map_base = (int64_t*)p;
+    plane_base = map_base + n;
+    q_base = plane_base + n;
+    snap_base = q_base + n;
+    plane_cap = (int32_t*)(snap_base + n);
+    band_count = plane_cap + n;
+  }
+};
+
+void FreeHostStage(hipr_context ctx) {
+  void** bufs[] = {(void**)&ctx->h_geo,  (void**)&ctx->h_cov,    (void**)&ctx->h_wcov,
+                   (void**)&ctx->h_so,   (void**)&ctx->h_bound,  (void**)&ctx->h_pred,
+                   (void**)&ctx->h_tables, (void**)&ctx->h_counts};
+  for (void** b : bufs) {
+    if (*b) (void)hipHostFree(*b);
+    *b = nullptr;
+  }
+  ctx->h_cap = 0;
+}
+
+// Pinned staging for at least n jobs.
 hipr_result HostStage(hipr_context ctx, size_t n) {
   if (n > ctx->h_cap) {
-    if (ctx->h_geo) (void)hipHostFree(ctx->h_geo);
-    if (ctx->h_cov) (void)hipHostFree(ctx->h_cov);
-    if (ctx->h_wcov) (void)hipHostFree(ctx->h_wcov);
-    if (ctx->h_so) (void)hipHostFree(ctx->h_so);
-    ctx->h_geo = nullptr;
-    ctx->h_cov = nullptr;
-    ctx->h_wcov = nullptr;
-    ctx->h_so = nullptr;
+    FreeHostStage(ctx);
     size_t want = n + n / 2 + 64;
     HIP_TRY(hipHostMalloc((void**)&ctx->h_geo, want * sizeof(JobGeo)));
     HIP_TRY(hipHostMalloc((void**)&ctx->h_cov, want * sizeof(JobCov)));
     HIP_TRY(hipHostMalloc((void**)&ctx->h_wcov, want * sizeof(JobCov)));
     HIP_TRY(hipHostMalloc((void**)&ctx->h_so, want * sizeof(StrokeOut)));
+    HIP_TRY(hipHostMalloc((void**)&ctx->h_bound, want * sizeof(int32_t)));
+    HIP_TRY(hipHostMalloc((void**)&ctx->h_pred, want * kMlpOut * sizeof(float)));
+    HIP_TRY(hipHostMalloc((void**)&ctx->h_tables, want * JobTables::kBytes));
+    HIP_TRY(hipHostMalloc((void**)&ctx->h_counts, 2 * sizeof(unsigned long long)));
     ctx->h_cap = want;
   }
   return HIPR_SUCCESS;
@@ -1525,14 +1557,18 @@ hipr_result RunPresize(Frame& f, std::vector<int32_t>* eest, std::vector<int32_t
                      ctx->mlp_preds.as<float>());
   HIP_TRY(hipGetLastError());
   StageEnd(ctx, HIPR_STAGE_PRESIZE, b);
-  std::vector<float> pred((size_t)kMlpOut * nj);
-  HIP_TRY(hipMemcpyAsync(pred.data(), ctx->mlp_preds.p, sizeof(float) * pred.size(),
+  const float* pred = ctx->h_pred;
+  HIP_TRY(hipMemcpyAsync(ctx->h_pred, ctx->mlp_preds.p, sizeof(float) * kMlpOut * nj,
                          hipMemcpyDeviceToHost, f.st));
   HIP_TRY(hipStreamSynchronize(f.st));
   eest->resize(nj);
   test->resize(nj);
   auto cap = [](float p, float m) {
-    double v = std::ceil(std::expm1((double)p + m));
+    // ceil(expm1(x)); exp is cheaper, and where exp(x) - 1 is farther from a
+    // whole number than its rounding error its ceiling is the same
+    const double x = (double)p + m, e = std::exp(x) - 1.0;
+    double v = std::ceil(e);
+    if (!(std::fabs(e - std::round(e)) > 1e-12 * (std::fabs(e) + 1.0))) v = std::ceil(std::expm1(x));
     return (int32_t)std::min(std::max(v, 1.0), 1.0e9);
   };
   for (int j = 0; j < nj; j++) {
@@ -1620,9 +1656,7 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
       ctx->cov.Ensure(sizeof(JobCov) * nj) != hipSuccess ||
       ctx->edge_base.Ensure(sizeof(int64_t) * nj) != hipSuccess ||
       ctx->edge_cap.Ensure(sizeof(int32_t) * nj) != hipSuccess ||
-      ctx->plane_base.Ensure(sizeof(int64_t) * nj) != hipSuccess ||
-      ctx->plane_cap.Ensure(sizeof(int32_t) * nj) != hipSuccess ||
-      ctx->map_base.Ensure(sizeof(int64_t) * nj) != hipSuccess)
+      ctx->tables.Ensure(JobTables::kBytes * nj) != hipSuccess)
     return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
   // ---- stage (a): stroke outlines, flatten, sort ----
   if ((r = RunStrokes(f, mode != HIPR_MODE_EXACT)) != HIPR_SUCCESS) return r;
@@ -1649,11 +1683,17 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   std::vector<int64_t> ebase;
   std::vector<int32_t> ecap;
   if ((r = Flatten(f, mode, eest.data(), &ebase, &ecap)) != HIPR_SUCCESS) return r;
-  if (mode == 0) {
-    // (the count pass read the bounds back already)
-  }
   int lds_width = 256;
-  std::vector<int64_t> mbase(nj + 1, 0);
+  // the per-job tables of the walk, on the host (pinned) and on the device
+  const JobTables ht(ctx->h_tables, nj), dt(ctx->tables.p, nj);
+  // each job's scan bounds and tiles, found once for all that follows
+  struct Span {
+    PixBounds pb;
+    TileRange tr;
+    int rows() const { return pb.empty ? 0 : pb.b - pb.t; }
+  };
+  std::vector<Span> spans(nj);
+  int64_t total_map = 0;
   for (int j = 0; j < nj; j++) {
     int64_t msz = 0;
     if (f.jobs[j].kind != kJobRect) {
@@ -1667,24 +1707,23 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
                      f.jobs[j].path);
         return HIPR_ERROR_NOT_SUPPORTED;
       }
-      PixBounds pb = JobScanBounds(g);
+      const PixBounds pb = JobScanBounds(g);
       const Canvas& cv = f.canvases[f.jobs[j].canvas];
-      TileRange tr = JobTiles(pb, cv.width, cv.height);
+      const TileRange tr = JobTiles(pb, cv.width, cv.height);
+      spans[j] = Span{pb, tr};
       // the walk's row holds the job's visible columns only
       if (tr.ntc > 0)
         lds_width = std::max(lds_width, std::min(pb.r, cv.width) - std::max(pb.l, 0));
       msz = (int64_t)tr.ntc * tr.ntr;
     }
-    mbase[j + 1] = mbase[j] + msz;
+    ht.map_base[j] = total_map;
+    total_map += msz;
   }
   lds_width = (lds_width + 255) & ~255;
   if (lds_width > kMaxCanvasSide) return HIPR_ERROR_CAPACITY;  // a layer wider than a canvas
-  int64_t total_map = mbase[nj];
   if (ctx->map0.Ensure(sizeof(int32_t) * std::max<int64_t>(total_map, 1)) != hipSuccess ||
       ctx->map1.Ensure(sizeof(int32_t) * std::max<int64_t>(total_map, 1)) != hipSuccess)
     return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
-  HIP_TRY(hipMemcpyAsync(ctx->map_base.p, mbase.data(), sizeof(int64_t) * nj,
-                         hipMemcpyHostToDevice, st));
   int nwalk = (int)pl->walk_jobs.size();
   if (ctx->bound.Ensure(sizeof(int32_t) * std::max(nj, 1)) != hipSuccess)
     return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
@@ -1702,7 +1741,7 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   wp.cov = ctx->cov.as<JobCov>();
   wp.lds_width = lds_width;
   wp.row_ints = WalkRowCapacity(ctx, lds_width, nwalk);
-  wp.map_base = ctx->map_base.as<int64_t>();
+  wp.map_base = dt.map_base;
   // ---- stage (b): walk ----
   // The walk keeps the active edge list in registers, one element per lane.
   // The sort bounded each job's list by its largest row overlap: a job takes
@@ -1710,17 +1749,15 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   // the rare list of more than 1,024 edges the unbanded 32- or 64-slot walk of
   // one wave (2,048 and 4,096 edges).  A longer list is refused
   // (HIPR_ERROR_CAPACITY).
-  std::vector<int32_t> bound(nj, 0);
-  HIP_TRY(hipMemcpyAsync(bound.data(), ctx->bound.p, sizeof(int32_t) * nj, hipMemcpyDeviceToHost,
+  const int32_t* bound = ctx->h_bound;  // of the walked jobs
+  HIP_TRY(hipMemcpyAsync(ctx->h_bound, ctx->bound.p, sizeof(int32_t) * nj, hipMemcpyDeviceToHost,
                          st));
   HIP_TRY(hipStreamSynchronize(st));
   const std::vector<int32_t>& all = pl->walk_jobs;
   // Planes a job can use at most: two per visible tile, a keep-zero job three
   // (every tile row belongs to one band).
   auto most_planes = [&](int32_t j) -> int64_t {
-    const Canvas& cv = f.canvases[f.jobs[j].canvas];
-    const TileRange tr = JobTiles(JobScanBounds(ctx->h_geo[j]), cv.width, cv.height);
-    return (int64_t)tr.ntc * tr.ntr * ((f.jobs[j].flags & kJobKeepZero) ? 3 : 2);
+    return (int64_t)spans[j].tr.ntc * spans[j].tr.ntr * ((f.jobs[j].flags & kJobKeepZero) ? 3 : 2);
   };
   // Exact form, uncounted: where the planes every job could use fit a bounded
   // buffer, they are reserved (a plane that is not used is not touched) and
@@ -1765,69 +1802,62 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   int band_min_rows = 0;
   if (!counted && !own_split) {
     int64_t total_rows = 0;
-    for (int32_t j : all) {
-      const PixBounds b = JobScanBounds(ctx->h_geo[j]);
-      if (!b.empty) total_rows += b.b - b.t;
-    }
+    for (int32_t j : all) total_rows += spans[j].rows();
     band_min_rows = (int)std::min<int64_t>(
         std::max<int64_t>(kBandMinRows, total_rows / kBandSlots), INT32_MAX);
   }
-  std::vector<int32_t> nbands(nj, 1);
-  std::vector<int64_t> qb(nj, 0), sb(nj, 0);
+  int32_t *const nbands = ht.band_count, *const pcap = ht.plane_cap;
+  std::fill_n(nbands, nj, 1);
+  std::fill_n(pcap, nj, 0);
+  std::fill_n(ht.plane_base, nj, 0);
+  std::fill_n(ht.q_base, nj, 0);
+  std::fill_n(ht.snap_base, nj, 0);
   int64_t q_total = 0, snap_total = 0;
   for (int32_t j : all) {
     // the 32- and 64-slot walks are unbanded
-    const PixBounds sb_j = JobScanBounds(ctx->h_geo[j]);
     // a tall path is a long sequential walk too, whatever its list width
-    const bool tall = band_min_rows > 0 && !sb_j.empty && sb_j.b - sb_j.t >= band_min_rows;
-    nbands[j] = (bound[j] >= band_min || tall) && tier[j] <= 16 ? BandCount(sb_j, band_rows) : 1;
-    qb[j] = q_total;
+    const bool tall = band_min_rows > 0 && spans[j].rows() >= band_min_rows;
+    nbands[j] = (bound[j] >= band_min || tall) && tier[j] <= 16
+                    ? BandCount(spans[j].pb, band_rows)
+                    : 1;
+    ht.q_base[j] = q_total;
     q_total += (int64_t)nbands[j] * ctx->h_geo[j].edges;
   }
   auto assign_snaps = [&](const std::vector<int32_t>& js) {
     for (int32_t j : js) {
-      sb[j] = snap_total;
+      ht.snap_base[j] = snap_total;
       snap_total += (int64_t)(nbands[j] - 1) * SnapStride(tier[j] * kWave);
     }
   };
   assign_snaps(all);
   if (ctx->qstate.Ensure(sizeof(EdgeRec) * std::max<int64_t>(q_total, 1)) != hipSuccess ||
-      ctx->q_base.Ensure(sizeof(int64_t) * nj) != hipSuccess ||
-      ctx->snap_base.Ensure(sizeof(int64_t) * nj) != hipSuccess ||
-      ctx->band_count.Ensure(sizeof(int32_t) * nj) != hipSuccess ||
       ctx->snaps.Ensure(std::max<int64_t>(snap_total, 1)) != hipSuccess ||
       ctx->wcov.Ensure(sizeof(JobCov) * nj) != hipSuccess)
     return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
-  HIP_TRY(hipMemcpyAsync(ctx->q_base.p, qb.data(), sizeof(int64_t) * nj, hipMemcpyHostToDevice,
-                         st));
-  HIP_TRY(hipMemcpyAsync(ctx->snap_base.p, sb.data(), sizeof(int64_t) * nj,
-                         hipMemcpyHostToDevice, st));
   wp.qstate = ctx->qstate.as<EdgeRec>();
-  wp.q_base = ctx->q_base.as<int64_t>();
+  wp.q_base = dt.q_base;
   wp.snaps = ctx->snaps.as<uint8_t>();
-  wp.snap_base = ctx->snap_base.as<int64_t>();
-  HIP_TRY(hipMemcpyAsync(ctx->band_count.p, nbands.data(), sizeof(int32_t) * nj,
-                         hipMemcpyHostToDevice, st));
-  wp.band_count = ctx->band_count.as<int32_t>();
-  std::vector<int64_t> pbase(nj, 0);
-  std::vector<int32_t> pcap(nj, 0);
+  wp.snap_base = dt.snap_base;
+  wp.band_count = dt.band_count;
+  // The tables are written again only after the stream has been waited for.
+  auto upload_tables = [&]() -> hipr_result {
+    HIP_TRY(hipMemcpyAsync(ctx->tables.p, ctx->h_tables, JobTables::kBytes * nj,
+                           hipMemcpyHostToDevice, st));
+    return HIPR_SUCCESS;
+  };
   int64_t plane_total = 0;
   auto upload_planes = [&]() -> hipr_result {
     if (plane_total >= kNoPlane) return HIPR_ERROR_CAPACITY;  // plane numbers are int32
     if (ctx->planes.EnsureKeep((size_t)kTilePlaneBytes * std::max<int64_t>(plane_total, 1),
                                ctx->planes.cap, st) != hipSuccess)
       return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
-    HIP_TRY(hipMemcpyAsync(ctx->plane_base.p, pbase.data(), sizeof(int64_t) * nj,
-                           hipMemcpyHostToDevice, st));
-    HIP_TRY(hipMemcpyAsync(ctx->plane_cap.p, pcap.data(), sizeof(int32_t) * nj,
-                           hipMemcpyHostToDevice, st));
-    return HIPR_SUCCESS;
+    return upload_tables();
   };
   auto assign_planes = [&](const std::vector<int32_t>& js) {
     for (int32_t j : js) {
       // the last chunk of each band may be left over in part
       if (nbands[j] > 1) pcap[j] += nbands[j] * kPlaneChunk;
-      pbase[j] = plane_total;
+      ht.plane_base[j] = plane_total;
       plane_total += pcap[j];
     }
   };
@@ -1849,22 +1879,28 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   };
   // Work items of a pass: one per job (count, schedule) or one per row band
   // (write), the bands of the longest walks first so they start first.
-  auto make_items = [&](const std::vector<int32_t>& js, int kmode) {
-    std::vector<int32_t> it;
+  // (a job's work rounded down to an eighth of a power of two is order enough,
+  // and 512 buckets are filled faster than the jobs are sorted)
+  auto make_items = [&](const std::vector<int32_t>& js, int kmode, std::vector<int32_t>* items) {
     if (kmode != kWalkWrite) {
-      for (int32_t j : js) it.push_back(j << kBandBits);
-      return it;
+      for (int32_t j : js) items->push_back(j << kBandBits);
+      return;
     }
-    std::vector<std::pair<int64_t, int32_t>> order;
+    auto bucket = [&](int32_t j) {
+      const uint64_t work =
+          (uint64_t)std::max(bound[j], 1) * std::max(spans[j].rows(), 1) / nbands[j] + 8;
+      const int e = 63 - __builtin_clzll(work);
+      return 511 - (e * 8 + (int)((work >> (e - 3)) & 7));
+    };
+    std::array<int32_t, 513> at{};
+    for (int32_t j : js) at[bucket(j) + 1] += nbands[j];
+    for (int k = 0; k < 512; k++) at[k + 1] += at[k];
+    const size_t begin = items->size();
+    items->resize(begin + at[512]);
     for (int32_t j : js) {
-      PixBounds pb = JobScanBounds(ctx->h_geo[j]);
-      int64_t work = (int64_t)std::max(bound[j], 1) * std::max(pb.b - pb.t, 1) / nbands[j];
-      order.push_back({-work, j});
+      int32_t& p = at[bucket(j)];
+      for (int b = 0; b < nbands[j]; b++) (*items)[begin + p++] = (j << kBandBits) | b;
     }
-    std::stable_sort(order.begin(), order.end());
-    for (auto& o : order)
-      for (int b = 0; b < nbands[o.second]; b++) it.push_back((o.second << kBandBits) | b);
-    return it;
   };
   const int run_flags = opt ? opt->flags : 0;
   const bool persistent = (run_flags & HIPR_FLAG_PERSISTENT) != 0;
@@ -1876,7 +1912,7 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   // of one kernel and 100 us more for one of two streams.)
   struct WalkLaunch {
     int kmode, K, stream;
-    std::vector<int32_t> jobs;
+    const std::vector<int32_t>* jobs;  // (lives until the plan has been launched)
   };
   auto run_plan = [&](const std::vector<WalkLaunch>& plan) -> hipr_result {
     hipr_result rr;
@@ -1885,16 +1921,13 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
     std::vector<double> work;
     double work_all = 0;
     for (const WalkLaunch& l : plan) {
-      std::vector<int32_t> it = make_items(l.jobs, l.kmode);
       off.push_back(all_items.size());
-      cnt.push_back(it.size());
-      all_items.insert(all_items.end(), it.begin(), it.end());
+      make_items(*l.jobs, l.kmode, &all_items);
+      cnt.push_back(all_items.size() - off.back());
       double w = 0;
       if (persistent) {
-        for (int32_t j : l.jobs) {
-          PixBounds pb = JobScanBounds(ctx->h_geo[j]);
-          w += (double)std::max(bound[j], 1) * std::max(pb.b - pb.t, 1);
-        }
+        for (int32_t j : *l.jobs)
+          w += (double)std::max(bound[j], 1) * std::max(spans[j].rows(), 1);
       }
       work.push_back(w);
       work_all += w;
@@ -1959,7 +1992,8 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
     if (whole) StageEnd(ctx, stage, whole, st);
     return HIPR_SUCCESS;
   };
-  constexpr int kTiers[] = {64, 32, 16, 8, 4, 2, 1};
+  constexpr int kTierCount = 7;  // 1, 2, 4, .. 64 waves (slots)
+  auto tier_index = [](int k) { return __builtin_ctz((unsigned)k); };
   // Streams: the device runs four hardware queues of this process at once, so
   // a plan's kernel chains go to four streams, the longest first, each to the
   // stream with the least before it.  A chain's length is its longest walk,
@@ -1968,10 +2002,8 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
     std::vector<std::pair<double, size_t>> order;
     for (size_t i = 0; i < chains.size(); i++) {
       double len = 0;
-      for (int32_t j : chains[i][0].jobs) {
-        const PixBounds pb = JobScanBounds(ctx->h_geo[j]);
-        len = std::max(len, (double)(pb.b - pb.t) * (4 + chains[i][0].K));
-      }
+      for (int32_t j : *chains[i][0].jobs)
+        len = std::max(len, (double)spans[j].rows() * (4 + chains[i][0].K));
       order.push_back({-len, i});
     }
     std::stable_sort(order.begin(), order.end());
@@ -1984,7 +2016,7 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
       load[best] -= o.first - 1;
       for (WalkLaunch& l : chains[o.second]) {
         l.stream = best;
-        plan.push_back(std::move(l));
+        plan.push_back(l);
       }
     }
     return plan;
@@ -1993,14 +2025,11 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   auto walk_pass = [&](int kmode, const std::vector<int32_t>& sm,
                        const std::vector<int32_t>& wd) -> hipr_result {
     std::vector<std::vector<WalkLaunch>> chains;
-    for (int k : kTiers) {
-      std::vector<int32_t> js;
-      for (int32_t j : wd)
-        if (tier[j] == k) js.push_back(j);
-      for (int32_t j : sm)
-        if (tier[j] == k) js.push_back(j);
-      if (!js.empty()) chains.push_back({{kmode, k, 0, std::move(js)}});
-    }
+    std::vector<int32_t> js[kTierCount];
+    for (int32_t j : wd) js[tier_index(tier[j])].push_back(j);
+    for (int32_t j : sm) js[tier_index(tier[j])].push_back(j);
+    for (int i = kTierCount - 1; i >= 0; i--)
+      if (!js[i].empty()) chains.push_back({{kmode, 1 << i, 0, &js[i]}});
     return run_plan(place_chains(std::move(chains)));
   };
   // A job of up to four waves whose list still outgrew them (flag 2) is
@@ -2017,9 +2046,8 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
         hipSuccess)
       return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
     wp.snaps = ctx->snaps.as<uint8_t>();
-    HIP_TRY(hipMemcpyAsync(ctx->snap_base.p, sb.data(), sizeof(int64_t) * nj,
-                           hipMemcpyHostToDevice, st));
     hipr_result rr;
+    if ((rr = upload_tables()) != HIPR_SUCCESS) return rr;
     if ((rr = walk_pass(kWalkCount, {}, moved)) != HIPR_SUCCESS) return rr;
     if ((rr = read_cov(&ctx->cov, ctx->h_cov)) != HIPR_SUCCESS) return rr;
     if ((rr = limit_error(ctx->h_cov, moved, 2 | 16 | 32)) != HIPR_SUCCESS) return rr;
@@ -2027,18 +2055,14 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
     if (moved_out) *moved_out = moved;
     return HIPR_SUCCESS;
   };
-  // Before a write pass over `js`: maps at -1 (all jobs) and the jobs'
-  // write-pass coverage records at zero.
+  // Before a write pass over `js`: maps at -1 and counters at zero (all jobs)
+  // and the jobs' write-pass coverage records at zero.
   auto prepare_write = [&](const std::vector<int32_t>* js) -> hipr_result {
     if (!js) {
-      hipLaunchKernelGGL(FillKernel, dim3(1024), dim3(256), 0, st, ctx->map0.as<int32_t>(),
-                         total_map, kNoTile);
-      hipLaunchKernelGGL(FillKernel, dim3(1024), dim3(256), 0, st, ctx->map1.as<int32_t>(),
-                         total_map, kNoTile);
-      hipLaunchKernelGGL(FillKernel, dim3(256), dim3(256), 0, st, (int32_t*)ctx->wcov.p,
-                         (int64_t)nj * (int64_t)(sizeof(JobCov) / 4), 0);
-      hipLaunchKernelGGL(FillKernel, dim3(1), dim3(kWave), 0, st, ctx->pool_ctr.as<int32_t>(),
-                         (int64_t)1, 0);
+      hipLaunchKernelGGL(PrepareWriteKernel, dim3(1024), dim3(256), 0, st, ctx->map0.as<int32_t>(),
+                         ctx->map1.as<int32_t>(), total_map, (int32_t*)ctx->wcov.p,
+                         (int64_t)nj * (int64_t)(sizeof(JobCov) / 4), ctx->pool_ctr.as<int32_t>(),
+                         ctx->counters.as<unsigned long long>());
     } else if (!js->empty()) {
       hipr_result rr = Upload(&ctx->gather_list, js->data(), js->size(), st);
       if (rr != HIPR_SUCCESS) return rr;
@@ -2057,6 +2081,7 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
       test[j] = pcap[j];
     }
   } else if (counted) {
+    if ((r = upload_tables()) != HIPR_SUCCESS) return r;
     // count pass over every job (recording the band snapshots), then planes
     // sized exactly
     if ((r = walk_pass(kWalkCount, small, wide)) != HIPR_SUCCESS) return r;
@@ -2077,13 +2102,15 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   const int64_t pool_base = plane_total;
   const int64_t pool_cap = mode == 0 ? 0 : std::max<int64_t>(plane_total / 4, 1 << 16);
   plane_total += pool_cap;
-  if (ctx->pool_ctr.Ensure(sizeof(int32_t)) != hipSuccess) return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
+  if (ctx->pool_ctr.Ensure(sizeof(int32_t)) != hipSuccess ||
+      ctx->counters.Ensure(2 * sizeof(unsigned long long)) != hipSuccess)
+    return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
   if ((r = upload_planes()) != HIPR_SUCCESS) return r;
   wp.pool_ctr = ctx->pool_ctr.as<int32_t>();
   wp.pool_base = (int32_t)pool_base;
   wp.pool_cap = (int32_t)pool_cap;
-  wp.plane_base = ctx->plane_base.as<int64_t>();
-  wp.plane_cap = ctx->plane_cap.as<int32_t>();
+  wp.plane_base = dt.plane_base;
+  wp.plane_cap = dt.plane_cap;
   wp.map0 = ctx->map0.as<int32_t>();
   wp.map1 = ctx->map1.as<int32_t>();
   wp.planes = ctx->planes.as<uint8_t>();
@@ -2107,18 +2134,18 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
         mixed |= tier[j] > 1;
       }
     const bool merge = mixed && plain_small > kBandSlots;
-    for (int k : kTiers) {
-      std::vector<int32_t> banded, plain;
-      for (int32_t j : all) {
-        if (nbands[j] > 1) {
-          if (tier[j] == k) banded.push_back(j);
-        } else if ((merge && tier[j] <= 4 ? 4 : tier[j]) == k) {
-          plain.push_back(j);
-        }
-      }
-      if (!banded.empty())
-        chains.push_back({{kWalkSchedule, k, 0, banded}, {kWalkWrite, k, 0, banded}});
-      if (!plain.empty()) chains.push_back({{kWalkWrite, k, 0, std::move(plain)}});
+    std::vector<int32_t> banded[kTierCount], plain[kTierCount];
+    for (int32_t j : all) {
+      if (nbands[j] > 1)
+        banded[tier_index(tier[j])].push_back(j);
+      else
+        plain[tier_index(merge && tier[j] <= 4 ? 4 : tier[j])].push_back(j);
+    }
+    for (int i = kTierCount - 1; i >= 0; i--) {
+      if (!banded[i].empty())
+        chains.push_back(
+            {{kWalkSchedule, 1 << i, 0, &banded[i]}, {kWalkWrite, 1 << i, 0, &banded[i]}});
+      if (!plain[i].empty()) chains.push_back({{kWalkWrite, 1 << i, 0, &plain[i]}});
     }
     if ((r = run_plan(place_chains(std::move(chains)))) != HIPR_SUCCESS) return r;
   }
@@ -2169,50 +2196,42 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
     max_active = std::max<int64_t>(max_active, hw[j].max_active);
   }
   f.stats.max_active = max_active;
-  surf->job_edges.assign(nj, -1);
-  surf->job_planes.assign(nj, -1);
-  surf->job_steps.assign(nj, 0);
-  surf->job_time.assign(nj, 0);
-  surf->job_phase.assign((size_t)nj * 5, 0);
-  surf->job_active.assign(nj, 0);
   surf->draw_serial = ++ctx->draw_serial;
-  surf->job_path.assign(nj, 0);
-  surf->job_kind.assign(nj, 0);
-  surf->job_canvas.assign(nj, 0);
-  surf->job_ebase.assign(nj, 0);
-  surf->job_mbase.assign(nj, 0);
-  surf->job_tiles.assign((size_t)nj * 5, 0);
+  for (auto* v : {&surf->job_edges, &surf->job_planes, &surf->job_steps, &surf->job_time,
+                  &surf->job_active, &surf->job_path, &surf->job_kind, &surf->job_canvas})
+    v->resize(nj);
+  surf->job_phase.resize((size_t)nj * 5);
+  surf->job_tiles.resize((size_t)nj * 5);
+  surf->job_ebase.resize(nj);
+  surf->job_mbase.resize(nj);
   for (int j = 0; j < nj; j++) {
+    const bool walked = f.jobs[j].kind != kJobRect;
+    const JobCov c = walked ? hw[j] : JobCov{};
+    const TileRange tr = walked ? spans[j].tr : TileRange{};
     surf->job_path[j] = f.jobs[j].path;
     surf->job_kind[j] = f.jobs[j].kind;
     surf->job_canvas[j] = f.jobs[j].canvas;
-    if (f.jobs[j].kind == kJobRect) continue;
-    surf->job_ebase[j] = ebase[j];
-    surf->job_mbase[j] = mbase[j];
-    const Canvas& cv = f.canvases[f.jobs[j].canvas];
-    TileRange tr = JobTiles(JobScanBounds(ctx->h_geo[j]), cv.width, cv.height);
+    surf->job_ebase[j] = walked ? ebase[j] : 0;
+    surf->job_mbase[j] = walked ? ht.map_base[j] : 0;
+    surf->job_edges[j] = walked ? ctx->h_geo[j].edges : -1;
+    surf->job_planes[j] = walked ? c.planes : -1;
+    surf->job_steps[j] = c.steps;
+    surf->job_time[j] = c.time_10ns;
+    surf->job_active[j] = c.max_active;
+    for (int k = 0; k < 5; k++) surf->job_phase[(size_t)j * 5 + k] = c.phase[k];
     int32_t* t = &surf->job_tiles[(size_t)j * 5];
     t[0] = tr.tc0;
     t[1] = tr.tr0;
     t[2] = tr.ntc;
     t[3] = tr.ntr;
-    t[4] = cv.tiles_x;
-  }
-  for (int j = 0; j < nj; j++) {
-    if (f.jobs[j].kind == kJobRect) continue;
-    surf->job_edges[j] = ctx->h_geo[j].edges;
-    surf->job_planes[j] = hw[j].planes;
-    surf->job_steps[j] = hw[j].steps;
-    surf->job_time[j] = hw[j].time_10ns;
-    surf->job_active[j] = hw[j].max_active;
-    for (int k = 0; k < 5; k++) surf->job_phase[(size_t)j * 5 + k] = hw[j].phase[k];
+    t[4] = walked ? f.canvases[f.jobs[j].canvas].tiles_x : 0;
   }
   // ---- composite: layers, blur, canvas ----
   CompositeParams cp{};
   cp.n_canvases = (int)f.canvases.size();
   cp.jobs = f.d_jobs;
   cp.cov = ctx->wcov.as<JobCov>();
-  cp.map_base = ctx->map_base.as<int64_t>();
+  cp.map_base = dt.map_base;
   cp.map0 = ctx->map0.as<int32_t>();
   cp.map1 = ctx->map1.as<int32_t>();
   cp.planes = ctx->planes.as<uint8_t>();
@@ -2337,14 +2356,12 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   mp.canvases = ctx->canvases.as<Canvas>();
   mp.n_canvases = n_targets;
   mp.total_tiles = main_tiles;
-  if (ctx->counters.Ensure(2 * sizeof(unsigned long long)) != hipSuccess)
-    return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
-  HIP_TRY(hipMemsetAsync(ctx->counters.p, 0, 2 * sizeof(unsigned long long), st));
   mp.counters = ctx->counters.as<unsigned long long>();
   STAGE_LAUNCH(ctx, HIPR_STAGE_COMPOSITE, composite(mp, main_tiles));
   HIP_TRY(hipGetLastError());
-  unsigned long long counts[2] = {0, 0};
-  HIP_TRY(hipMemcpyAsync(counts, ctx->counters.p, sizeof(counts), hipMemcpyDeviceToHost, st));
+  unsigned long long* const counts = ctx->h_counts;
+  HIP_TRY(hipMemcpyAsync(counts, ctx->counters.p, 2 * sizeof(unsigned long long),
+                         hipMemcpyDeviceToHost, st));
   HIP_TRY(hipEventRecord(ctx->ev1, st));
   HIP_TRY(hipEventSynchronize(ctx->ev1));
   f.stats.blends = (int64_t)counts[0];
@@ -2863,25 +2880,21 @@ static void FreeContext(hipr_context ctx) {
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
   DevBuf* bufs[] = {&ctx->job_tiles, &ctx->canvases, &ctx->layer_canvases, &ctx->geo, &ctx->cov, &ctx->edge_base,
-                    &ctx->edge_cap, &ctx->edges, &ctx->wedges, &ctx->gkeys, &ctx->plane_base,
-                    &ctx->plane_cap, &ctx->planes, &ctx->map_base, &ctx->map0, &ctx->map1,
+                    &ctx->edge_cap, &ctx->edges, &ctx->wedges, &ctx->gkeys,
+                    &ctx->planes, &ctx->tables, &ctx->map0, &ctx->map1,
                     &ctx->sub_list, &ctx->big_list, &ctx->bound, &ctx->gather_list, &ctx->stroke_out, &ctx->o_verbs, &ctx->o_pts, &ctx->o_w,
                     &ctx->s_verbs, &ctx->s_pts, &ctx->s_w, &ctx->layers, &ctx->blur_rows,
                     &ctx->blur_cols, &ctx->blur_rb, &ctx->blur_cb, &ctx->blur_tmp,
                     &ctx->blur_jobs, &ctx->blur_lines, &ctx->d_verbs, &ctx->d_pts, &ctx->d_w,
                     &ctx->d_jobs, &ctx->run_jobs, &ctx->counters, &ctx->wcov,
-                    &ctx->qstate, &ctx->q_base, &ctx->snaps, &ctx->snap_base,
-                    &ctx->band_count, &ctx->queues, &ctx->flatten_redo, &ctx->pool_ctr, &ctx->stroke_redo,
+                    &ctx->qstate, &ctx->snaps, &ctx->queues, &ctx->flatten_redo, &ctx->pool_ctr, &ctx->stroke_redo,
                     &ctx->stroke_redo_out, &ctx->blur_raw, &ctx->blur_styles};
   for (DevBuf* b : bufs) b->Free();
   DevBuf* mlp[] = {&ctx->mlp_prm, &ctx->mlp_ops, &ctx->mlp_feats, &ctx->mlp_preds,
                    &ctx->mlp_targets, &ctx->mlp_grads, &ctx->mlp_loss, &ctx->mlp_m,
                    &ctx->mlp_v, &ctx->mlp_gsum, &ctx->mlp_curve};
   for (DevBuf* b : mlp) b->Free();
-  if (ctx->h_geo) (void)hipHostFree(ctx->h_geo);
-  if (ctx->h_cov) (void)hipHostFree(ctx->h_cov);
-  if (ctx->h_wcov) (void)hipHostFree(ctx->h_wcov);
-  if (ctx->h_so) (void)hipHostFree(ctx->h_so);
+  FreeHostStage(ctx);
   for (hipEvent_t e : ctx->ev_pool) (void)hipEventDestroy(e);
   (void)hipEventDestroy(ctx->ev0);
   (void)hipEventDestroy(ctx->ev1);
