@@ -1122,16 +1122,16 @@ void SetTiles(std::vector<Canvas>* cvs) {
 }
 
 // Nominal rows per walk band (the write pass runs the bands of a path
-// concurrently).  Exact form: every path is banded by its count pass;
-// estimate forms: only the widest paths, after a schedule pass, whose
-// banded write then ends the walk stage, so shorter bands pay there
-// (curves + strokes at 2048^2: learned 155.0 -> 152.6 ms with 64 rows;
-// exact 305 -> 308 ms).
+// concurrently).  With a count pass every path is banded by it; without one
+// only the widest and tallest paths are, after a schedule pass, whose banded
+// write then ends the walk stage, so shorter bands pay there (curves +
+// strokes at 2048^2, when the lines were drawn: learned 155.0 -> 152.6 ms
+// with 64 rows; counted 305 -> 308 ms).
 constexpr int kBandRowsExact = 128;
 constexpr int kBandRowsEstimates = 64;
-// Estimate modes: paths whose active-edge bound reaches this are banded:
-// the paths of the 8- and 16-slot walks, the longest sequential walks of a
-// frame, whose schedule pass and banded write run beside the 4-slot writes.
+// Without a count pass: paths whose active-edge bound reaches this are banded,
+// the longest sequential walks of a frame, whose schedule pass and banded
+// write run beside the writes of shorter lists.
 // (Banding every path costs more schedule work than it saves; the
 // autotuner tries other thresholds.)
 constexpr int kBandMinEdges = 4 * kWave + 1;
@@ -1500,11 +1500,18 @@ hipr_result Flatten(Frame& f, int mode, const int32_t* edge_est, std::vector<int
 hipr_result SortGather(Frame& f, const int32_t* d_list, int n, int32_t* d_bound = nullptr) {
   if (n == 0) return HIPR_SUCCESS;
   hipr_context ctx = f.ctx;
-  STAGE_LAUNCH(ctx, HIPR_STAGE_SORT,
-    hipLaunchKernelGGL(SortGatherKernel, dim3(n), dim3(kSortThreads), 0, f.st, d_list, n,
-                     ctx->geo.as<JobGeo>(), ctx->edge_base.as<int64_t>(),
-                     ctx->edges.as<EdgeRec>(), ctx->wedges.as<EdgeRec>(),
-                     ctx->gkeys.as<uint64_t>(), d_bound));
+  // (the flatten stage has read the jobs' counts and bounds back)
+  bool small = false, large = false;
+  for (int32_t j : f.pl->walk_jobs) (SortIsSmall(ctx->h_geo[j]) ? small : large) = true;
+  auto launch = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(n), dim3(threads), 0, f.st, d_list, n, ctx->geo.as<JobGeo>(),
+                       ctx->edge_base.as<int64_t>(), ctx->edges.as<EdgeRec>(),
+                       ctx->wedges.as<EdgeRec>(), ctx->gkeys.as<uint64_t>(), d_bound);
+  };
+  hipEvent_t b = StageBegin(ctx, f.st);
+  if (large) launch(SortGatherKernel<kSortThreads, kSortLdsKeys>, kSortThreads);
+  if (small) launch(SortGatherKernel<kWave, kSortSmallKeys>, kWave);
+  StageEnd(ctx, HIPR_STAGE_SORT, b, f.st);
   HIP_TRY(hipGetLastError());
   return HIPR_SUCCESS;
 }
