@@ -103,7 +103,7 @@ struct Canvas {
   int32_t tile_begin;   // first global tile index
   int32_t job_begin, job_end;  // jobs drawn on this canvas, in order
   int32_t format;              // kFormat* bits (0: premultiplied RGBA)
-  int32_t pad;
+  int32_t row_begin;    // first global tile row index
 };
 
 // ---- wave helpers ------------------------------------------------------------

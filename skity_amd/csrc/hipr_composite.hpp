@@ -403,6 +403,11 @@ struct CompositeParams {
   // per job, the canvas tiles it touches: {tc0, tr0, tc1, tr1} (half-open;
   // empty when tc0 >= tc1), written by JobTileRangeKernel
   const int4* job_tiles;
+  // optional: per tile row of the targets, the jobs that meet it, in order
+  // (RowJobsKernel; row r's list begins at r * row_stride)
+  const int32_t* row_jobs;
+  const int32_t* row_count;
+  int32_t row_stride;
   // optional: [0] += pixel blends performed, [1] += target pixels touched
   unsigned long long* counters;
 };
@@ -432,6 +437,52 @@ __global__ void __launch_bounds__(256)
     if (tr.ntc > 0) r = make_int4(tr.tc0, tr.tr0, tr.tc0 + tr.ntc, tr.tr0 + tr.ntr);
   }
   out[j] = r;
+}
+
+// The jobs that meet each tile row of the target canvases, in draw order, so
+// that a tile of a frame of many jobs scans those of its row and not all of
+// them (a page of 16,900 glyphs has 128 rows of about 260).  One block per tile
+// row; bound by the latency of its passes over the jobs, 1,024 at a time.
+constexpr int kRowThreads = 1024;
+__global__ void __launch_bounds__(kRowThreads)
+    RowJobsKernel(const Canvas* __restrict__ canvases, int n_canvases,
+                  const int4* __restrict__ job_tiles, int stride, int32_t* __restrict__ row_jobs,
+                  int32_t* __restrict__ row_count) {
+  __shared__ int32_t part[kRowThreads / kWave];
+  const int row = blockIdx.x;
+  int lo = 0, hi = n_canvases - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (canvases[mid].row_begin <= row) {
+      lo = mid;
+    } else {
+      hi = mid - 1;
+    }
+  }
+  const int begin = canvases[lo].job_begin, end = canvases[lo].job_end;
+  const int ty = row - canvases[lo].row_begin;
+  const int wave = threadIdx.x / kWave;
+  int32_t* out = row_jobs + (int64_t)row * stride;
+  int n = 0;
+  for (int first = begin; first < end; first += kRowThreads) {
+    const int j = first + threadIdx.x;
+    bool in = false;
+    if (j < end) {
+      const int4 tb = job_tiles[j];
+      in = tb.x < tb.z && ty >= tb.y && ty < tb.w;
+    }
+    const uint64_t mask = __ballot(in);
+    if (Lane() == 0) part[wave] = __popcll(mask);
+    __syncthreads();
+    int at = n;
+    for (int w = 0; w < kRowThreads / kWave; w++) {
+      if (w < wave) at += part[w];
+      n += part[w];
+    }
+    if (in) out[at + __popcll(mask & ((1ull << Lane()) - 1))] = j;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) row_count[row] = n;
 }
 
 // SWSpanBrush::BrushH for one pixel and cover (sw_span_brush.cc:108-138):
@@ -595,8 +646,16 @@ __global__ void __launch_bounds__(64) CompositeKernel(CompositeParams P) {
   auto plane_word = [&](int plane) {
     return *((const uint32_t*)(P.planes + (int64_t)plane * kTilePlaneBytes) + lane);
   };
-  for (int jb = cv.job_begin; jb < cv.job_end; jb += kWave) {
-    int j = jb + lane;
+  // the jobs to scan: the tile row's list, or all of the canvas
+  const int32_t* list = nullptr;
+  int scan = cv.job_end - cv.job_begin;
+  if (P.row_jobs) {
+    list = P.row_jobs + (int64_t)(cv.row_begin + ty) * P.row_stride;
+    scan = P.row_count[cv.row_begin + ty];
+  }
+  for (int first = 0; first < scan; first += kWave) {
+    const int i = first + lane;
+    const int j = i >= scan ? cv.job_end : list ? list[i] : cv.job_begin + i;
     int s0 = kNoTile, s1 = kNoTile;
     uint32_t s_color = 0;
     bool present = false, plain = false;
@@ -661,7 +720,7 @@ __global__ void __launch_bounds__(64) CompositeKernel(CompositeParams P) {
         }
         continue;
       }
-      int jj = jb + b;
+      const int jj = __builtin_amdgcn_readlane(j, b);
       const Job job = P.jobs[jj];
       // fields are read where used (the paint index is wave-uniform)
       const PaintDev& pd = P.paints[job.paint];

@@ -323,6 +323,7 @@ struct hipr_context_s {
   DevBuf planes, map0, map1, sub_list, big_list, bound,
       gather_list;
   DevBuf wcov, qstate, snaps;  // write-pass coverage, row bands
+  DevBuf row_jobs;                        // per tile row, the jobs that meet it
   DevBuf tables;                          // per-job offsets of the walk (JobTables)
   DevBuf queues;                          // persistent walk: item counters
   DevBuf srgb;                            // sRGB colour-filter tables (512 bytes)
@@ -1112,14 +1113,25 @@ void BuildPlan(const hipr_scene* s, hipr_prepared_s* pl) {
 }
 
 void SetTiles(std::vector<Canvas>* cvs) {
-  int total = 0;
+  int total = 0, rows = 0;
   for (auto& cv : *cvs) {
     cv.tiles_x = (cv.width + kTile - 1) / kTile;
     cv.tiles_y = (cv.height + kTile - 1) / kTile;
     cv.tile_begin = total;
     total += cv.tiles_x * cv.tiles_y;
+    cv.row_begin = rows;
+    rows += cv.tiles_y;
   }
 }
+
+// The composite scans per tile row the jobs that meet it where a target has
+// this many jobs, as long as the rows' lists (room for every job) stay within
+// 64 MiB.  A text page of 16,900 glyphs: composite 0.568 ms scanning all of
+// them for every tile, 0.434 by rows.  421 jobs on 1280 x 720: 0.112 and 0.106;
+// 4,096 jobs that cover most of their target: 8.3 and 8.4.  Below 256 jobs the
+// scan is four passes at most, and the lists' kernel takes as long.
+constexpr int kRowJobsMin = 256;
+constexpr int64_t kRowJobsRoom = 16 << 20;
 
 // Nominal rows per walk band (the write pass runs the bands of a path
 // concurrently).  With a count pass every path is banded by it; without one
@@ -2364,7 +2376,28 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   mp.n_canvases = n_targets;
   mp.total_tiles = main_tiles;
   mp.counters = ctx->counters.as<unsigned long long>();
-  STAGE_LAUNCH(ctx, HIPR_STAGE_COMPOSITE, composite(mp, main_tiles));
+  int target_rows = 0;
+  int32_t most_jobs = 0;
+  for (int t = 0; t < n_targets; t++) {
+    target_rows += f.canvases[t].tiles_y;
+    most_jobs = std::max(most_jobs, f.canvases[t].job_end - f.canvases[t].job_begin);
+  }
+  const bool by_row =
+      most_jobs >= kRowJobsMin && (int64_t)target_rows * most_jobs <= kRowJobsRoom;
+  hipEvent_t composite_begin = StageBegin(ctx, st);
+  if (by_row) {
+    const int64_t entries = (int64_t)target_rows * most_jobs;
+    if (ctx->row_jobs.Ensure(sizeof(int32_t) * (entries + target_rows)) != hipSuccess)
+      return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
+    mp.row_jobs = ctx->row_jobs.as<int32_t>();
+    mp.row_count = mp.row_jobs + entries;
+    mp.row_stride = most_jobs;
+    hipLaunchKernelGGL(RowJobsKernel, dim3(target_rows), dim3(kRowThreads), 0, st, mp.canvases,
+                       n_targets, mp.job_tiles, most_jobs, ctx->row_jobs.as<int32_t>(),
+                       ctx->row_jobs.as<int32_t>() + entries);
+  }
+  composite(mp, main_tiles);
+  StageEnd(ctx, HIPR_STAGE_COMPOSITE, composite_begin, st);
   HIP_TRY(hipGetLastError());
   unsigned long long* const counts = ctx->h_counts;
   HIP_TRY(hipMemcpyAsync(counts, ctx->counters.p, 2 * sizeof(unsigned long long),
@@ -2888,7 +2921,7 @@ static void FreeContext(hipr_context ctx) {
   (void)hipStreamSynchronize(ctx->stream);
   DevBuf* bufs[] = {&ctx->job_tiles, &ctx->canvases, &ctx->layer_canvases, &ctx->geo, &ctx->cov, &ctx->edge_base,
                     &ctx->edge_cap, &ctx->edges, &ctx->wedges, &ctx->gkeys,
-                    &ctx->planes, &ctx->tables, &ctx->map0, &ctx->map1,
+                    &ctx->planes, &ctx->tables, &ctx->row_jobs, &ctx->map0, &ctx->map1,
                     &ctx->sub_list, &ctx->big_list, &ctx->bound, &ctx->gather_list, &ctx->stroke_out, &ctx->o_verbs, &ctx->o_pts, &ctx->o_w,
                     &ctx->s_verbs, &ctx->s_pts, &ctx->s_w, &ctx->layers, &ctx->blur_rows,
                     &ctx->blur_cols, &ctx->blur_rb, &ctx->blur_cb, &ctx->blur_tmp,

@@ -119,3 +119,38 @@ def test_covers_of_one_colour(ctx, n, filtered):
         surf.close()
         want = O.render_ex(sc.scene, sc.width, sc.height, alpha, colour)
         assert diff_report(got, want) == (0, 0)
+
+
+@pytest.mark.parametrize("n", [255, 256, 1024, 1025])
+def test_many_paths(ctx, n):
+    """Small paths, rectangles and whole-canvas draws on two targets of one
+    batch: either side of the number of jobs from which the composite scans by
+    tile row, and of the 1,024 jobs that a pass over them takes."""
+    rng = np.random.default_rng(n)
+    scs = []
+    for w, h in ((70, 150), (33, 49)):
+        c = Canvas(w, h)
+        for i in range(n if w == 70 else 40):
+            paint = Paint((*rng.uniform(0, 1, 3), rng.uniform(0.2, 1.0)))
+            if i % 97 == 5:
+                c.draw_paint(paint)
+                continue
+            x, y, s = rng.uniform(-10, w + 10), rng.uniform(-10, h + 10), rng.uniform(0.5, 9)
+            c.draw_path(Path().add_circle(x, y, s) if i % 3 else
+                        Path().add_rect(x, y, x + s, y + 4 * s), paint)
+        scs.append(c.scene())
+    surfs = [device.Surface(ctx, sc.width, sc.height) for sc in scs]
+    preps = [device.Prepared(ctx, sc.scene) for sc in scs]
+    batch = device.Batch(ctx)
+    for su, pr in zip(surfs, preps):
+        batch.add(su, pr)
+    for mode in (abi.MODE_EXACT, abi.MODE_LEARNED):
+        print(f"{n} paths, mode {mode}", flush=True)
+        for su in surfs:
+            su.clear(0)
+        batch.draw(mode=mode)
+        for su, sc in zip(surfs, scs):
+            assert diff_report(su.read(), O.render(sc.scene, sc.width, sc.height)) == (0, 0)
+    batch.close()
+    for x in surfs + preps:
+        x.close()
