@@ -1655,22 +1655,25 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
 }
 
 // The slot walk's kernel (paths of more than 64 active edges; up to 64 walk as
-// a team of one wave, hipr_walk_team.hpp).  Without a queue, workgroup i walks item i (the
-// dispatcher hands out items in list order).  With a queue (persistent
-// form), a grid sized to the resident waves takes items from an atomic
-// counter until the list is exhausted; every wave leaves when the counter
-// passes n_walk.
-// The 4- and 8-slot walks are held to 256 registers (two waves per SIMD):
-// the 4-slot walk fits without spilling; the 8-slot walk spills, which its
-// row bands more than make up for, since 4-slot waves can then share its
-// SIMDs.  The 16-, 32- and 64-slot walks take what they need.
+// a team of one wave, hipr_walk_team.hpp).  Without a queue, workgroup i walks
+// item i (the dispatcher hands out items in list order).  With a queue
+// (persistent form), a grid sized to the resident waves takes items from an
+// atomic counter until the list is exhausted; every wave leaves when the
+// counter passes n_walk.
+// Bound by instruction issue and by the chain of a path's sub-steps; HBM is
+// idle.  Curves + strokes, 4,096 paths at 2048^2: the write pass 144 ms with
+// one trapezoid per lane and one row per turn, 88.5 ms now.  The 2-, 4- and
+// 8-slot walks are held to 256 registers (two waves per SIMD); a tighter cap
+// does not let more waves in, since a walk's LDS (17.6 KB at 2048 px) holds
+// nine to a CU: capped to 168 and 128 registers the pass took 90.9 and 91.7
+// ms.  The 16-, 32- and 64-slot walks take what they need.
 template <int K, int kMode>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 8 ? 2 : 1)))
 WalkKernel(WalkParams P) {
   extern __shared__ int32_t lds[];
   // The 8- and 16-slot walks hold the paths with the widest active lists,
   // the longest sequential walks of a frame: their waves take precedence in
-  // instruction issue over the 4-slot waves sharing their SIMD.
+  // instruction issue over the waves of shorter lists on their SIMD.
   if (K >= 8) __builtin_amdgcn_s_setprio(2);
   // one call site, so the item body is inlined once
   auto take = [&]() -> int {
@@ -1723,7 +1726,7 @@ __global__ void PrepareWriteKernel(int32_t* __restrict__ map0, int32_t* __restri
   }
   for (int64_t i = first; i < n_cov; i += step) cov[i] = 0;
   if (first == 0) *pool_ctr = 0;
-  if (first < 2) counters[first] = 0;
+  for (int64_t i = first; i < kCounterWords; i += step) counters[i] = 0;
 }
 
 // Zeroes the coverage records of the listed jobs (before a write pass redoes

@@ -528,7 +528,7 @@ hipr_result HostStage(hipr_context ctx, size_t n) {
     HIP_TRY(hipHostMalloc((void**)&ctx->h_bound, want * sizeof(int32_t)));
     HIP_TRY(hipHostMalloc((void**)&ctx->h_pred, want * kMlpOut * sizeof(float)));
     HIP_TRY(hipHostMalloc((void**)&ctx->h_tables, want * JobTables::kBytes));
-    HIP_TRY(hipHostMalloc((void**)&ctx->h_counts, 2 * sizeof(unsigned long long)));
+    HIP_TRY(hipHostMalloc((void**)&ctx->h_counts, kCounterWords * sizeof(unsigned long long)));
     ctx->h_cap = want;
   }
   return HIPR_SUCCESS;
@@ -1126,10 +1126,11 @@ void SetTiles(std::vector<Canvas>* cvs) {
 
 // The composite scans per tile row the jobs that meet it where a target has
 // this many jobs, as long as the rows' lists (room for every job) stay within
-// 64 MiB.  A text page of 16,900 glyphs: composite 0.568 ms scanning all of
-// them for every tile, 0.434 by rows.  421 jobs on 1280 x 720: 0.112 and 0.106;
-// 4,096 jobs that cover most of their target: 8.3 and 8.4.  Below 256 jobs the
-// scan is four passes at most, and the lists' kernel takes as long.
+// 64 MiB.  A text page of 16,900 glyphs: the composite takes 0.134 ms more when
+// every tile scans all of them (0.21 against 0.08).  421 jobs on 1280 x 720:
+// 0.006 more; 4,096 jobs that cover most of their target: 0.1 less of 8.3.
+// Below 256 jobs the scan is four passes at most, and the lists' kernel takes
+// as long.
 constexpr int kRowJobsMin = 256;
 constexpr int64_t kRowJobsRoom = 16 << 20;
 
@@ -2122,7 +2123,7 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   const int64_t pool_cap = mode == 0 ? 0 : std::max<int64_t>(plane_total / 4, 1 << 16);
   plane_total += pool_cap;
   if (ctx->pool_ctr.Ensure(sizeof(int32_t)) != hipSuccess ||
-      ctx->counters.Ensure(2 * sizeof(unsigned long long)) != hipSuccess)
+      ctx->counters.Ensure(kCounterWords * sizeof(unsigned long long)) != hipSuccess)
     return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
   if ((r = upload_planes()) != HIPR_SUCCESS) return r;
   wp.pool_ctr = ctx->pool_ctr.as<int32_t>();
@@ -2399,13 +2400,15 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   composite(mp, main_tiles);
   StageEnd(ctx, HIPR_STAGE_COMPOSITE, composite_begin, st);
   HIP_TRY(hipGetLastError());
-  unsigned long long* const counts = ctx->h_counts;
-  HIP_TRY(hipMemcpyAsync(counts, ctx->counters.p, 2 * sizeof(unsigned long long),
-                         hipMemcpyDeviceToHost, st));
+  const unsigned long long* const counts = ctx->h_counts;
+  HIP_TRY(hipMemcpyAsync(ctx->h_counts, ctx->counters.p,
+                         kCounterWords * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
   HIP_TRY(hipEventRecord(ctx->ev1, st));
   HIP_TRY(hipEventSynchronize(ctx->ev1));
-  f.stats.blends = (int64_t)counts[0];
-  f.stats.pixels = (int64_t)counts[1];
+  for (int k = 0; k < kCounterSlots; k++) {
+    f.stats.blends += (int64_t)counts[k * kCounterStride];
+    f.stats.pixels += (int64_t)counts[k * kCounterStride + 1];
+  }
   float ms = 0;
   HIP_TRY(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
   f.stats.ms_total = ms;
