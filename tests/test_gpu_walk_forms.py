@@ -154,3 +154,23 @@ def test_many_paths(ctx, n):
     batch.close()
     for x in surfs + preps:
         x.close()
+
+
+@pytest.mark.parametrize("join", [abi.JOIN_MITER, abi.JOIN_ROUND, abi.JOIN_BEVEL])
+def test_runs_of_lines(ctx, join):
+    """Stroked polylines either side of the shortest run that lanes share, of a
+    wave's 64 lines and of a chunk's 128 calls."""
+    rng = np.random.default_rng(join)
+    c = Canvas(260, 190)
+    for i, n in enumerate((1, 2, 3, 4, 63, 64, 65, 66, 127, 128, 129, 130, 300)):
+        paint = Paint((*rng.uniform(0, 1, 3), 0.7))
+        paint.set_style(abi.STYLE_STROKE).set_stroke_width(float(rng.uniform(0.4, 6)))
+        paint.set_stroke_join(join).set_stroke_cap(i % 3)
+        p = Path().move_to(130, 95)
+        x, y = 130.0, 95.0
+        for k in range(n):
+            if k % 11 != 5:  # (else a line of no length)
+                x, y = np.clip((x + rng.normal(0, 14), y + rng.normal(0, 14)), 2, 185)
+            p.line_to(x, y)
+        c.draw_path(p.close() if i % 4 == 1 else p, paint)
+    check(ctx, c.scene(), f"join {join}")

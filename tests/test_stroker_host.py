@@ -181,3 +181,44 @@ def test_width_zero_open_strokes_draw_nothing():
     sc = _hairline_scene(False)
     img = O.render(sc.scene, sc.width, sc.height)
     assert not img.any()
+
+
+def _polyline(rng, n, close):
+    """n lines, some back on themselves, straight on, too short to stroke or
+    of no length."""
+    p = Path()
+    x, y = rng.uniform(20, 140, 2)
+    p.move_to(x, y)
+    dx, dy = 7.0, 2.0
+    for _ in range(n):
+        k = rng.integers(0, 12)
+        if k == 0:
+            dx, dy = -dx, -dy
+        elif k == 1:
+            x, y = x + 1e-5, y
+        elif k > 3:
+            dx, dy = rng.normal(0, 9, 2)
+        if k not in (1, 2):
+            x, y = x + dx, y + dy
+        p.line_to(x, y)
+    return p.close() if close else p
+
+
+@pytest.mark.parametrize("join", [abi.JOIN_MITER, abi.JOIN_ROUND, abi.JOIN_BEVEL])
+@pytest.mark.parametrize("cap", [abi.CAP_BUTT, abi.CAP_ROUND, abi.CAP_SQUARE])
+def test_runs_of_lines(host, join, cap):
+    """Runs either side of the shortest that lanes share, of a wave's 64 and of
+    a chunk's 128 calls, with a quad between two of them."""
+    rng = np.random.default_rng(31 * join + cap)
+    c = Canvas(160, 160)
+    for n in (1, 2, 3, 4, 63, 64, 65, 66, 127, 128, 129, 130, 300):
+        p = Paint().set_style(abi.STYLE_STROKE).set_stroke_width(float(rng.uniform(0.5, 12)))
+        p.set_stroke_join(join).set_stroke_cap(cap)
+        path = _polyline(rng, n, n % 2 == 0)
+        path.quad_to(30, 40, 90, 20)
+        for x, y in rng.uniform(0, 160, (n % 7, 2)):
+            path.line_to(x, y)
+        c.draw_path(path, p)
+    sc = c.scene()
+    for i in range(sc.n_paths):
+        assert _same(host, sc.scene, i), i
