@@ -68,12 +68,18 @@ def frame_alg_bytes(sc, st, blur_bytes=0):
 
 
 PMC_SUMMARY = os.path.join(HERE, "profiles", "pmc_curves_strokes_4096.json")
-STAGE_KERNELS = {"walk": ("hipr::WalkKernel<4, 1>", "hipr::WalkKernel<8, 1>",
-                          "hipr::WalkKernel<16, 1>"),
-                 "walk_count": ("hipr::WalkKernel<4, 0>", "hipr::WalkKernel<8, 0>",
-                                "hipr::WalkKernel<16, 0>"),
-                 "composite": ("hipr::CompositeKernel",), "flatten": ("hipr::FlattenKernel<1>",),
-                 "sort": ("hipr::SortGatherKernel",)}
+# (a pass that writes planes counts as the walk, its schedule kernels included)
+STAGE_KERNELS = {"walk": tuple(f"hipr::{k}, {m}>" for m in (1, 2)
+                               for k in ("TeamWalkKernel<1", "TeamWalkKernel<8",
+                                         "TeamWalkKernel<16", "WalkKernel<2", "WalkKernel<4",
+                                         "WalkKernel<8", "WalkKernel<16")),
+                 "walk_count": tuple(f"hipr::{k}, 0>" for k in (
+                     "TeamWalkKernel<1", "WalkKernel<2", "WalkKernel<4", "WalkKernel<8",
+                     "WalkKernel<16")),
+                 "composite": ("hipr::CompositeKernel<false>", "hipr::RowJobsKernel"),
+                 "flatten": ("hipr::FlattenKernel<1>",),
+                 "sort": ("hipr::SortGatherKernel<64, 1024>",
+                          "hipr::SortGatherKernel<256, 8192>")}
 
 
 def measured_traffic(stage, form):
@@ -430,8 +436,8 @@ def main():
         return
     world = int(os.environ.get("WORLD_SIZE", "1"))
     if args.gpus != 1 or world != 1:
-        print("bench.py measures one GPU: every box of this build has a single MI355X "
-              "and the pipeline has no multi-GPU path; run with --gpus 1.", file=sys.stderr)
+        print("bench.py measures one GPU: the pipeline has no multi-GPU path; run with --gpus 1.",
+              file=sys.stderr)
         sys.exit(2)
 
     import torch

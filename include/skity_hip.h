@@ -258,7 +258,8 @@ typedef struct hipr_options {
                                      counts the planes unless it is 0 */
   int32_t band_min_edges;         /* estimate modes: band only the paths whose
                                      active-edge bound reaches this; 0 = default
-                                     (257: the 8- and 16-slot walks), < 0 =
+                                     (257, and the paths that are tall for
+                                     their frame), < 0 =
                                      every path, a huge value = none */
   int32_t flags;                  /* HIPR_FLAG_* */
   int32_t chunk_points;           /* a draw of more source points than this
@@ -268,7 +269,8 @@ typedef struct hipr_options {
                                      Draws with mask filters run whole. */
 } hipr_options;
 enum {
-  HIPR_FLAG_NO_GRAPH = 1,   /* launch the walk passes directly, not as hipGraphs */
+  HIPR_FLAG_NO_GRAPH = 1,   /* time every walk kernel by itself, not each pass as
+                               a whole (walk passes are direct launches either way) */
   HIPR_FLAG_PERSISTENT = 2  /* persistent walk kernels on an atomic work queue   */
 };
 

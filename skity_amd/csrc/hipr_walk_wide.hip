@@ -1,7 +1,7 @@
 // The 32- and 64-slot walks: paths whose rows keep more than 1024 active
 // edges (WalkEdges keeps its active list as a linked list of any length,
 // src/render/sw/sw_raster.cc:546-677).  The active list stays in the
-// K x 64-lane register layout of the narrower walks; at these widths most of
+// K x 64-lane register layout of the 2- to 16-slot walks; at these widths most of
 // it lives in scratch memory, which is the price of a rare path, not of the
 // frame.  These jobs are walked unbanded (no schedule pass), so only the
 // count and write modes exist.  Compiled as its own translation unit so the
