@@ -253,7 +253,8 @@ typedef struct hipr_options {
   const int32_t* tile_estimates;  /* n_paths or NULL */
   int32_t blur_impl;              /* HIPR_BLUR_IMPL_*; 0 = MFMA */
   int32_t band_rows;              /* rows per walk band: 0 = default (128
-                                     where the planes are counted, else 64),
+                                     where the planes are counted, else 64, or
+                                     16 in a frame of few rows),
                                      < 0 = one band per path; exact mode
                                      counts the planes unless it is 0 */
   int32_t band_min_edges;         /* estimate modes: band only the paths whose

@@ -1157,6 +1157,18 @@ constexpr int kBandMinEdges = 4 * kWave + 1;
 // more than it saves (curves + strokes at 2048^2, learned: 175 -> 231 ms).
 constexpr int kBandMinRows = 128;
 constexpr int kBandSlots = 2048;
+// A frame whose rows, spread over those walks, are fewer than kBandMinRows apiece
+// leaves waves idle while its bands are written: its bands are one tile row
+// each (as far as the 32 bands of a path go).  Bands of 64 and of 16 rows: 64
+// polygons at 800 x 600 1.29 and 1.02 ms, 48 polylines 12.9 and 11.0, blend
+// options 1.45 and 1.24, a batch of 3,120 outlines (225,000 rows, 110 apiece)
+// 8.5 and 7.6, a 4K picture (107 apiece) 4.13 and 4.12.  Beyond, every band is
+// another start for waves that have work: 300 curves (293 apiece) 50.4 and 51.9
+// ms, 4,096 curves 105 and 110.  A band holds the state of its path's quad
+// edges, 64 bytes an edge, so the frame's edges are limited as well (2^21: 4
+// GiB).
+constexpr int kBandRowsShort = kTile;
+constexpr int64_t kBandShortEdges = 2 << 20;
 // Exact form: planes for every tile a path could cover, up to this many (4
 // GiB), make the count pass unnecessary.
 constexpr int64_t kUncountedPlanes = 16 << 20;
@@ -1805,9 +1817,9 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   }
   // Row bands: each job's rows are split into bands walked concurrently by
   // the write pass; the count or schedule pass records where they start.
-  const int band_rows = opt && opt->band_rows != 0 ? std::max(opt->band_rows, 0)
-                        : counted                      ? kBandRowsExact
-                                                       : kBandRowsEstimates;
+  int band_rows = opt && opt->band_rows != 0 ? std::max(opt->band_rows, 0)
+                  : counted                      ? kBandRowsExact
+                                                 : kBandRowsEstimates;
   // Without a count pass banding costs a schedule pass, so only the paths
   // with the widest active lists (the longest walks) are banded.
   const bool own_split = mode != 0 && opt && opt->band_min_edges != 0;
@@ -1825,6 +1837,9 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
     for (int32_t j : all) total_rows += spans[j].rows();
     band_min_rows = (int)std::min<int64_t>(
         std::max<int64_t>(kBandMinRows, total_rows / kBandSlots), INT32_MAX);
+    if (!(opt && opt->band_rows != 0) && total_rows / kBandSlots < kBandMinRows &&
+        f.stats.edges <= kBandShortEdges)
+      band_rows = kBandRowsShort;
   }
   int32_t *const nbands = ht.band_count, *const pcap = ht.plane_cap;
   std::fill_n(nbands, nj, 1);
