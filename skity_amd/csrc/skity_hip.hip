@@ -505,6 +505,12 @@ struct JobTables {
   }
 };
 
+// Waits for everything the context has launched.
+void SyncStreams(hipr_context ctx) {
+  for (hipStream_t side : ctx->side) (void)hipStreamSynchronize(side);
+  (void)hipStreamSynchronize(ctx->stream);
+}
+
 void FreeHostStage(hipr_context ctx) {
   void** bufs[] = {(void**)&ctx->h_geo,  (void**)&ctx->h_cov,    (void**)&ctx->h_wcov,
                    (void**)&ctx->h_so,   (void**)&ctx->h_bound,  (void**)&ctx->h_pred,
@@ -1208,7 +1214,6 @@ hipr_result LaunchWalk(hipr_context ctx, void (*kernel)(WalkParams), int waves, 
                        int stage, WalkParams P, hipStream_t st, bool timed, int32_t* queue,
                        double share) {
   if (P.n_walk == 0) return HIPR_SUCCESS;
-  if (hipr_result r = WalkLdsCheck(ctx, waves, lds)) return r;
   unsigned grid = (unsigned)P.n_walk;
   P.queue = queue;
   if (queue) {
@@ -1264,12 +1269,23 @@ WalkShape ShapeOf(int tier, int mode, int64_t items) {
                       : WalkKernel<16, kWalkWrite>,
           1, false};
 }
+size_t ShapeLdsBytes(const WalkShape& w, int tier, int lds_width, int row_ints) {
+  return w.team ? (size_t)TeamLdsInts(w.waves, lds_width, row_ints) * sizeof(int32_t)
+                : WalkLdsBytes(tier, lds_width, row_ints);
+}
+// Refuses a tier whose workgroup would not fit the device (before anything of
+// its plan is launched).
+hipr_result TierLdsCheck(hipr_context ctx, int tier, int mode, int lds_width, int row_ints,
+                         int64_t items) {
+  if (tier > kMaxTeam)
+    return WalkLdsCheck(ctx, tier, WalkLdsBytes(tier, lds_width, WalkRowInts(lds_width)));
+  return WalkLdsCheck(ctx, tier,
+                      ShapeLdsBytes(ShapeOf(tier, mode, items), tier, lds_width, row_ints));
+}
 hipr_result LaunchTier(hipr_context ctx, int tier, int mode, const WalkParams& P, hipStream_t st,
                        bool timed, int32_t* queue, double share) {
   const WalkShape w = ShapeOf(tier, mode, P.n_walk);
-  const size_t lds =
-      w.team ? (size_t)TeamLdsInts(w.waves, P.lds_width, P.row_ints) * sizeof(int32_t)
-             : WalkLdsBytes(tier, P.lds_width, P.row_ints);
+  const size_t lds = ShapeLdsBytes(w, tier, P.lds_width, P.row_ints);
   const int stage = mode == kWalkCount   ? HIPR_STAGE_WALK_COUNT
                     : mode == kWalkWrite ? HIPR_STAGE_WALK
                                          : HIPR_STAGE_WALK_SCHEDULE;
@@ -1285,7 +1301,6 @@ hipr_result LaunchWalkWide(hipr_context ctx, int K, int kmode, WalkParams P, hip
   // (their lists fill the LDS: one delta row)
   P.row_ints = WalkRowInts(P.lds_width);
   size_t lds = WalkLdsBytes(K, P.lds_width, P.row_ints);
-  if (hipr_result r = WalkLdsCheck(ctx, K, lds)) return r;
   P.queue = nullptr;
   const int stage = kmode == kWalkCount ? HIPR_STAGE_WALK_COUNT : HIPR_STAGE_WALK;
   hipEvent_t b = timed ? StageBegin(ctx, st) : nullptr;
@@ -1617,8 +1632,8 @@ hipr_result RunPresize(Frame& f, std::vector<int32_t>* eest, std::vector<int32_t
 // Draws a planned scene whose canvases [0, targets.size()) are the given
 // surfaces (the others are mask-filter layers); statistics, stage times and
 // per-job profiles go to `surf`.
-hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface surf,
-                        hipr_prepared_s* pl, const hipr_options* opt) {
+hipr_result RunPasses(const std::vector<hipr_surface>& targets, hipr_surface surf,
+                      hipr_prepared_s* pl, const hipr_options* opt) {
   hipr_context ctx = surf->ctx;
   const int n_targets = (int)targets.size();
   if (n_targets != pl->n_targets) return HIPR_ERROR_INVALID_ARGUMENT;
@@ -1966,6 +1981,9 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
       }
       work.push_back(w);
       work_all += w;
+      if (cnt.back() && (rr = TierLdsCheck(ctx, l.K, l.kmode, wp.lds_width, wp.row_ints,
+                                           (int64_t)cnt.back())) != HIPR_SUCCESS)
+        return rr;
     }
     if (all_items.empty()) return HIPR_SUCCESS;
     if ((rr = Upload(&ctx->sub_list, all_items.data(), all_items.size(), st)) != HIPR_SUCCESS)
@@ -2436,6 +2454,16 @@ hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface s
   }
   surf->stats = f.stats;
   return HIPR_SUCCESS;
+}
+
+// RunPasses, and where it fails a wait for what it has launched: a walk plan
+// that ends early leaves kernels on side streams that nothing joins, and the
+// next draw takes their buffers and the pinned tables.
+hipr_result RunPipeline(const std::vector<hipr_surface>& targets, hipr_surface surf,
+                        hipr_prepared_s* pl, const hipr_options* opt) {
+  const hipr_result r = RunPasses(targets, surf, pl, opt);
+  if (r != HIPR_SUCCESS) SyncStreams(surf->ctx);
+  return r;
 }
 
 hipr_result LaunchBlurMfma(hipr_context ctx, const std::vector<BlurJob>& rows,
@@ -2936,7 +2964,7 @@ HIPR_API void hipr_context_destroy(hipr_context ctx) { ReleaseContext(ctx); }
 
 static void FreeContext(hipr_context ctx) {
   (void)hipSetDevice(ctx->device);
-  (void)hipStreamSynchronize(ctx->stream);
+  SyncStreams(ctx);
   DevBuf* bufs[] = {&ctx->job_tiles, &ctx->canvases, &ctx->layer_canvases, &ctx->geo, &ctx->cov, &ctx->edge_base,
                     &ctx->edge_cap, &ctx->edges, &ctx->wedges, &ctx->gkeys,
                     &ctx->planes, &ctx->tables, &ctx->row_jobs, &ctx->map0, &ctx->map1,
@@ -2958,7 +2986,6 @@ static void FreeContext(hipr_context ctx) {
   (void)hipEventDestroy(ctx->ev1);
   (void)hipEventDestroy(ctx->ev_fork);
   for (int k = 0; k < kSideStreams; k++) {
-    (void)hipStreamSynchronize(ctx->side[k]);
     (void)hipStreamDestroy(ctx->side[k]);
     (void)hipEventDestroy(ctx->ev_join[k]);
   }

@@ -1,0 +1,117 @@
+"""The library's host side on a HIP runtime of host memory
+(host_runtime/host_runtime.hip), which runs no kernel but can refuse launches
+and allocations: what a draw leaves behind when one of its steps fails."""
+import ctypes
+import glob
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from skity_amd import abi, build, device, presizer
+from skity_amd.canvas import Canvas, Paint, Path
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+SRC = os.path.join(HERE, "host_runtime", "host_runtime.hip")
+LIB = os.path.join(HERE, "host_runtime", "libskity_host_runtime.so")
+ERROR_DEVICE, ERROR_OUT_OF_DEVICE_MEMORY = -6, -7
+OBJS = [os.path.join(build.HERE, "_build", u.replace(".hip", ".o")) for u in build.HIP_UNITS]
+
+
+@pytest.fixture(scope="module")
+def runtime():
+    if not os.path.exists(build.HIPCC):
+        pytest.skip("hipcc not available")
+    units = glob.glob(os.path.join(build.HERE, "csrc", "*.h*"))
+    if not all(map(os.path.exists, OBJS)) or \
+            min(map(os.path.getmtime, OBJS)) < max(map(os.path.getmtime, units)):
+        build.build_hip()
+    if not os.path.exists(LIB) or \
+            os.path.getmtime(LIB) < max(map(os.path.getmtime, OBJS + [SRC])):
+        obj = LIB + ".o"
+        subprocess.run([build.HIPCC, "--cuda-host-only", "-O1", "-std=c++17", "-fPIC",
+                        "-DHIPR_TEMPLATES_ONLY", "-Wno-unused-value", "-Wno-unused-result",
+                        "-c", "-o", obj, SRC], check=True)
+        subprocess.run(["g++", "-shared", "-o", LIB + ".tmp", *OBJS, obj, "-Wl,-Bsymbolic"],
+                       check=True)
+        os.remove(obj)
+        os.replace(LIB + ".tmp", LIB)
+    real, real_load = device._lib, abi.load
+    L = ctypes.CDLL(LIB)
+    L.test_log.restype = ctypes.c_char_p
+    L.test_limit_malloc.argtypes = [ctypes.c_int64]
+    for fn in (L.test_unfinished, L.test_copied):
+        fn.restype = ctypes.c_int64
+    device._lib, abi.load = None, lambda name: L
+    device.lib()
+    abi.load = real_load
+    yield L
+    device._lib = real
+
+
+class Frame:
+    """`n` draws on a canvas of `side` pixels whose flattened bounds, edge
+    counts and active-edge bounds are the given ones, in turn."""
+
+    def __init__(self, L, side, n, ltrb, edges, bound):
+        L.test_reset()
+        a = [np.ascontiguousarray(ltrb, np.float32), np.ascontiguousarray(edges, np.int32),
+             np.ascontiguousarray(bound, np.int32)]
+        L.test_set_frame(len(a[1]), *(ctypes.c_void_p(x.ctypes.data) for x in a))
+        self.L = L
+        self.ctx = device.Context(0)
+        presizer.install(self.ctx, *presizer.load())
+        c = Canvas(side, side)
+        for i in range(n):
+            c.draw_path(Path().move_to(1, 1).line_to(9, 2).line_to(3, 8).close(),
+                        Paint((0.5, 0.1, 0.1, 1.0)))
+        self.scene = c.scene()
+        self.surf = device.Surface(self.ctx, side, side)
+        self.prep = device.Prepared(self.ctx, self.scene.scene)
+
+    def kernels(self):
+        return self.L.test_log().decode().split()
+
+    def draw(self, **kw):
+        self.L.test_reset()
+        self.surf.draw(self.prep, **kw)
+        return self.kernels()
+
+    def close(self):
+        self.surf.close()
+        self.prep.close()
+        self.ctx.close()
+
+
+def tiers(L):
+    """Draws of every width of the walk (1 .. 64 slots), some tall: a plan of
+    schedule passes and writes on all streams."""
+    side = 2048
+    tall, low = (0, 0, 300, 1900), (10, 10, 500, 90)
+    bound = [40, 40, 100, 200, 200, 400, 900, 1500, 3000]
+    ltrb = [low, tall, low, tall, low, tall, tall, low, tall]
+    return Frame(L, side, len(bound), ltrb, [200] * 5 + [4000] * 4, bound)
+
+
+@pytest.mark.parametrize("kw", [dict(mode=abi.MODE_EXACT), dict(mode=abi.MODE_EXACT, band_rows=64),
+                                dict(mode=abi.MODE_LEARNED),
+                                dict(mode=abi.MODE_LEARNED, flags=abi.FLAG_PERSISTENT)])
+def test_a_plan_that_fails_leaves_nothing_running(runtime, kw):
+    """Whichever walk launch of a draw is refused, every kernel launched before
+    it has been waited for when the draw returns: the next draw takes their
+    buffers."""
+    f = tiers(runtime)
+    names = f.draw(**kw)
+    walks = sum("WalkKernel" in k for k in names)
+    assert walks >= 8
+    assert runtime.test_unfinished() == 0
+    for at in range(walks):
+        runtime.test_reset()
+        runtime.test_fail_launch(b"WalkKernel", at)
+        with pytest.raises(device.HiprError) as e:
+            f.surf.draw(f.prep, **kw)
+        assert e.value.code == ERROR_DEVICE
+        assert runtime.test_unfinished() == 0, at
+        assert f.draw(**kw) == names
+    f.close()
