@@ -238,7 +238,8 @@ typedef struct hipr_stats {
 
 /* Execution options.  mode 0 = plain exact: edges are counted, then written;
  * tile planes are reserved for every tile a path could cover where that takes
- * at most 4 GiB (one walk), else counted and then written (two walks);
+ * at most 4 GiB and can be allocated (one walk), else counted and then written
+ * (two walks); the context keeps its largest reservation;
  * mode 1 = pre-sized single pass from the caller-supplied per-path estimates
  * (estimates != NULL), falling back to the exact two-pass method for every
  * path whose estimate was too small; mode 2 = pre-sized from the context's

@@ -53,14 +53,24 @@ namespace {
 struct DevBuf {
   void* p = nullptr;
   size_t cap = 0;
-  hipError_t Ensure(size_t bytes) {
+  // A refused allocation leaves no error behind for the next check of a launch.
+  static hipError_t Allocate(void** q, size_t bytes) {
+    hipError_t e = hipMalloc(q, bytes);
+    if (e != hipSuccess) {
+      *q = nullptr;
+      (void)hipGetLastError();
+    }
+    return e;
+  }
+  // Room for `bytes` and a quarter more, as far as `most` bytes.
+  hipError_t Ensure(size_t bytes, size_t most = SIZE_MAX) {
     if (bytes <= cap && p) return hipSuccess;
     if (p) hipFree(p);
     p = nullptr;
     cap = 0;
     size_t want = std::max<size_t>(bytes, 256);
-    want = want + want / 4;
-    hipError_t e = hipMalloc(&p, want);
+    want += std::min(want / 4, most > want ? most - want : 0);
+    hipError_t e = Allocate(&p, want);
     if (e == hipSuccess) cap = want;
     return e;
   }
@@ -70,7 +80,7 @@ struct DevBuf {
     size_t want = std::max<size_t>(bytes, 256);
     want = want + want / 4;
     void* q = nullptr;
-    hipError_t e = hipMalloc(&q, want);
+    hipError_t e = Allocate(&q, want);
     if (e != hipSuccess) return e;
     if (p) {
       keep = std::min(keep, cap);
@@ -1176,7 +1186,8 @@ constexpr int kBandSlots = 2048;
 constexpr int kBandRowsShort = kTile;
 constexpr int64_t kBandShortEdges = 2 << 20;
 // Exact form: planes for every tile a path could cover, up to this many (4
-// GiB), make the count pass unnecessary.
+// GiB), make the count pass unnecessary.  The buffer grows to that many at
+// most, and a few for the bands; where it cannot be had the planes are counted.
 constexpr int64_t kUncountedPlanes = 16 << 20;
 
 size_t WalkLdsBytes(int K, int lds_width, int row_ints) {
@@ -1814,9 +1825,7 @@ hipr_result RunPasses(const std::vector<hipr_surface>& targets, hipr_surface sur
   // counted form.
   int64_t most_total = 0;
   for (int32_t j : all) most_total += std::max<int64_t>(most_planes(j), 1);
-  const bool uncounted =
-      mode == 0 && !(opt && opt->band_rows != 0) && most_total <= kUncountedPlanes;
-  const bool counted = mode == 0 && !uncounted;
+  bool counted = mode == 0 && ((opt && opt->band_rows != 0) || most_total > kUncountedPlanes);
   std::vector<int32_t> small, wide;
   std::vector<int8_t> tier(nj, 1);  // waves (slots) of each job's walk
   for (int32_t j : all) {
@@ -1832,58 +1841,88 @@ hipr_result RunPasses(const std::vector<hipr_surface>& targets, hipr_surface sur
   }
   // Row bands: each job's rows are split into bands walked concurrently by
   // the write pass; the count or schedule pass records where they start.
-  int band_rows = opt && opt->band_rows != 0 ? std::max(opt->band_rows, 0)
-                  : counted                      ? kBandRowsExact
-                                                 : kBandRowsEstimates;
-  // Without a count pass banding costs a schedule pass, so only the paths
-  // with the widest active lists (the longest walks) are banded.
-  const bool own_split = mode != 0 && opt && opt->band_min_edges != 0;
-  const int band_min = counted     ? 0
-                       : own_split ? std::max(opt->band_min_edges, 0)
-                                   : kBandMinEdges;
-  // (default split only) paths this tall are banded too: at least
-  // kBandMinRows, and taller than the frame's rows spread over kBandSlots
-  // concurrent walks, so that only paths that would outlast the rest of the
-  // walk are split (a frame of many paths keeps its unbanded walks; one of a
-  // few large outlines bands them)
-  int band_min_rows = 0;
-  if (!counted && !own_split) {
-    int64_t total_rows = 0;
-    for (int32_t j : all) total_rows += spans[j].rows();
-    band_min_rows = (int)std::min<int64_t>(
-        std::max<int64_t>(kBandMinRows, total_rows / kBandSlots), INT32_MAX);
-    if (!(opt && opt->band_rows != 0) && total_rows / kBandSlots < kBandMinRows &&
-        f.stats.edges <= kBandShortEdges)
-      band_rows = kBandRowsShort;
-  }
   int32_t *const nbands = ht.band_count, *const pcap = ht.plane_cap;
-  std::fill_n(nbands, nj, 1);
-  std::fill_n(pcap, nj, 0);
-  std::fill_n(ht.plane_base, nj, 0);
-  std::fill_n(ht.q_base, nj, 0);
-  std::fill_n(ht.snap_base, nj, 0);
   int64_t q_total = 0, snap_total = 0;
-  for (int32_t j : all) {
-    // the 32- and 64-slot walks are unbanded
-    // a tall path is a long sequential walk too, whatever its list width
-    const bool tall = band_min_rows > 0 && spans[j].rows() >= band_min_rows;
-    nbands[j] = (bound[j] >= band_min || tall) && tier[j] <= 16
-                    ? BandCount(spans[j].pb, band_rows)
-                    : 1;
-    ht.q_base[j] = q_total;
-    q_total += (int64_t)nbands[j] * ctx->h_geo[j].edges;
-  }
   auto assign_snaps = [&](const std::vector<int32_t>& js) {
     for (int32_t j : js) {
       ht.snap_base[j] = snap_total;
       snap_total += (int64_t)(nbands[j] - 1) * SnapStride(tier[j] * kWave);
     }
   };
-  assign_snaps(all);
-  if (ctx->qstate.Ensure(sizeof(EdgeRec) * std::max<int64_t>(q_total, 1)) != hipSuccess ||
-      ctx->snaps.Ensure(std::max<int64_t>(snap_total, 1)) != hipSuccess ||
-      ctx->wcov.Ensure(sizeof(JobCov) * nj) != hipSuccess)
+  // Bands of `rows` rows for the paths whose list reaches min_edges or that
+  // span min_rows rows (0: no path by its rows), and room for their states.
+  auto assign_bands = [&](int rows, int min_edges, int min_rows) -> bool {
+    std::fill_n(nbands, nj, 1);
+    std::fill_n(pcap, nj, 0);
+    std::fill_n(ht.plane_base, nj, 0);
+    std::fill_n(ht.q_base, nj, 0);
+    std::fill_n(ht.snap_base, nj, 0);
+    q_total = snap_total = 0;
+    for (int32_t j : all) {
+      // the 32- and 64-slot walks are unbanded
+      // a tall path is a long sequential walk too, whatever its list width
+      const bool tall = min_rows > 0 && spans[j].rows() >= min_rows;
+      nbands[j] = (bound[j] >= min_edges || tall) && tier[j] <= 16 ? BandCount(spans[j].pb, rows)
+                                                                   : 1;
+      ht.q_base[j] = q_total;
+      q_total += (int64_t)nbands[j] * ctx->h_geo[j].edges;
+    }
+    assign_snaps(all);
+    return ctx->qstate.Ensure(sizeof(EdgeRec) * std::max<int64_t>(q_total, 1)) == hipSuccess &&
+           ctx->snaps.Ensure(std::max<int64_t>(snap_total, 1)) == hipSuccess;
+  };
+  auto plan_bands = [&]() -> bool {
+    int band_rows = opt && opt->band_rows != 0 ? std::max(opt->band_rows, 0)
+                    : counted                  ? kBandRowsExact
+                                               : kBandRowsEstimates;
+    // Without a count pass banding costs a schedule pass, so only the paths
+    // with the widest active lists (the longest walks) are banded.
+    const bool own_split = mode != 0 && opt && opt->band_min_edges != 0;
+    const int band_min = counted     ? 0
+                         : own_split ? std::max(opt->band_min_edges, 0)
+                                     : kBandMinEdges;
+    // (default split only) paths this tall are banded too: at least
+    // kBandMinRows, and taller than the frame's rows spread over kBandSlots
+    // concurrent walks, so that only paths that would outlast the rest of the
+    // walk are split (a frame of many paths keeps its unbanded walks; one of a
+    // few large outlines bands them)
+    int band_min_rows = 0;
+    if (!counted && !own_split) {
+      int64_t total_rows = 0;
+      for (int32_t j : all) total_rows += spans[j].rows();
+      band_min_rows = (int)std::min<int64_t>(
+          std::max<int64_t>(kBandMinRows, total_rows / kBandSlots), INT32_MAX);
+      if (!(opt && opt->band_rows != 0) && total_rows / kBandSlots < kBandMinRows &&
+          f.stats.edges <= kBandShortEdges)
+        band_rows = kBandRowsShort;
+    }
+    // One band per path holds one state an edge: the least that a walk takes.
+    return assign_bands(band_rows, band_min, band_min_rows) || assign_bands(0, 0, 0);
+  };
+  if (!plan_bands() || ctx->wcov.Ensure(sizeof(JobCov) * nj) != hipSuccess)
     return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
+  int64_t plane_total = 0;
+  auto assign_planes = [&](const std::vector<int32_t>& js) {
+    for (int32_t j : js) {
+      // the last chunk of each band may be left over in part
+      if (nbands[j] > 1) pcap[j] += nbands[j] * kPlaneChunk;
+      ht.plane_base[j] = plane_total;
+      plane_total += pcap[j];
+    }
+  };
+  auto plane_bytes = [](int64_t n) { return (size_t)kTilePlaneBytes * std::max<int64_t>(n, 1); };
+  if (mode == 0 && !counted) {
+    // Where the reservation cannot be had, the planes are counted after all:
+    // the frame uses only some of them.
+    for (int32_t j : all) pcap[j] = (int32_t)std::max<int64_t>(most_planes(j), 1);
+    test.assign(pcap, pcap + nj);
+    assign_planes(all);
+    if (ctx->planes.Ensure(plane_bytes(plane_total), plane_bytes(kUncountedPlanes)) != hipSuccess) {
+      counted = true;
+      plane_total = 0;
+      if (!plan_bands()) return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
+    }
+  }
   wp.qstate = ctx->qstate.as<EdgeRec>();
   wp.q_base = dt.q_base;
   wp.snaps = ctx->snaps.as<uint8_t>();
@@ -1894,22 +1933,6 @@ hipr_result RunPasses(const std::vector<hipr_surface>& targets, hipr_surface sur
     HIP_TRY(hipMemcpyAsync(ctx->tables.p, ctx->h_tables, JobTables::kBytes * nj,
                            hipMemcpyHostToDevice, st));
     return HIPR_SUCCESS;
-  };
-  int64_t plane_total = 0;
-  auto upload_planes = [&]() -> hipr_result {
-    if (plane_total >= kNoPlane) return HIPR_ERROR_CAPACITY;  // plane numbers are int32
-    if (ctx->planes.EnsureKeep((size_t)kTilePlaneBytes * std::max<int64_t>(plane_total, 1),
-                               ctx->planes.cap, st) != hipSuccess)
-      return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
-    return upload_tables();
-  };
-  auto assign_planes = [&](const std::vector<int32_t>& js) {
-    for (int32_t j : js) {
-      // the last chunk of each band may be left over in part
-      if (nbands[j] > 1) pcap[j] += nbands[j] * kPlaneChunk;
-      ht.plane_base[j] = plane_total;
-      plane_total += pcap[j];
-    }
   };
   auto read_cov = [&](DevBuf* src, JobCov* dst) -> hipr_result {
     HIP_TRY(hipMemcpyAsync(dst, src->p, sizeof(JobCov) * nj, hipMemcpyDeviceToHost, st));
@@ -2127,13 +2150,7 @@ hipr_result RunPasses(const std::vector<hipr_surface>& targets, hipr_surface sur
     return HIPR_SUCCESS;
   };
   JobCov* hw = ctx->h_wcov;
-  if (uncounted) {
-    test.resize(nj, 0);
-    for (int32_t j : all) {
-      pcap[j] = (int32_t)std::max<int64_t>(most_planes(j), 1);
-      test[j] = pcap[j];
-    }
-  } else if (counted) {
+  if (counted) {
     if ((r = upload_tables()) != HIPR_SUCCESS) return r;
     // count pass over every job (recording the band snapshots), then planes
     // sized exactly
@@ -2143,12 +2160,13 @@ hipr_result RunPasses(const std::vector<hipr_surface>& targets, hipr_surface sur
     if ((r = limit_error(ctx->h_cov, all, 16 | 32)) != HIPR_SUCCESS) return r;
     if ((r = move_overflowed(ctx->h_cov, nullptr)) != HIPR_SUCCESS) return r;
     for (int32_t j : all) pcap[j] = ctx->h_cov[j].planes;
-  } else {
+    assign_planes(all);
+  } else if (mode != 0) {
     // planes from the estimates, at most what the job can use
     for (int32_t j : all)
       pcap[j] = (int32_t)std::max<int64_t>(std::min<int64_t>(test[j], most_planes(j)), 1);
+    assign_planes(all);
   }
-  assign_planes(all);
   // Estimate modes: a shared pool after the estimated ranges serves the
   // planes of under-estimated jobs; only a job that finds the pool spent is
   // walked again.
@@ -2158,7 +2176,11 @@ hipr_result RunPasses(const std::vector<hipr_surface>& targets, hipr_surface sur
   if (ctx->pool_ctr.Ensure(sizeof(int32_t)) != hipSuccess ||
       ctx->counters.Ensure(kCounterWords * sizeof(unsigned long long)) != hipSuccess)
     return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
-  if ((r = upload_planes()) != HIPR_SUCCESS) return r;
+  if (plane_total >= kNoPlane) return HIPR_ERROR_CAPACITY;  // plane numbers are int32
+  // (nothing of an earlier draw's planes is kept)
+  if (ctx->planes.Ensure(plane_bytes(plane_total)) != hipSuccess)
+    return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
+  if ((r = upload_tables()) != HIPR_SUCCESS) return r;
   wp.pool_ctr = ctx->pool_ctr.as<int32_t>();
   wp.pool_base = (int32_t)pool_base;
   wp.pool_cap = (int32_t)pool_cap;
@@ -2231,9 +2253,13 @@ hipr_result RunPasses(const std::vector<hipr_surface>& targets, hipr_surface sur
       f.stats.fallbacks += (int64_t)(redo_small.size() + redo_wide.size());
       std::vector<int32_t> redo = redo_small;
       redo.insert(redo.end(), redo_wide.begin(), redo_wide.end());
+      const size_t written = plane_bytes(plane_total);
       for (int32_t j : redo) pcap[j] = hw[j].planes;
       assign_planes(redo);
-      if ((r = upload_planes()) != HIPR_SUCCESS) return r;
+      if (plane_total >= kNoPlane) return HIPR_ERROR_CAPACITY;
+      if (ctx->planes.EnsureKeep(plane_bytes(plane_total), written, st) != hipSuccess)
+        return HIPR_ERROR_OUT_OF_DEVICE_MEMORY;
+      if ((r = upload_tables()) != HIPR_SUCCESS) return r;
       wp.planes = ctx->planes.as<uint8_t>();
       if ((r = prepare_write(&redo)) != HIPR_SUCCESS) return r;
       if ((r = walk_pass(kWalkWrite, redo_small, redo_wide)) != HIPR_SUCCESS) return r;

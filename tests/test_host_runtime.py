@@ -4,6 +4,7 @@ and allocations: what a draw leaves behind when one of its steps fails."""
 import ctypes
 import glob
 import os
+import re
 import subprocess
 
 import numpy as np
@@ -73,8 +74,10 @@ class Frame:
     def kernels(self):
         return self.L.test_log().decode().split()
 
-    def draw(self, **kw):
+    def draw(self, limit=-1, **kw):
+        """The kernels of a draw that may allocate `limit` bytes at a time."""
         self.L.test_reset()
+        self.L.test_limit_malloc(limit)
         self.surf.draw(self.prep, **kw)
         return self.kernels()
 
@@ -115,3 +118,62 @@ def test_a_plan_that_fails_leaves_nothing_running(runtime, kw):
         assert runtime.test_unfinished() == 0, at
         assert f.draw(**kw) == names
     f.close()
+
+
+COUNT, WRITE, SCHEDULE = "0", "1", "2"
+
+
+def walk_modes(names):
+    return {m.group(1) for m in (re.search(r"WalkKernelILi\d+ELi(\d)E", k) for k in names) if m}
+
+
+def test_planes_are_counted_where_they_cannot_be_reserved(runtime):
+    """64 draws over all of 2048 x 2048 could use 512 MiB of planes.  An exact
+    draw that cannot reserve them counts them, as one with bands of its own
+    does, and reserves them again once it can."""
+    f = Frame(runtime, 2048, 64, [(0, 0, 2048, 2048)], [50], [40])
+    assert walk_modes(f.draw(limit=64 << 20)) == {COUNT, WRITE}
+    assert COUNT not in walk_modes(f.draw())
+    assert COUNT not in walk_modes(f.draw(limit=64 << 20))  # kept from the last draw
+    assert runtime.test_copied() == 0
+    f.close()
+
+
+def test_bands_are_given_up_where_their_states_cannot_be_reserved(runtime):
+    """Two draws of 4,000 edges and 32 bands hold 16 MiB of edge states, and
+    512 KiB without bands."""
+    f = Frame(runtime, 2048, 2, [(0, 0, 64, 1900)], [4000], [40])
+    assert walk_modes(f.draw(limit=8 << 20)) == {WRITE}
+    assert walk_modes(f.draw()) == {SCHEDULE, WRITE}
+    f.close()
+
+
+@pytest.mark.parametrize("mode", [abi.MODE_EXACT, abi.MODE_LEARNED])
+def test_a_draw_without_memory_is_refused_alone(runtime, mode):
+    """Whatever allocation is refused, the draw says so, and the next one is
+    not told of it."""
+    f = tiers(runtime)
+    names = f.draw(mode=mode)
+    f.close()
+    for limit in (100, 4 << 10, 16 << 10, 64 << 10, 256 << 10):
+        f = tiers(runtime)
+        with pytest.raises(device.HiprError) as e:
+            f.draw(limit=limit, mode=mode)
+        assert e.value.code == ERROR_OUT_OF_DEVICE_MEMORY, limit
+        assert runtime.test_unfinished() == 0
+        assert f.draw(mode=mode) == names
+        f.close()
+
+
+def test_growing_planes_are_not_copied(runtime):
+    """A larger frame on the same context takes larger planes; nothing of the
+    last frame's is kept."""
+    small = Frame(runtime, 2048, 4, [(0, 0, 300, 300)], [50], [40])
+    for mode in (abi.MODE_EXACT, abi.MODE_LEARNED):
+        for side in (300, 900, 2000):
+            runtime.test_set_frame(1, *(x.ctypes.data_as(ctypes.c_void_p) for x in (
+                np.array([0, 0, side, side], np.float32), np.array([50], np.int32),
+                np.array([40], np.int32))))
+            small.draw(mode=mode)
+            assert runtime.test_copied() == 0, (mode, side)
+    small.close()
