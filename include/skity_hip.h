@@ -449,14 +449,17 @@ HIPR_API hipr_result hipr_batch_add(hipr_batch batch, hipr_surface surface,
                                     hipr_prepared scene);
 HIPR_API hipr_result hipr_batch_clear(hipr_batch batch);
 HIPR_API hipr_result hipr_batch_draw(hipr_batch batch, const hipr_options* options);
-/* The work split used when options leave band_rows / band_min_edges /
- * flags at 0. */
+/* The work split used, in every mode, when options leave band_rows /
+ * band_min_edges / flags at 0. */
 HIPR_API hipr_result hipr_batch_set_split(hipr_batch batch, int32_t band_rows,
                                           int32_t band_min_edges, int32_t flags);
-/* Autotuner: draws the batch with each candidate work split (rows per walk
- * band, banded paths, persistent or dispatched walk kernels) in `mode`
- * (EXACT or LEARNED), keeps the fastest by device time and returns it.  The
- * targets' contents are left undefined (clear them before drawing). */
+/* Autotuner: draws the batch with the library's default work split (returned
+ * as 0, 0, 0) and with each other candidate (rows per walk band, banded paths,
+ * persistent or dispatched walk kernels; EXACT: other bands only where the
+ * default counts its planes) in `mode` (EXACT or LEARNED), keeps the fastest by
+ * device time and returns it.  A split found in EXACT mode is used by exact
+ * draws, one found in LEARNED mode by learned and estimate draws.  The targets'
+ * contents are left undefined (clear them before drawing). */
 HIPR_API hipr_result hipr_batch_autotune(hipr_batch batch, int32_t mode, int32_t repeats,
                                          int32_t* out_band_rows,
                                          int32_t* out_band_min_edges, int32_t* out_flags);

@@ -440,6 +440,9 @@ struct hipr_prepared_s {
   }
 };
 
+// The forms that a batch's work split is used in.
+enum TunedFor { kTunedForAll, kTunedForExact, kTunedForEstimates };
+
 // Many (surface, prepared scene) pairs drawn by one pipeline run: the plans
 // are merged into one (`merged`), whose canvases [0, pairs) are the pairs'
 // surfaces and whose jobs are the pairs' jobs in pair order.
@@ -451,6 +454,7 @@ struct hipr_batch_s {
   hipr_surface_s sink;      // statistics of the last draw (no pixels)
   int32_t tuned_band_rows = 0, tuned_band_min_edges = 0;  // 0: library defaults
   int32_t tuned_flags = 0;
+  TunedFor tuned_for = kTunedForAll;
 };
 
 namespace {
@@ -3469,9 +3473,12 @@ HIPR_API hipr_result hipr_batch_draw(hipr_batch b, const hipr_options* options) 
   if (b->dirty && (r = MergeBatch(b)) != HIPR_SUCCESS) return r;
   hipr_options opt{};
   if (options) opt = *options;
-  if (opt.band_rows == 0) opt.band_rows = b->tuned_band_rows;
-  if (opt.band_min_edges == 0) opt.band_min_edges = b->tuned_band_min_edges;
-  if (opt.flags == 0) opt.flags = b->tuned_flags;
+  if (b->tuned_for == kTunedForAll ||
+      b->tuned_for == (opt.mode == HIPR_MODE_EXACT ? kTunedForExact : kTunedForEstimates)) {
+    if (opt.band_rows == 0) opt.band_rows = b->tuned_band_rows;
+    if (opt.band_min_edges == 0) opt.band_min_edges = b->tuned_band_min_edges;
+    if (opt.flags == 0) opt.flags = b->tuned_flags;
+  }
   std::vector<hipr_surface> targets;
   for (const auto& pr : b->pairs) targets.push_back(pr.first);
   return RunPlan(targets, &b->sink, &b->merged, &opt);
@@ -3480,6 +3487,7 @@ HIPR_API hipr_result hipr_batch_draw(hipr_batch b, const hipr_options* options) 
 HIPR_API hipr_result hipr_batch_set_split(hipr_batch b, int32_t band_rows, int32_t band_min_edges,
                                           int32_t flags) {
   if (!b) return HIPR_ERROR_INVALID_HANDLE;
+  b->tuned_for = kTunedForAll;
   b->tuned_band_rows = band_rows;
   b->tuned_band_min_edges = band_min_edges;
   b->tuned_flags = flags;
@@ -3494,27 +3502,16 @@ HIPR_API hipr_result hipr_batch_autotune(hipr_batch b, int32_t mode, int32_t rep
       mode == HIPR_MODE_ESTIMATES)
     return HIPR_ERROR_INVALID_ARGUMENT;
   if (b->pairs.empty()) return HIPR_SUCCESS;
-  // Work splits: rows per walk band, and (estimate modes) which paths are
-  // banded.  Each candidate is drawn once to warm up, then `repeats` times;
-  // the device time of its fastest draw decides.
-  const int32_t rows[] = {-1, 64, 128, 256};
-  const int32_t mins[] = {INT32_MAX, 4 * kWave + 1, 3 * kWave + 1, 2 * kWave + 1, -1};
+  // Work splits: the default, then rows per walk band and (estimate modes)
+  // which paths are banded.  Each candidate is drawn once to warm up, then
+  // `repeats` times; the device time of its fastest draw decides.
   struct Cand {
     int32_t rows, min_edges, flags;
   };
-  std::vector<Cand> cands;
-  for (int32_t f : {0, (int32_t)HIPR_FLAG_PERSISTENT}) {
-    for (int32_t r : rows) {
-      if (mode == HIPR_MODE_EXACT || r < 0) {
-        cands.push_back({r, 0, f});
-      } else {
-        for (int32_t m : mins) cands.push_back({r, m, f});
-      }
-    }
-  }
+  b->tuned_band_rows = b->tuned_band_min_edges = b->tuned_flags = 0;
   double best_ms = 1e30;
-  Cand best = cands[0];
-  for (const Cand& c : cands) {
+  Cand best{0, 0, 0};
+  auto time = [&](const Cand& c) -> hipr_result {
     hipr_options opt{};
     opt.mode = mode;
     opt.band_rows = c.rows;
@@ -3530,7 +3527,31 @@ HIPR_API hipr_result hipr_batch_autotune(hipr_batch b, int32_t mode, int32_t rep
       best_ms = t;
       best = c;
     }
+    return HIPR_SUCCESS;
+  };
+  hipr_result r;
+  if ((r = time({0, 0, 0})) != HIPR_SUCCESS) return r;
+  // An exact draw with bands of its own counts its planes, a second walk, so
+  // the other splits are tried only where the default counts them as well (256
+  // draws on 16 uneven canvases of 256 to 4096 pixels: 46.0 ms by the default,
+  // 101.8 to 194.0 by the others; 741 draws, counted: 143.8 and 144.0 to 254.5).
+  const bool splits =
+      mode != HIPR_MODE_EXACT || b->sink.stage_launches[HIPR_STAGE_WALK_COUNT] > 0;
+  const int32_t mins[] = {INT32_MAX, 4 * kWave + 1, 3 * kWave + 1, 2 * kWave + 1, -1};
+  for (int32_t f : {0, (int32_t)HIPR_FLAG_PERSISTENT}) {
+    if (f != 0 && (r = time({0, 0, f})) != HIPR_SUCCESS) return r;
+    if (!splits) continue;
+    for (int32_t rows : {-1, 64, 128, 256}) {
+      if (mode == HIPR_MODE_EXACT && rows == kBandRowsExact) continue;  // the default
+      if (mode == HIPR_MODE_EXACT || rows < 0) {
+        if ((r = time({rows, 0, f})) != HIPR_SUCCESS) return r;
+      } else {
+        for (int32_t m : mins)
+          if ((r = time({rows, m, f})) != HIPR_SUCCESS) return r;
+      }
+    }
   }
+  b->tuned_for = mode == HIPR_MODE_EXACT ? kTunedForExact : kTunedForEstimates;
   b->tuned_band_rows = best.rows;
   b->tuned_band_min_edges = best.min_edges;
   b->tuned_flags = best.flags;

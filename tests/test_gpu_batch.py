@@ -111,6 +111,32 @@ def test_batch_learned_and_autotuned_equal_exact(ctx):
         p.close()
 
 
+def test_tuned_exact_batch(ctx):
+    """A batch tuned for exact draws keeps the form that does not count its
+    planes, and its pixels."""
+    scs = uneven_scenes(6, 820, max_paths=40)
+    preps = [device.Prepared(ctx, sc.scene) for sc in scs]
+    surfs = [device.Surface(ctx, sc.width, sc.height) for sc in scs]
+    b = device.Batch(ctx)
+    for s, p in zip(surfs, preps):
+        b.add(s, p)
+    b.draw()
+    assert b.stage_times()["walk_count"][1] == 0
+    want = [s.read() for s in surfs]
+    split = b.autotune(abi.MODE_EXACT, repeats=1)
+    print("tuned split", split, flush=True)
+    assert split[:2] == (0, 0)
+    for s in surfs:
+        s.clear(0)
+    b.draw()
+    assert b.stage_times()["walk_count"][1] == 0
+    for s, w in zip(surfs, want):
+        assert np.array_equal(s.read(), w)
+    b.close()
+    for x in surfs + preps:
+        x.close()
+
+
 def test_batch_rejects_a_surface_twice(ctx):
     sc = scenes.generate(1, seed=3)
     p = device.Prepared(ctx, sc.scene)

@@ -177,3 +177,66 @@ def test_growing_planes_are_not_copied(runtime):
             small.draw(mode=mode)
             assert runtime.test_copied() == 0, (mode, side)
     small.close()
+
+
+def batch_of(f):
+    b = device.Batch(f.ctx)
+    b.add(f.surf, f.prep)
+    return b
+
+
+def batch_draw(f, b, **kw):
+    f.L.test_reset()
+    b.draw(**kw)
+    return f.kernels()
+
+
+def test_the_default_split_is_tried_first(runtime):
+    """Device time is the number of kernels here.  The exact form is fastest
+    without a count pass, which every other split asks for; where nothing is
+    banded all splits tie, and the default, the first, is kept."""
+    f = tiers(runtime)
+    b = batch_of(f)
+    names = batch_draw(f, b)
+    assert b.autotune(abi.MODE_EXACT, repeats=1) == (0, 0, 0)
+    assert batch_draw(f, b) == names
+    b.close()
+    f.close()
+    f = Frame(runtime, 256, 4, [(0, 0, 90, 90)], [50], [40])
+    b = batch_of(f)
+    for mode in (abi.MODE_EXACT, abi.MODE_LEARNED):
+        assert b.autotune(mode, repeats=1) == (0, 0, 0)
+    b.close()
+    f.close()
+
+
+def test_splits_are_tried_where_planes_are_counted(runtime):
+    """More planes than are ever reserved: the default counts them too, and one
+    band per path saves nothing but may be chosen."""
+    f = Frame(runtime, 2048, 520, [(0, 0, 2048, 2048)], [50], [40])
+    b = batch_of(f)
+    assert COUNT in walk_modes(batch_draw(f, b))
+    runtime.test_reset()
+    assert b.autotune(abi.MODE_EXACT, repeats=1) == (0, 0, 0)
+    draws = sum("JobTileRangeKernel" in k for k in f.kernels())
+    assert draws >= 2 * 2 * 4  # two draws each of four splits, launched in two ways
+    b.close()
+    f.close()
+
+
+def test_a_split_is_used_by_the_form_it_was_tuned_for(runtime):
+    """A split tuned for learned draws would make exact ones count.  Tuning
+    again does not start from the split found before."""
+    f = tiers(runtime)
+    b = batch_of(f)
+    exact = batch_draw(f, b)
+    split = b.autotune(abi.MODE_LEARNED, repeats=1)
+    assert split[0] < 0  # no schedule pass: the fewest kernels
+    tuned = batch_draw(f, b, mode=abi.MODE_LEARNED)
+    assert walk_modes(tuned) == {WRITE}
+    assert batch_draw(f, b) == exact
+    assert b.autotune(abi.MODE_LEARNED, repeats=1) == split
+    b.set_split(64, 0)  # a caller's own split holds for every form
+    assert COUNT in walk_modes(batch_draw(f, b))
+    b.close()
+    f.close()
