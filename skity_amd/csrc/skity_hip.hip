@@ -1226,18 +1226,19 @@ constexpr int64_t kTeamWaves = 1024;
 
 // Launches `kernel` (a slot walk, or a team of `waves` waves) over P's items.
 hipr_result LaunchWalk(hipr_context ctx, void (*kernel)(WalkParams), int waves, size_t lds,
-                       int stage, WalkParams P, hipStream_t st, bool timed, int32_t* queue,
-                       double share) {
+                       int stage, WalkParams P, hipStream_t st, bool timed, int32_t* queue) {
   if (P.n_walk == 0) return HIPR_SUCCESS;
   unsigned grid = (unsigned)P.n_walk;
   P.queue = queue;
   if (queue) {
-    // persistent form: as many workgroups as fit at once (this tier's share)
+    // persistent form: as many workgroups as fit at once.  (Kernels beside it
+    // take their places as its workgroups end.  With the tier's share of the
+    // frame's work, a pass of few long items and one of many short ones got too
+    // few: 741 learned draws on 16 uneven canvases 135 ms, and 58.9 by this.)
     int per_cu = 0;
     HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)kernel,
                                                          waves * kWave, lds));
     int64_t cap = (int64_t)std::max(per_cu, 1) * std::max(ctx->n_cus, 1);
-    cap = std::max<int64_t>(1, (int64_t)((double)cap * share));
     grid = (unsigned)std::min<int64_t>(P.n_walk, cap);
   }
   hipEvent_t b = timed ? StageBegin(ctx, st) : nullptr;
@@ -1298,13 +1299,13 @@ hipr_result TierLdsCheck(hipr_context ctx, int tier, int mode, int lds_width, in
                       ShapeLdsBytes(ShapeOf(tier, mode, items), tier, lds_width, row_ints));
 }
 hipr_result LaunchTier(hipr_context ctx, int tier, int mode, const WalkParams& P, hipStream_t st,
-                       bool timed, int32_t* queue, double share) {
+                       bool timed, int32_t* queue) {
   const WalkShape w = ShapeOf(tier, mode, P.n_walk);
   const size_t lds = ShapeLdsBytes(w, tier, P.lds_width, P.row_ints);
   const int stage = mode == kWalkCount   ? HIPR_STAGE_WALK_COUNT
                     : mode == kWalkWrite ? HIPR_STAGE_WALK
                                          : HIPR_STAGE_WALK_SCHEDULE;
-  return LaunchWalk(ctx, w.kernel, w.waves, lds, stage, P, st, timed, queue, share);
+  return LaunchWalk(ctx, w.kernel, w.waves, lds, stage, P, st, timed, queue);
 }
 
 // The 32- and 64-slot walks (hipr_walk_wide.hip): one wave per job, never
@@ -1995,19 +1996,10 @@ hipr_result RunPasses(const std::vector<hipr_surface>& targets, hipr_surface sur
     hipr_result rr;
     std::vector<int32_t> all_items;
     std::vector<size_t> off, cnt;
-    std::vector<double> work;
-    double work_all = 0;
     for (const WalkLaunch& l : plan) {
       off.push_back(all_items.size());
       make_items(*l.jobs, l.kmode, &all_items);
       cnt.push_back(all_items.size() - off.back());
-      double w = 0;
-      if (persistent) {
-        for (int32_t j : *l.jobs)
-          w += (double)std::max(bound[j], 1) * std::max(spans[j].rows(), 1);
-      }
-      work.push_back(w);
-      work_all += w;
       if (cnt.back() && (rr = TierLdsCheck(ctx, l.K, l.kmode, wp.lds_width, wp.row_ints,
                                            (int64_t)cnt.back())) != HIPR_SUCCESS)
         return rr;
@@ -2056,11 +2048,10 @@ hipr_result RunPasses(const std::vector<hipr_surface>& targets, hipr_surface sur
       wpl.n_walk = (int32_t)cnt[i];
       wpl.cov = l.kmode == kWalkWrite ? ctx->wcov.as<JobCov>() : ctx->cov.as<JobCov>();
       int32_t* qi = q ? q + i : nullptr;
-      double share = work_all > 0 ? work[i] / work_all : 1.0;
       const int sk = stream_of(i);
       hipStream_t ls = sk == 0 ? st : ctx->side[sk - 1];
       hipr_result lr;
-      lr = l.K <= kMaxTeam ? LaunchTier(ctx, l.K, l.kmode, wpl, ls, timed, qi, share)
+      lr = l.K <= kMaxTeam ? LaunchTier(ctx, l.K, l.kmode, wpl, ls, timed, qi)
                            : LaunchWalkWide(ctx, l.K, l.kmode, wpl, ls, timed);
       if (lr != HIPR_SUCCESS) return lr;
     }

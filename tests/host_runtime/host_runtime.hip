@@ -3,7 +3,7 @@
 // Linked with the objects of libskity_hip.so in place of the real runtime, it
 // runs no kernel.  It keeps, for every stream, how many kernels were launched
 // on it and up to which one the host has waited (through stream and event
-// waits, also of other streams), logs the kernels' names in launch order, and
+// waits, also of other streams), logs the kernels' names and grids in launch order, and
 // refuses allocations and launches on request, with the error left behind as
 // the real runtime leaves it.  The two kernels whose results steer the host,
 // the flatten (bounds and edge counts) and the sort (active-edge bounds), write
@@ -145,13 +145,14 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipSt
   *stream = c.stream;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t stream) {
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void** args, size_t,
+                           hipStream_t stream) {
   const std::string& name = Names()[f];
   if (g_fail_at >= 0 && name.find(g_fail_name) != std::string::npos && g_fail_at-- == 0)
     return Fail(hipErrorLaunchFailure);
   Stream* s = (Stream*)stream;
   s->known[s->id] = ++g_launched[s->id];
-  g_log += name + "\n";
+  g_log += name + " " + std::to_string(grid.x) + "\n";
   g_ms += 1;
   if (name.find("FlattenKernel") != std::string::npos) Flatten(args);
   if (name.find("SortGatherKernel") != std::string::npos) Sort(args);

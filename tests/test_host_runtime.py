@@ -72,7 +72,7 @@ class Frame:
         self.prep = device.Prepared(self.ctx, self.scene.scene)
 
     def kernels(self):
-        return self.L.test_log().decode().split()
+        return self.L.test_log().decode().splitlines()
 
     def draw(self, limit=-1, **kw):
         """The kernels of a draw that may allocate `limit` bytes at a time."""
@@ -239,4 +239,23 @@ def test_a_split_is_used_by_the_form_it_was_tuned_for(runtime):
     b.set_split(64, 0)  # a caller's own split holds for every form
     assert COUNT in walk_modes(batch_draw(f, b))
     b.close()
+    f.close()
+
+
+@pytest.mark.parametrize("mode", [abi.MODE_EXACT, abi.MODE_LEARNED])
+def test_persistent_walks_fill_the_device(runtime, mode):
+    """Every walk of the persistent form has a workgroup per item, up to the
+    2,048 that fit the device at once here, whatever the frame's other walks."""
+    def grids(names):
+        return [int(k.split()[1]) for k in names if "WalkKernel" in k]
+
+    f = Frame(runtime, 2048, 300, [(0, 0, 300, 1900)] * 2 + [(9, 9, 90, 50)] * 3,
+              [300] * 5, [40, 300, 20, 100, 600])
+    plain = grids(f.draw(mode=mode))
+    assert len(plain) >= 5 and max(plain) < 2048
+    assert grids(f.draw(mode=mode, flags=abi.FLAG_PERSISTENT)) == plain
+    f.close()
+    f = Frame(runtime, 2048, 3000, [(9, 9, 90, 50)], [300], [20])
+    assert grids(f.draw(mode=mode)) == [3000]
+    assert grids(f.draw(mode=mode, flags=abi.FLAG_PERSISTENT)) == [2048]
     f.close()
