@@ -3,11 +3,12 @@
 // Linked with the objects of libskity_hip.so in place of the real runtime, it
 // runs no kernel.  It keeps, for every stream, how many kernels were launched
 // on it and up to which one the host has waited (through stream and event
-// waits, also of other streams), logs the kernels' names and grids in launch order, and
-// refuses allocations and launches on request, with the error left behind as
-// the real runtime leaves it.  The two kernels whose results steer the host,
-// the flatten (bounds and edge counts) and the sort (active-edge bounds), write
-// what the test set for the frame.  Device time is one millisecond per kernel.
+// waits, also of other streams), logs the kernels' names, grids and hardware
+// queues (streams take them in turn) in launch order, and refuses allocations
+// and launches on request, with the error left behind as the real runtime
+// leaves it.  The two kernels whose results steer the host, the flatten (bounds
+// and edge counts) and the sort (active-edge bounds), write what the test set
+// for the frame.  Device time is one millisecond per kernel.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -44,6 +45,7 @@ std::map<const void*, std::string>& Names() {
 std::vector<Config> g_config;
 Clock g_launched, g_done;
 int g_streams = 0;
+constexpr int kQueues = 4;
 double g_ms = 0;
 hipError_t g_error = hipSuccess;
 std::string g_log;
@@ -152,7 +154,7 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void** args, size_t,
     return Fail(hipErrorLaunchFailure);
   Stream* s = (Stream*)stream;
   s->known[s->id] = ++g_launched[s->id];
-  g_log += name + " " + std::to_string(grid.x) + "\n";
+  g_log += name + " " + std::to_string(grid.x) + " " + std::to_string(s->id % kQueues) + "\n";
   g_ms += 1;
   if (name.find("FlattenKernel") != std::string::npos) Flatten(args);
   if (name.find("SortGatherKernel") != std::string::npos) Sort(args);

@@ -71,8 +71,15 @@ class Frame:
         self.surf = device.Surface(self.ctx, side, side)
         self.prep = device.Prepared(self.ctx, self.scene.scene)
 
-    def kernels(self):
+    def launches(self):
         return self.L.test_log().decode().splitlines()
+
+    def kernels(self):
+        """Names and grids, in launch order."""
+        return [k.rsplit(" ", 1)[0] for k in self.launches()]
+
+    def queues(self):
+        return {int(k.rsplit(" ", 1)[1]) for k in self.launches()}
 
     def draw(self, limit=-1, **kw):
         """The kernels of a draw that may allocate `limit` bytes at a time."""
@@ -259,3 +266,16 @@ def test_persistent_walks_fill_the_device(runtime, mode):
     assert grids(f.draw(mode=mode)) == [3000]
     assert grids(f.draw(mode=mode, flags=abi.FLAG_PERSISTENT)) == [2048]
     f.close()
+
+
+def test_contexts_take_different_queues(runtime):
+    """Frames of one walk kernel run on their context's main stream alone; four
+    contexts use the four hardware queues."""
+    frames = [Frame(runtime, 256, 4, [(0, 0, 90, 90)], [50], [40]) for _ in range(4)]
+    used = []
+    for f in frames:
+        f.draw()
+        used.append(f.queues())
+        f.close()
+    assert all(len(q) == 1 for q in used)
+    assert set.union(*used) == {0, 1, 2, 3}
