@@ -810,8 +810,9 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
           nM = __builtin_amdgcn_ds_permute(4 * r, nM);
         }
       }
-      const int mn = DppWaveMin(mine && (!initial || nLY > y) ? nLY : kMaxS32);
-      min_ly = Min32(min_ly, mn);
+      const int least = DppWaveMin(mine ? nLY : kMaxS32);
+      min_ly = Min32(min_ly, least);
+      const int mn = initial ? DppWaveMin(mine && nLY > y ? nLY : kMaxS32) : least;
       // insertion positions: P0 = #{a : x_a <= x_N0};
       // Pi = max(P(i-1), #{a : x_a < x_Ni}); list element q moves to
       // q + #{i : Pi <= q}, new edge i goes to Pi + i
@@ -923,7 +924,7 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
     int rk[K];
     Fixed nX[K], nDX[K], nDY[K], nLY[K];
     int nM[K];
-    int mn = kMaxS32;
+    int mn = kMaxS32, least = kMaxS32;
 #pragma unroll
     for (int s = 0; s < K; s++) {
       const int p = s * kWave + lane;
@@ -941,11 +942,12 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
         nDY[s] = L.sDY[p];
         nLY[s] = L.sLY[p];
         nM[s] = L.sM[p];
+        least = Min32(least, nLY[s]);
         if (!initial || nLY[s] > y) mn = Min32(mn, nLY[s]);
       }
     }
     mn = DppWaveMin(mn);
-    min_ly = Min32(min_ly, mn);
+    min_ly = Min32(min_ly, DppWaveMin(least));
     WaveSync();
 #pragma unroll
     for (int s = 0; s < K; s++) {
@@ -1126,9 +1128,12 @@ __device__ __forceinline__ void WalkItem(const WalkParams& P, int wi, int32_t* l
     // or together linearly, so a list in order now and after `rows` rows is in
     // order on all rows between, and the steps up to there are taken as one.
     // A list of few edges, most of them, takes 16 rows (a band, as many delta
-    // rows as fit) in little more than the time of one.
+    // rows as fit) in little more than the time of one.  (The first row may hold
+    // edges that have ended before it: a tall quad whose first piece runs
+    // upward, by the rounding of its forward differences.  They take this row's
+    // step and go on or end after it.)
     int rows = 1;
-    if ((y & 0xFFFF) == 0) {
+    if ((y & 0xFFFF) == 0 && min_ly > y) {
       int most = Min32((nny - 1) >> 16, stop_fixed >> 16) - row;
       if (kWrite && stop_y != kMaxS32) most = Min32(most, (stop_y >> 16) - row);
       if (!kWrite && next_b < nb) {

@@ -629,7 +629,7 @@ __device__ __forceinline__ void TeamWalkItem(const WalkParams& P, int wi, int32_
       }
     }
     if (n + k > CAP) return false;
-    int mn, shift = 0;
+    int mn, least, shift = 0;  // smallest lower_y after y, and of all
     bool crosses = false;
     if (k <= kTile) {
       // a few: lane i of every wave takes new edge i
@@ -660,7 +660,8 @@ __device__ __forceinline__ void TeamWalkItem(const WalkParams& P, int wi, int32_
           nM = __builtin_amdgcn_ds_permute(4 * r, nM);
         }
       }
-      mn = DppWaveMin(mine && (!initial || nLY > y) ? nLY : kMaxS32);
+      least = DppWaveMin(mine ? nLY : kMaxS32);
+      mn = initial ? DppWaveMin(mine && nLY > y ? nLY : kMaxS32) : least;
       int cnt = 0;
       if (n > 0) {
         for (int i = 0; i < k; i++) {
@@ -723,7 +724,8 @@ __device__ __forceinline__ void TeamWalkItem(const WalkParams& P, int wi, int32_
         wide[me] = X;
         wide[CAP + me] = X + DX;
       }
-      mn = DppWaveMin(mine && (!initial || nLY > y) ? nLY : kMaxS32);
+      least = DppWaveMin(mine ? nLY : kMaxS32);
+      mn = initial ? DppWaveMin(mine && nLY > y ? nLY : kMaxS32) : least;
       sync();
       int r = 0;
       for (int q = 0; q < k; q++) {
@@ -765,11 +767,12 @@ __device__ __forceinline__ void TeamWalkItem(const WalkParams& P, int wi, int32_
         }
         shift = 1 + c;
       }
-      const Share s = share(make_int4(__ballot(f) != 0 ? 1 : 0, mn, 0, 0),
+      const Share s = share(make_int4(__ballot(f) != 0 ? 1 : 0, mn, least, 0),
                             make_int4(0, 0, 0, 0), false);
       if (NW == 1) sync();
       crosses = __ballot(mate && s.a.x != 0) != 0;
       mn = DppWaveMin(mate ? s.a.y : kMaxS32);
+      least = DppWaveMin(mate ? s.a.z : kMaxS32);
       if (me < n) store_fields(me + shift);
       if (mine) {
         const int c = pos + r;
@@ -785,7 +788,7 @@ __device__ __forceinline__ void TeamWalkItem(const WalkParams& P, int wi, int32_
     pp += k;
     if (me < n) load_fields(me);
     if (!initial && crosses) nny = y + (kFixed1 >> kAcc);
-    min_ly = Min32(min_ly, mn);
+    min_ly = Min32(min_ly, least);
     if (mn > y && mn < nny) nny = mn;
     sync();
     relink();
@@ -882,9 +885,10 @@ __device__ __forceinline__ void TeamWalkItem(const WalkParams& P, int wi, int32_
     // or together linearly, so a list in order now and after `rows` rows is in
     // order on all rows between, and the steps up to there are taken as one.
     // A list of few edges takes 16 rows (a band, as many delta rows as fit)
-    // in little more than the time of one.
+    // in little more than the time of one.  (Not where edges have ended before
+    // the first row, see hipr_walk.hpp.)
     int rows = 1;
-    if ((y & 0xFFFF) == 0) {
+    if ((y & 0xFFFF) == 0 && min_ly > y) {
       int most = Min32((nny - 1) >> 16, stop_fixed >> 16) - row;
       if (kWrite && stop_y != kMaxS32) most = Min32(most, (stop_y >> 16) - row);
       if (!kWrite && next_b < nb) {

@@ -174,3 +174,25 @@ def test_runs_of_lines(ctx, join):
             p.line_to(x, y)
         c.draw_path(p.close() if i % 4 == 1 else p, paint)
     check(ctx, c.scene(), f"join {join}")
+
+
+@pytest.mark.parametrize("bars", [0, 31, 150])
+def test_quads_that_end_above_their_first_row(ctx, bars):
+    """Quads over more than 8,192 rows, whose forward differences wrap as the
+    reference's do: their first pieces run upward, so that the first row holds
+    edges that have ended before it.  They take that row's step and then go on;
+    rows are taken several at a time only after that.  With bars beside them the
+    lists are of 64 and of 302 edges."""
+    rng = np.random.default_rng(4)
+    n = 40
+    c = Canvas(10 * n + 4 * bars, 300)
+    for i in range(n):
+        x = 10 * i + rng.uniform(-60, 60, 4)
+        top = -float(np.floor(rng.uniform(300, 600)))
+        y = np.sort(rng.uniform(7700, 8100, 2))
+        p = Path().move_to(x[0], top).quad_to(x[1], y[0], x[2], y[1]).line_to(x[3], top).close()
+        for k in range(bars):
+            p.add_rect(10 * n + 60 + 4 * k, top, 10 * n + 62.5 + 4 * k, 8000)
+        p.fill_type = abi.FILL_EVEN_ODD
+        c.draw_path(p, Paint((0.1 + 0.02 * i, 0.9 - 0.02 * i, 0.4, 1.0)))
+    check(ctx, c.scene(), "tall quads")
