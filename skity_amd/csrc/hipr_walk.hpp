@@ -69,7 +69,7 @@ __host__ __device__ inline int64_t SnapStride(int cap) {
 
 struct WalkParams {
   const Job* jobs;
-  const int32_t* walk_list;  // work items: job << 4 | band
+  const int32_t* walk_list;  // work items: job << kBandBits | band
   int32_t n_walk;
   const JobGeo* geo;
   const int64_t* edge_base;

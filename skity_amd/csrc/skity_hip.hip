@@ -1807,12 +1807,12 @@ hipr_result RunPasses(const std::vector<hipr_surface>& targets, hipr_surface sur
   wp.row_ints = WalkRowCapacity(ctx, lds_width, nwalk);
   wp.map_base = dt.map_base;
   // ---- stage (b): walk ----
-  // The walk keeps the active edge list in registers, one element per lane.
-  // The sort bounded each job's list by its largest row overlap: a job takes
-  // a team of one wave per 64 edges of its bound (1, 2, 4, 8 or 16 waves), and
-  // the rare list of more than 1,024 edges the unbanded 32- or 64-slot walk of
-  // one wave (2,048 and 4,096 edges).  A longer list is refused
-  // (HIPR_ERROR_CAPACITY).
+  // The walk keeps the active edge list in registers, one element per lane and
+  // slot.  The sort bounded each job's list by its largest row overlap: a job's
+  // tier is the number of slots (or, in a team, waves) of 64 edges that hold it,
+  // 1 to 16 (ShapeOf), and for the rare list of more than 1,024 edges the
+  // unbanded 32- or 64-slot walk (2,048 and 4,096 edges).  A longer list is
+  // refused (HIPR_ERROR_CAPACITY).
   const int32_t* bound = ctx->h_bound;  // of the walked jobs
   HIP_TRY(hipMemcpyAsync(ctx->h_bound, ctx->bound.p, sizeof(int32_t) * nj, hipMemcpyDeviceToHost,
                          st));
@@ -1833,7 +1833,7 @@ hipr_result RunPasses(const std::vector<hipr_surface>& targets, hipr_surface sur
   for (int32_t j : all) most_total += std::max<int64_t>(most_planes(j), 1);
   bool counted = mode == 0 && ((opt && opt->band_rows != 0) || most_total > kUncountedPlanes);
   std::vector<int32_t> small, wide;
-  std::vector<int8_t> tier(nj, 1);  // waves (slots) of each job's walk
+  std::vector<int8_t> tier(nj, 1);  // slots (waves) of each job's walk
   for (int32_t j : all) {
     if (bound[j] > kMaxSlots * kWave) {
       std::fprintf(stderr, "skity_hip: draw %d keeps up to %d edges active (limit %d)\n",
@@ -2104,8 +2104,8 @@ hipr_result RunPasses(const std::vector<hipr_surface>& targets, hipr_surface sur
       if (!js[i].empty()) chains.push_back({{kmode, 1 << i, 0, &js[i]}});
     return run_plan(place_chains(std::move(chains)));
   };
-  // A job of up to four waves whose list still outgrew them (flag 2) is
-  // counted again by a team of 16 (recording its snapshots there); the bound
+  // A job of up to four slots whose list still outgrew them (flag 2) is
+  // counted again by the 16-slot walk (recording its snapshots there); the bound
   // makes this a safety net.  `from` holds the flags of the pass that overflowed.
   auto move_overflowed = [&](const JobCov* from, std::vector<int32_t>* moved_out) -> hipr_result {
     std::vector<int32_t> moved, keep;
@@ -2226,7 +2226,7 @@ hipr_result RunPasses(const std::vector<hipr_surface>& targets, hipr_surface sur
   } else {
     if ((r = limit_error(hw, wide, 2)) != HIPR_SUCCESS) return r;
     if ((r = limit_error(hw, all, 16 | 32)) != HIPR_SUCCESS) return r;
-    // a one-band 4-slot job (not scheduled) whose list outgrew 256 edges is
+    // a one-band job of up to four slots (not scheduled) whose list outgrew them is
     // counted by the 16-slot walk and redone below with its exact planes
     std::vector<int32_t> moved;
     if ((r = move_overflowed(hw, &moved)) != HIPR_SUCCESS) return r;

@@ -236,10 +236,12 @@ def evaluate_large(ctx, n_paths=1 << 20, side=8192, slice_paths=1 << 17, seed=0x
                    box=(-8.0, -3.0), log=print):
     """The pre-sizer's evaluation at its stated scale: n_paths outlines of the
     uneven family on a side x side canvas, drawn as consecutive scenes of
-    slice_paths paths, by the exact two-pass method, by the learned method
-    and by a linear estimate; the three frames must be identical.  Returns
-    per-form device time, fallbacks, under-estimates and capacity totals."""
-    forms = {"exact": abi.MODE_EXACT, "learned": abi.MODE_LEARNED,
+    slice_paths paths, by the exact method (planes reserved for every tile where
+    that fits), by the exact two-pass method (planes counted, then written: the
+    exact form with bands of the caller's), by the learned method and by a
+    linear estimate; the four frames must be identical.  Returns per-form
+    device time, fallbacks, under-estimates and capacity totals."""
+    forms = {"exact": abi.MODE_EXACT, "two_pass": abi.MODE_EXACT, "learned": abi.MODE_LEARNED,
              "linear_estimate": abi.MODE_ESTIMATES}
     surfs = {k: device.Surface(ctx, side, side) for k in forms}
     rep = {k: {"ms": 0.0, "fallbacks": 0, "underestimates": 0, "jobs": 0, "edges": 0,
@@ -253,8 +255,10 @@ def evaluate_large(ctx, n_paths=1 << 20, side=8192, slice_paths=1 << 17, seed=0x
         t_gen += time.time() - t0
         prep = device.Prepared(ctx, sc.scene)
         ee, te = linear_estimates(sc)
+        options = {"linear_estimate": {"edge_estimates": ee, "tile_estimates": te},
+                   "two_pass": {"band_rows": 128}}
         for k, mode in forms.items():
-            kw = {"edge_estimates": ee, "tile_estimates": te} if k == "linear_estimate" else {}
+            kw = options.get(k, {})
             surfs[k].draw(prep, mode=mode, **kw)
             surfs[k].finish()
             st = surfs[k].stats()

@@ -199,8 +199,9 @@ def test_row_bands_with_estimates(ctx, band_rows, band_min_edges):
 @pytest.mark.parametrize("flags", [abi.FLAG_NO_GRAPH, abi.FLAG_PERSISTENT,
                                    abi.FLAG_PERSISTENT | abi.FLAG_NO_GRAPH])
 def test_walk_launch_forms_match(ctx, flags):
-    """The walk passes drawn as hipGraphs (default), as direct launches, and
-    as persistent kernels on an atomic item queue give the same pixels."""
+    """The walk passes drawn by a workgroup per item (default) and by persistent
+    kernels on an atomic item queue, timed as a whole and kernel by kernel, give
+    the same pixels."""
     sc = workload(2, 40, seed=33)
     n = sc.n_paths
     ref, st_ref = render_gpu(ctx, sc.scene, sc.width, sc.height, mode=0)
@@ -212,6 +213,27 @@ def test_walk_launch_forms_match(ctx, flags):
                         edge_estimates=np.full(n, 3000, np.int32),
                         tile_estimates=np.full(n, 60, np.int32))
     assert np.array_equal(est, ref)
+
+
+def test_walk_kernels_timed_alone(ctx):
+    """FLAG_NO_GRAPH times every walk kernel by itself: a frame of two schedule
+    passes and their writes reports them as such, and as one walk without it."""
+    c = Canvas(700, 400)
+    p = Path().move_to(2.5, 390)
+    for i in range(90):  # a list of 180 edges
+        p.line_to(5 + 7.5 * i, 10 + i % 5).line_to(8 + 7.5 * i, 390 - i % 3)
+    c.draw_path(p.close(), Paint((0.9, 0.1, 0.2, 0.8)))
+    c.draw_path(Path().add_circle(350, 200, 190), Paint((0.1, 0.6, 0.2, 0.8)))
+    sc = c.scene()
+    want = O.render(sc.scene, sc.width, sc.height)
+    for flags, schedules, walks in ((0, 0, 1), (abi.FLAG_NO_GRAPH, 2, 2)):
+        surf = device.Surface(ctx, sc.width, sc.height)
+        surf.draw(sc.scene, flags=flags)
+        got, stages = surf.read(), surf.stage_times()
+        surf.close()
+        assert stages["walk_schedule"][1] == schedules
+        assert stages["walk"][1] == walks
+        assert np.array_equal(got, want)
 
 
 def test_single_pass_stroke_outgrows_its_range(ctx):
@@ -250,8 +272,8 @@ def test_stroke_degenerate_segments(ctx, cap, mode):
     points, a folded quad, a cusp cubic, a width far above the curve size):
     the stroke kernel's lanes stroke segments ahead from the quad path's
     points, and the stroker must fall back where its own point differs.
-    Exact form (count + write) and the single-pass form of the estimate
-    modes."""
+    The exact form and the estimate forms write the outlines in one pass, into
+    ranges of their own."""
     c = Canvas(200, 160)
     for k, width in enumerate((3.0, 40.0)):
         p = Paint((0.9, 0.3, 0.1, 0.7)).set_style(abi.STYLE_STROKE).set_stroke_width(width)
