@@ -1,6 +1,7 @@
 """The library's host side on a HIP runtime of host memory
 (host_runtime/host_runtime.hip), which runs no kernel but can refuse launches
-and allocations: what a draw leaves behind when one of its steps fails."""
+and allocations: what a draw leaves behind when one of its steps fails, which
+forms and splits are taken, and the grids and queues of the kernels."""
 import ctypes
 import glob
 import os
